@@ -26,8 +26,9 @@
 //       (slices whose sums a second kernel adds), A cut into token tiles
 //       for few rows of B.
 // Above 128 rows of A (prefill) the product is bound by the matrix cores:
-// gemm_i8w_prefill_kernel, a tiled GEMM whose B tiles are converted on their
-// way into LDS (see the prefill section); from 4096 rows on (kLtMinM) the
+// gemm_i8w_tile_kernel, a tiled GEMM that loads A and the codes of B straight
+// into LDS and converts the codes on their way to the matrix cores (see the
+// prefill section), with the residual add or SwiGLU in its epilogue; from 4096 rows on (kLtMinM) the
 // reference's composition through hipBLASLt, which is faster there. B stored
 // [K, N] always goes through the composition (dequantize, then hipBLASLt).
 // Each fused kernel also has a shared form (ng_gemm_int8_shared_a) that runs
@@ -1322,55 +1323,113 @@ __global__ __launch_bounds__(256) void split_reduce_shared_kernel(SharedSet s, S
 
 
 // ---- prefill variant (M > 128) ----------------------------------------------
-// Many rows of A: the product is bound by the matrix cores, not by reading
-// the weights. A block computes a BM x BN tile of C (BM = 16 TM WM rows of A,
-// BN = 16 TN WN rows of B) with WM x WN waves, each a TM x TN grid of 16x16
-// MFMA tiles, over a slice of K in steps of 64:
-//   * the A tile (fp16) and the B tile go through LDS; the B codes are
-//     converted to exact fp16 integers once, on their way into LDS, so a code
-//     is converted once per block that uses it and the matrix cores read fp16;
-//   * two LDS buffers: the loads of step kt + 1 are issued before step kt is
-//     multiplied, then stored into the other buffer; one barrier per step;
-//   * rows of 64 k are 128 bytes; piece q (16 bytes) of row r sits at
-//     q xor ((r / 2) mod 8), so that the 16 lanes of an MFMA operand read
-//     (rows r0 .. r0 + 15, one piece) hit 16 different 16-byte slots of the
-//     256 bytes the banks serve per clock;
-//   * A and B are read through buffer resources based at the block's first
-//     row: 32-bit offsets, and rows past M (or N) read zeros;
-//   * tiles are handed out XCD by XCD: consecutive block ids go to different
-//     XCDs, so block b takes tile (b mod 8) * (tiles / 8) + b / 8, and the
-//     tiles of one XCD (and of its L2) are neighbours, grouped kPfGroupM rows
-//     of tiles at a time so that they share rows of A and of B;
+// Many rows of A: the product is bound by the matrix cores (2 M flop per
+// weight byte), so a block computes a BM x BN tile of C with WM x WN waves over
+// steps of 64 k, and everything else has to hide under the MFMAs:
+//   * A (fp16) and the codes of B go from memory straight into LDS
+//     (buffer_load ... lds, 16 bytes per lane), NST steps deep: no registers,
+//     no conversion and no LDS store on the way in. A step is waited for two or
+//     more steps after its loads were issued;
+//   * B stays int8 in LDS (half the LDS bytes of fp16) and is converted to
+//     exact fp16 integers on its way from LDS into the MFMAs, the next column
+//     of 32 rows of B under the MFMAs of the current one; each code is
+//     converted by the WM waves that read it;
+//   * v_mfma_f32_32x32x16_f16 with the weights as first operand: a lane then
+//     holds 4 consecutive n of one row of C. Lane l supplies row l % 32 of each
+//     operand; MFMA (P, j) of a step (P, j in {0, 1}) takes k = 32 P + 16 (l /
+//     32) + 8 j .. + 7, so that one 16-byte read of codes feeds two MFMAs;
+//   * the fragments of the next 16 k are read while the current ones multiply,
+//     across steps too: the one barrier of a step stands before its last
+//     quarter, whose fragments are already in registers;
+//   * LDS rows of A are 128 bytes, 16-byte piece q of row r at q xor ((r / 2)
+//     mod 8); rows of B are 64 bytes, piece q at q xor ((r / 4) mod 4). The lanes
+//     that a 16-byte read serves together (measured: 0-3, 12-15, 20-27 and
+//     4-11, 16-19, 28-31 of each half wave) then touch all 64 banks once;
+//   * rows past M or N repeat the last one and are not stored; k past K (K % 64
+//     != 0) repeat k below K and are zeroed in both operands in a last step of
+//     its own (an inf times a zero code would give NaN);
+//   * the tile is stored through LDS in whole 16-byte pieces of rows of C;
+//   * tiles are handed out XCD by XCD: block b takes tile (b mod 8) * (tiles /
+//     8) + b / 8, grouped kPfGroupM rows of tiles at a time, so that the tiles
+//     of one XCD (and of its L2) share rows of A and of B;
 //   * with S > 1 the K steps are split into S slices (slice-major over the
-//     tiles); each block stores its fp32 sums in `part` [S][M][N] and
-//     split_reduce_kernel adds the slices in slice order.
-// Sums in fp32 in MFMA order; scale[n] multiplies the sum, as on the
-// streaming paths. Launch shapes, measured on MI355X with random data
-// (q_proj 4096 x 4096 at M = 4096: 16 waves of 64 x 64 on a 256 x 256 tile,
-// 127 us, against 162 us for 4 waves on 128 x 128 and 169 us for 4 waves of
-// 128 x 128 on 256 x 256, whose fragment loads the compiler serialises
-// behind each group of MFMAs): 256 x 256 with 16 waves and no K slices when
-// that gives 192 tiles or more, otherwise 128 x 128 with 4 waves and enough
-// K slices for about 512 blocks.
+//     tiles); each block stores its fp32 sums in `part` [S][M][N] and the
+//     reduction adds the slices in slice order.
+// Every output is the sum over k in one order whatever the tile shape, so only
+// S (a function of M, N and K alone) shows in the bits. Measured on MI355X, back
+// to back, against the kernel this replaces (A and B through registers, B stored
+// to LDS as fp16, two LDS buffers): o at 1024 tokens of Mistral-7B 46.8 against
+// 55.3 us, gate/up with SwiGLU 224.8 against 244.2, down 138.2 against 148.1; o
+// at 333 tokens 28.0 against 37.0; a whole layer at 333 tokens of Llama-2-7B 261
+// against 350 us, at 1024 tokens of Mistral-7B 526 against 598. What bounds it on
+// 256 x 256 tiles (1024 x 28672, K = 4096: 206 us, 1.17 PFLOP/s): the power limit
+// with the matrix cores 64% busy (1.75 GHz). The MFMAs alone (no loads, no LDS
+// reads) took 130 us, without the LDS reads 164, without the loads into LDS 182,
+// without converting codes 193. Four waves of 128 x 128 on the same tile: 220.
 constexpr int kPfBK = 64;
 constexpr int kPfGroupM = 8;
-constexpr int kPfBlocks = 512;
 
-__device__ __forceinline__ int pf_slot(int row, int q) { return row * 8 + (q ^ ((row >> 1) & 7)); }
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <int TM, int TN, int WM, int WN>
-__device__ __forceinline__ void gemm_i8w_prefill_block(
-    uint16_t* __restrict__ c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b,
-    const float* __restrict__ scale, float* __restrict__ part, int M, int N, int K, int tiles_m, int tiles_n,
-    int S, int cps, int blk) {
-    constexpr int kThreads = WM * WN * kWave;
-    constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    constexpr int kAP = BM * 8 / kThreads;  // 16-byte pieces (8 k) of A per thread per step
-    constexpr int kBP = BN * 4 / kThreads;  // 16-code pieces of B per thread per step
-    static_assert(BM * 8 % kThreads == 0 && BN * 4 % kThreads == 0, "tile pieces must divide among the threads");
-    static_assert((kThreads / 8) % 16 == 0 && (kThreads / 4) % 16 == 0, "row strides must keep the swizzle");
-    __shared__ __align__(16) u32x4 lds_a[2][BM * 8];
-    __shared__ __align__(16) u32x4 lds_b[2][BN * 8];
+// 16 bytes per lane from (voff + soff) of a buffer to LDS at lds + 16 lane.
+// Written out because the compiler waits for all outstanding loads (vmcnt(0))
+// before any LDS read that follows its builtin; the kernel waits by count. The
+// load has no register result. m0 is no allocatable register: the compiler sets
+// it before each use of its own and keeps nothing in it. s_nop: the wait state
+// between a write of m0 and a load that reads it.
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
+                 "s"(r), "s"(soff)
+                 : "memory");
+}
+
+// At most N of this wave's vector memory operations still outstanding.
+template <int N>
+__device__ __forceinline__ void wait_vmem() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// This wave's LDS reads are in its registers, then the block's barrier; no
+// memory access moves across it.
+__device__ __forceinline__ void lds_read_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// 8 codes (two dwords) as exact fp16 integers.
+__device__ __forceinline__ f16x8 codes8_to_operand(uint32_t lo, uint32_t hi) {
+    const u32x4 x = {codes_to_f16x2<0x04010400u>(lo), codes_to_f16x2<0x04030402u>(lo),
+                     codes_to_f16x2<0x04010400u>(hi), codes_to_f16x2<0x04030402u>(hi)};
+    return __builtin_bit_cast(f16x8, x);
+}
+
+// What follows the product of a launch with one K slice: nothing, the
+// residual add (out, res), or SwiGLU (SW: the tile's columns 0 .. BN / 2 - 1
+// are gate's, the others up's).
+struct TileEpi {
+    uint16_t* out;        // residual add or SwiGLU; null: none
+    const uint16_t* res;  // residual add
+};
+
+template <int BM, int BN, int WM, int WN, int NST, bool SW>
+__device__ __forceinline__ void gemm_i8w_tile_block(
+    uint16_t* c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b, const float* __restrict__ scale,
+    float* __restrict__ part, int M, int N, int K, int tiles_m, int tiles_n, int S, int cps, int blk,
+    const TileEpi& ep, const SwigluArgs* sw = nullptr) {
+    constexpr int NW = WM * WN;
+    constexpr int TM = BM / WM / 32, TN = BN / WN / 32;   // a wave's 32 x 32 tiles
+    constexpr int kAI = BM / 8 / NW, kBI = BN / 16 / NW;  // loads of 1 KiB per wave and step
+    constexpr int kABytes = BM * 128, kStage = kABytes + BN * 64;
+    constexpr int kLoads = kAI + kBI;
+    constexpr int kRow = BN * 2 + 16;  // a row of the tile of C in LDS, padded
+    static_assert(TM * WM * 32 == BM && TN * WN * 32 == BN, "tiles must divide among the waves");
+    static_assert(kAI * 8 * NW == BM && kBI * 16 * NW == BN, "loads must divide among the waves");
+    static_assert(!SW || BN / 2 % 16 == 0, "a load of B lies in gate or in up");
+    __shared__ __align__(1024) uint8_t lds[NST * kStage > BM * kRow ? NST * kStage : BM * kRow];
+    const uint32_t lds0 =
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
+    constexpr int BNC = SW ? BN / 2 : BN;  // columns of one matrix C in the tile
 
     const int ntiles = tiles_m * tiles_n;
     int t = blk;
@@ -1382,162 +1441,304 @@ __device__ __forceinline__ void gemm_i8w_prefill_block(
     const int gm = min(kPfGroupM, tiles_m - grp0);
     const int tm = grp0 + (t % per_group) % gm;
     const int tn = (t % per_group) / gm;
-    const int m0 = tm * BM, n0 = tn * BN;
+    const int m0 = tm * BM, n0 = tn * BNC;
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int wm = wave / WN, wn = wave % WN;
+    const int grp = lane >> 5;
 
     const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(a + static_cast<size_t>(m0) * K), 0,
         static_cast<int>(min(static_cast<long long>(M - m0) * K * 2, 0x7fffffffll)), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<int8_t*>(b + static_cast<size_t>(n0) * K), 0,
-        static_cast<int>(min(static_cast<long long>(N - n0) * K, 0x7fffffffll)), 0x00020000);
-    // Thread tid loads A pieces (row tid / 8 + j kThreads / 8, piece tid % 8)
-    // and B pieces (row tid / 4 + j kThreads / 4, codes 16 (tid % 4) ..).
-    const int aq = tid & 7, bp = tid & 3;
-    const uint32_t aoff0 = static_cast<uint32_t>((tid >> 3) * K * 2 + 16 * aq);
-    const uint32_t boff0 = static_cast<uint32_t>((tid >> 2) * K + 16 * bp);
-    const uint32_t astride = static_cast<uint32_t>((kThreads / 8) * K * 2);
-    const uint32_t bstride = static_cast<uint32_t>((kThreads / 4) * K);
-    const int aslot0 = pf_slot(tid >> 3, aq);
-    const int bslot0 = pf_slot(tid >> 2, 2 * bp), bslot1 = pf_slot(tid >> 2, 2 * bp + 1);
+    const auto rsrc_b = [&](const int8_t* p) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<int8_t*>(p + static_cast<size_t>(n0) * K), 0,
+            static_cast<int>(min(static_cast<long long>(N - n0) * K, 0x7fffffffll)), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rsb = rsrc_b(SW ? sw->bg : b), rsu = rsrc_b(SW ? sw->bu : b);
 
-    f32x4 acc[TM][TN];
+    // Load j of a step fills 1 KiB of LDS in lane order: 8 rows of A (lane l:
+    // row l / 8, slot l % 8) or 16 rows of B (row l / 4, slot l % 4). The
+    // swizzle is in which piece a lane fetches. Rows past M or N repeat the last.
+    const auto a_row = [&](int j) { return (wave * kAI + j) * 8 + (lane >> 3); };
+    const auto a_piece = [&](int j) { return (lane & 7) ^ ((a_row(j) >> 1) & 7); };
+    const auto b_row = [&](int j) { return (wave * kBI + j) * 16 + (lane >> 2); };
+    const int b_piece = (lane & 3) ^ ((lane >> 4) & 3);
+    uint32_t av[kAI], bv[kBI];
+#pragma unroll
+    for (int j = 0; j < kAI; ++j) av[j] = static_cast<uint32_t>(min(a_row(j), M - 1 - m0) * K * 2 + 16 * a_piece(j));
+#pragma unroll
+    for (int j = 0; j < kBI; ++j)
+        bv[j] = static_cast<uint32_t>(min(SW ? b_row(j) % BNC : b_row(j), N - 1 - n0) * K + 16 * b_piece);
+    const int nk = (K + kPfBK - 1) / kPfBK;
+    const int krem = K % kPfBK;  // k of a partial last step (a multiple of 16)
+    // Loads j0 .. j1 - 1 (A's, then B's) of a step into stage st.
+    const auto load = [&](int step, int st, int j0, int j1) {
+        const uint32_t base = lds0 + static_cast<uint32_t>(st * kStage);
+        const uint32_t k0 = static_cast<uint32_t>(step * kPfBK);
+        // Pieces past K of a partial last step fetch the step's first piece.
+        const bool part_step = krem != 0 && step == nk - 1;
+#pragma unroll
+        for (int j = 0; j < kAI; ++j) {
+            if (j < j0 || j >= j1) continue;
+            const uint32_t v = part_step && 8 * a_piece(j) >= krem ? av[j] - 16 * a_piece(j) : av[j];
+            load_lds16(rsa, base + static_cast<uint32_t>((wave * kAI + j) * 1024), v, 2 * k0);
+        }
+#pragma unroll
+        for (int j = 0; j < kBI; ++j) {
+            if (kAI + j < j0 || kAI + j >= j1) continue;
+            const uint32_t v = part_step && 16 * b_piece >= krem ? bv[j] - 16 * b_piece : bv[j];
+            const bool up = SW && (wave * kBI + j) * 16 >= BNC;
+            load_lds16(up ? rsu : rsb, base + static_cast<uint32_t>(kABytes + (wave * kBI + j) * 1024), v, k0);
+        }
+    };
+
+    f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int jn = 0; jn < TN; ++jn) acc[i][jn] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    const int nk = (K + kPfBK - 1) / kPfBK;
-    const int c0 = sl * cps, c1 = min(nk, c0 + cps);
-    u32x4 ra[kAP], rb[kBP];
-    // Loads of step kt. In a last step that runs past K (K % 64 != 0) the
-    // pieces past K are zeroed in both operands, so that they add nothing (an
-    // inf times a zero would be NaN). The step offset is part of the vector
-    // offset, which the buffer's range check covers: a piece past K of the
-    // last row of A or B lies past num_records and reads zeros without a
-    // memory access (pieces past K of other rows read the next row, in
-    // bounds, and are zeroed here).
-    auto load = [&](int kt) {
-        const int k0 = kt * kPfBK;
+    const int ar = wm * TM * 32 + (lane & 31), br = wn * TN * 32 + (lane & 31);
+    const uint32_t aoff = static_cast<uint32_t>(ar * 128 + (((2 * grp) ^ ((ar >> 1) & 7)) << 4));
+    const uint32_t boff = static_cast<uint32_t>(kABytes + br * 64 + ((grp ^ ((br >> 2) & 3)) << 4));
+    // Fragments of A for MFMA (q / 2, q % 2), and codes of B for MFMAs (P, 0) and (P, 1).
+    const auto read_a = [&](int st, int q, u32x4 (&f)[TM]) {
+        const uint8_t* p = lds + st * kStage + (aoff ^ ((4 * (q >> 1) + (q & 1)) << 4));
 #pragma unroll
-        for (int j = 0; j < kAP; ++j)
-            ra[j] = __builtin_amdgcn_raw_buffer_load_b128(rsa, aoff0 + j * astride + static_cast<uint32_t>(2 * k0), 0, 0);
-#pragma unroll
-        for (int j = 0; j < kBP; ++j)
-            rb[j] = __builtin_amdgcn_raw_buffer_load_b128(rsb, boff0 + j * bstride + static_cast<uint32_t>(k0), 0, 0);
-        if (k0 + kPfBK > K) {
-            if (k0 + 8 * aq >= K) {
-#pragma unroll
-                for (int j = 0; j < kAP; ++j) ra[j] = u32x4{0u, 0u, 0u, 0u};
-            }
-            if (k0 + 16 * bp >= K) {
-#pragma unroll
-                for (int j = 0; j < kBP; ++j) rb[j] = u32x4{0u, 0u, 0u, 0u};
-            }
-        }
+        for (int i = 0; i < TM; ++i) f[i] = *reinterpret_cast<const u32x4*>(p + i * 32 * 128);
     };
-    auto stage = [&](int buf) {
+    const auto read_b = [&](int st, int P, u32x4 (&f)[TN]) {
+        const uint8_t* p = lds + st * kStage + (boff ^ (P << 5));
 #pragma unroll
-        for (int j = 0; j < kAP; ++j) lds_a[buf][aslot0 + j * (kThreads / 8) * 8] = ra[j];
-#pragma unroll
-        for (int j = 0; j < kBP; ++j) {
-            f16x8 lo, hi;
-            codes16_to_operands(rb[j], lo, hi);
-            lds_b[buf][bslot0 + j * (kThreads / 4) * 8] = __builtin_bit_cast(u32x4, lo);
-            lds_b[buf][bslot1 + j * (kThreads / 4) * 8] = __builtin_bit_cast(u32x4, hi);
-        }
+        for (int j = 0; j < TN; ++j) f[j] = *reinterpret_cast<const u32x4*>(p + j * 32 * 64);
     };
-    const int ar0 = wm * TM * 16 + (lane & 15);
-    const int br0 = wn * TN * 16 + (lane & 15);
-    auto frags = [&](int buf, int s2, u32x4 (&af)[TM], u32x4 (&bf)[TN]) {
-        const int q = 4 * s2 + (lane >> 4);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) af[i] = lds_a[buf][pf_slot(ar0 + 16 * i, q)];
-#pragma unroll
-        for (int jn = 0; jn < TN; ++jn) bf[jn] = lds_b[buf][pf_slot(br0 + 16 * jn, q)];
-    };
-    auto mma = [&](const u32x4 (&af)[TM], const u32x4 (&bf)[TN]) {
+    // The MFMAs of column j with its weights w; the next column's codes are
+    // converted into w under them.
+    f16x8 w;
+    const auto column = [&](const u32x4 (&f)[TM], int j, uint32_t next_lo, uint32_t next_hi) {
+        const f16x8 next = codes8_to_operand(next_lo, next_hi);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, __builtin_bit_cast(f16x8, f[i]), acc[i][j], 0, 0, 0);
 #pragma unroll
-            for (int jn = 0; jn < TN; ++jn)
-                acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, af[i]),
-                                                                    __builtin_bit_cast(f16x8, bf[jn]), acc[i][jn],
-                                                                    0, 0, 0);
+        for (int i = 0; i < TM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, (10 + TM - 1) / TM, 0);
+        }
+        w = next;
+    };
+    // Columns j0 .. j1 - 1 of MFMA (., J) from the codes cb; after the last
+    // column comes column 0 of MFMA (., NJ) from ncb.
+    const auto columns = [&](const u32x4 (&f)[TM], const u32x4 (&cb)[TN], int J, const u32x4 (&ncb)[TN], int NJ,
+                             int j0, int j1) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            if (j < j0 || j >= j1) continue;
+            const u32x4 nc = j + 1 < TN ? cb[j + 1 < TN ? j + 1 : 0] : ncb[0];
+            const int o = 2 * (j + 1 < TN ? J : NJ);
+            column(f, j, nc[o], nc[o + 1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
 
-    if (c0 < c1) {
-        load(c0);
-        stage(0);
-        __syncthreads();
-        for (int kt = c0; kt < c1; ++kt) {
-            const int buf = (kt - c0) & 1;
-            if (kt + 1 < c1) load(kt + 1);
-            u32x4 af0[TM], bf0[TN], af1[TM], bf1[TN];
-            frags(buf, 0, af0, bf0);
-            frags(buf, 1, af1, bf1);
-            mma(af0, bf0);
-            mma(af1, bf1);
-            if (kt + 1 < c1) stage(buf ^ 1);
-            __syncthreads();
+    const int c0 = sl * cps, c1 = min(nk, c0 + cps);
+    const int n = c1 - c0;                            // steps of this block
+    const int full = c1 == nk && krem ? n - 1 : n;    // of them whole ones
+    u32x4 fa[2][TM], cb[2][TN];
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+        if (s < n) load(c0 + s, s, 0, kLoads);
+    if (n >= NST) wait_vmem<(NST - 1) * kLoads>();
+    else wait_vmem<0>();
+    lds_read_barrier();
+    read_a(0, 0, fa[0]);
+    read_b(0, 0, cb[0]);
+    w = codes8_to_operand(cb[0][0][0], cb[0][0][1]);
+    int st = 0;
+    // Step c0 + i's last quarter and step c0 + i + 1's first two issue the
+    // loads of step c0 + i + NST, a third each, between two columns of MFMAs:
+    // issued in one go behind the barrier they held the MFMAs up (256 x 256 at
+    // 1024 x 28672, K = 4096: 206 against 215 us; one by one between all
+    // columns: 210).
+    constexpr int kThird = (kLoads + 2) / 3, kEarly = TN > 1 ? 1 : 0;
+    for (int i = 0; i < full; ++i) {
+        const int nx = st + 1 == NST ? 0 : st + 1, prev = st == 0 ? NST - 1 : st - 1;
+        const bool more = i > 0 && i - 1 + NST < n;  // loads left of step i - 1 + NST
+        read_a(st, 1, fa[1]);
+        read_b(st, 1, cb[1]);
+        columns(fa[0], cb[0], 0, cb[0], 1, 0, 1);
+        if (more) load(c0 + i - 1 + NST, prev, kThird, 2 * kThird);
+        columns(fa[0], cb[0], 0, cb[0], 1, 1, TN);
+        read_a(st, 2, fa[0]);
+        columns(fa[1], cb[0], 1, cb[1], 0, 0, 1);
+        if (more) load(c0 + i - 1 + NST, prev, 2 * kThird, kLoads);
+        columns(fa[1], cb[0], 1, cb[1], 0, 1, TN);
+        read_a(st, 3, fa[1]);
+        columns(fa[0], cb[1], 0, cb[1], 1, 0, TN);
+        // Step i + 1 is in LDS once every wave has waited for its own loads of
+        // it; stage st is free once every wave has read its last fragments.
+        if (i + NST <= n) wait_vmem<(NST - 2) * kLoads>();
+        else wait_vmem<0>();
+        lds_read_barrier();
+        columns(fa[1], cb[1], 1, cb[0], 0, 0, kEarly);
+        read_b(nx, 0, cb[0]);
+        read_a(nx, 0, fa[0]);
+        if (i + NST < n) load(c0 + i + NST, st, 0, kThird);
+        columns(fa[1], cb[1], 1, cb[0], 0, kEarly, TN);
+        st = nx;
+    }
+    if (full < n) {
+        // The partial last step: k past K zeroed in both operands.
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool kin = 32 * (q >> 1) + 16 * grp + 8 * (q & 1) < krem;
+            read_a(st, q, fa[0]);
+            read_b(st, q >> 1, cb[0]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                if (!kin) fa[0][i] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                w = codes8_to_operand(cb[0][j][2 * (q & 1)], cb[0][j][2 * (q & 1) + 1]);
+                if (!kin) w = __builtin_bit_cast(f16x8, u32x4{0u, 0u, 0u, 0u});
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, __builtin_bit_cast(f16x8, fa[0][i]),
+                                                                       acc[i][j], 0, 0, 0);
+            }
         }
     }
 
-    const int mb = m0 + wm * TM * 16 + 4 * (lane >> 4);
+    // acc[i][j][4 q + e] is C[m0 + wm TM 32 + 32 i + l % 32][n0 + wn TN 32 + 32 j + 8 q + 4 (l / 32) + e].
+    if (S > 1) {
+        float* mine = part + static_cast<size_t>(sl) * M * N;
+        const bool vec = N % 4 == 0;
 #pragma unroll
-    for (int jn = 0; jn < TN; ++jn) {
-        const int n = n0 + wn * TN * 16 + 16 * jn + (lane & 15);
-        if (n >= N) continue;
-        if (S == 1) {
-            const float sc = scale[n];
+        for (int i = 0; i < TM; ++i) {
+            const int m = m0 + wm * TM * 32 + 32 * i + (lane & 31);
+            if (m >= M) continue;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int nn = n0 + wn * TN * 32 + 32 * j + 8 * q + 4 * grp;
+                    const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    float* o = mine + static_cast<size_t>(m) * N + nn;
+                    if (vec) {
+                        if (nn < N) *reinterpret_cast<f32x4*>(o) = v;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (nn + e < N) o[e] = v[e];
+                    }
+                }
+        }
+        return;
+    }
+    lds_read_barrier();  // the stages are free
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int nl = wn * TN * 32 + 32 * j + 8 * q + 4 * grp;
+            const float* sc = SW ? (nl < BNC ? sw->sg : sw->su) : scale;
+            float s[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = sc[min(n0 + (SW ? nl % BNC : nl) + e, N - 1)];
 #pragma unroll
             for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int m = mb + 16 * i + e;
-                    if (m < M) c[static_cast<size_t>(m) * N + n] = from_f32<f16>(acc[i][jn][e] * sc);
-                }
+                *reinterpret_cast<u32x2*>(lds + (wm * TM * 32 + 32 * i + (lane & 31)) * kRow + 2 * nl) =
+                    u32x2{pack2<f16>(acc[i][j][4 * q] * s[0], acc[i][j][4 * q + 1] * s[1]),
+                          pack2<f16>(acc[i][j][4 * q + 2] * s[2], acc[i][j][4 * q + 3] * s[3])};
+        }
+    __syncthreads();
+    constexpr int kPieces = BNC / 8;  // 16-byte pieces of a row of one matrix C
+    const auto store = [&](uint16_t* p, size_t o, int n_ok, const u32x4& v, bool vec) {
+        if (vec) {
+            st16(p + o, v);
         } else {
-            float* mine = part + static_cast<size_t>(sl) * M * N;
+            for (int e = 0; e < 8; ++e)
+                if (e < n_ok) p[o + e] = lane16(v, e);
+        }
+    };
+    const auto on16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    const bool vec = N % 8 == 0 && on16(SW ? sw->gate : c) && (!SW || on16(sw->up)) &&
+                     (ep.out == nullptr || on16(ep.out)) && (ep.res == nullptr || on16(ep.res));
+    for (int p = tid; p < BM * kPieces; p += NW * kWave) {
+        const int r = p / kPieces, q = p % kPieces;
+        const int m = m0 + r, nn = n0 + 8 * q;
+        if (m >= M || nn >= N) continue;
+        const size_t o = static_cast<size_t>(m) * N + nn;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * kRow + 16 * q);
+        if constexpr (SW) {
+            const u32x4 u = *reinterpret_cast<const u32x4*>(lds + r * kRow + 2 * BNC + 16 * q);
+            u32x4 y;
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int m = mb + 16 * i + e;
-                    if (m < M) mine[static_cast<size_t>(m) * N + n] = acc[i][jn][e];
+            for (int h = 0; h < 4; ++h)
+                y[h] = pack2<f16>(swiglu_f32(el_get<f16, 0>(v[h]), el_get<f16, 0>(u[h])),
+                                  swiglu_f32(el_get<f16, 1>(v[h]), el_get<f16, 1>(u[h])));
+            store(sw->gate, o, N - nn, v, vec);
+            store(sw->up, o, N - nn, u, vec);
+            store(ep.out, o, N - nn, y, vec);
+        } else {
+            if (ep.out == nullptr) {
+                store(c, o, N - nn, v, vec);
+            } else {
+                u32x4 x;
+                if (vec) {
+                    x = ld16(ep.res + o);
+                } else {
+                    for (int h = 0; h < 4; ++h)
+                        x[h] = (2 * h < N - nn ? ep.res[o + 2 * h] : 0u) |
+                               ((2 * h + 1 < N - nn ? ep.res[o + 2 * h + 1] : 0u) << 16);
                 }
+                u32x4 y;
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    y[h] = pack2<f16>(el_add<f16, 0>(v[h], x[h]), el_add<f16, 1>(v[h], x[h]));
+                store(c, o, N - nn, v, vec);
+                store(ep.out, o, N - nn, y, vec);
+            }
         }
     }
 }
 
-template <int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_prefill_kernel(
-    uint16_t* __restrict__ c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b,
-    const float* __restrict__ scale, float* __restrict__ part, int M, int N, int K, int tiles_m, int tiles_n,
-    int S, int cps) {
-    gemm_i8w_prefill_block<TM, TN, WM, WN>(c, a, b, scale, part, M, N, K, tiles_m, tiles_n, S, cps, blockIdx.x);
+// One or more products that share A (ng_gemm_int8_shared_a): each keeps its
+// own tiles, K slices and partial-sum region. In SplitSet, `tiles` holds the
+// product's tiles along N and `TT` its tiles along M. ep follows the product of
+// a launch of one with one K slice (out may be c or res itself: each element
+// is read and written by one thread, out last).
+template <int BM, int BN, int WM, int WN, int NST>
+__global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_kernel(SharedSet s, SplitSet sp,
+                                                                           const uint16_t* __restrict__ a, int M,
+                                                                           int K, TileEpi ep) {
+    shared_dispatch(s, [&](uint16_t* c, const int8_t* b, const float* scale, int n, int blk, int p) {
+        gemm_i8w_tile_block<BM, BN, WM, WN, NST, false>(
+            c, a, b, scale, pick4(p, sp.part[0], sp.part[1], sp.part[2], sp.part[3]), M, n, K,
+            pick4(p, sp.TT[0], sp.TT[1], sp.TT[2], sp.TT[3]),
+            pick4(p, sp.tiles[0], sp.tiles[1], sp.tiles[2], sp.tiles[3]),
+            pick4(p, sp.S[0], sp.S[1], sp.S[2], sp.S[3]), pick4(p, sp.cps[0], sp.cps[1], sp.cps[2], sp.cps[3]), blk,
+            ep);
+    });
 }
 
-// Products that share A on one prefill tile shape (ng_gemm_int8_shared_a):
-// each product keeps its own tiles, K slices and partial-sum region. In
-// SplitSet, `tiles` holds the product's tiles along N and `TT` its tiles
-// along M. A product's blocks keep their own launch's placement on the XCDs up
-// to a rotation: the tiles that one launch gives to one XCD still share one.
-template <int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_prefill_shared_kernel(SharedSet s, SplitSet sp,
-                                                                                     const uint16_t* __restrict__ a,
-                                                                                     int M, int K) {
-    shared_dispatch(s, [&](uint16_t* c, const int8_t* b, const float* scale, int n, int blk, int p) {
-        gemm_i8w_prefill_block<TM, TN, WM, WN>(c, a, b, scale, pick4(p, sp.part[0], sp.part[1], sp.part[2], sp.part[3]),
-                                               M, n, K, pick4(p, sp.TT[0], sp.TT[1], sp.TT[2], sp.TT[3]),
-                                               pick4(p, sp.tiles[0], sp.tiles[1], sp.tiles[2], sp.tiles[3]),
-                                               pick4(p, sp.S[0], sp.S[1], sp.S[2], sp.S[3]),
-                                               pick4(p, sp.cps[0], sp.cps[1], sp.cps[2], sp.cps[3]), blk);
-    });
+// gate, up and SwiGLU (ng_gemm_int8_silu_mul) with one K slice: a block's tile
+// is BN / 2 columns of gate and the same columns of up. Each output's sum over k
+// is its own launch's, so gate and up keep their bits.
+template <int BM, int BN, int WM, int WN, int NST>
+__global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_swiglu_kernel(SwigluArgs sa,
+                                                                                  const uint16_t* __restrict__ a,
+                                                                                  int M, int N, int K, int tiles_m,
+                                                                                  int tiles_n, int cps) {
+    const TileEpi ep{sa.out, nullptr};
+    gemm_i8w_tile_block<BM, BN, WM, WN, NST, true>(nullptr, a, nullptr, nullptr, nullptr, M, N, K, tiles_m, tiles_n, 1,
+                                                   cps, blockIdx.x, ep, &sa);
 }
 
 // ---- hipBLASLt path ----------------------------------------------------------
@@ -1910,53 +2111,229 @@ bool use_prefill(const void* a, const void* b, int M, int K, int N, bool transpo
            static_cast<long long>(M) * K * 2 < (1ll << 31) && static_cast<long long>(N) * K < (1ll << 31);
 }
 
-// K slices of a prefill launch of `tiles` tiles of `area` outputs: for about
-// kPfBlocks blocks, at most 8, each of 4 steps or more; none for 256 x 256
-// tiles, which are only chosen when there are enough of them to fill the CUs.
-void prefill_slices(int tiles, int area, int K, int& S, int& cps) {
-    const int nk = (K + kPfBK - 1) / kPfBK;
-    S = area >= 65536 ? 1 : max(1, min((kPfBlocks + tiles - 1) / tiles, min(8, nk / 4)));
-    cps = (nk + S - 1) / S;
-    S = (nk + cps - 1) / cps;
-}
+// Per-product plan of a shared split-K launch: K slices, batches per slice,
+// tiles along N and along M (the split kernel: token tiles), and blocks.
+struct SharedPlan {
+    int S[kMaxShared], cps[kMaxShared], tn[kMaxShared], tm[kMaxShared];
+    long long blocks[kMaxShared];
+};
 
-template <int TM, int TN, int WM, int WN>
-int launch_prefill(uint16_t* c, const uint16_t* a, const int8_t* b, const float* scale, int M, int N, int K,
-                   float* scratch, size_t scratch_bytes, const ResEpi* ep = nullptr) {
-    constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const int tiles = tiles_m * tiles_n;
-    int S = 0, cps = 0;
-    prefill_slices(tiles, BM * BN, K, S, cps);
-    const hipStream_t s = stream();
+// Products that share A on one split-K kernel shape: one launch of the kernel
+// (`launch(set, sp, blocks, stream)`), then one of the reduction for the products with
+// more than one slice of K, each product with its own slices and its own
+// region of the stream's partial-sum buffer (the lock is held until both
+// kernels are enqueued, as in launch_split).
+// With sw (gate and up, both with several K slices, as count 2), the
+// reduction is split_reduce_swiglu_kernel's; otherwise it returns 1 before
+// launching anything. With ep (a product alone), the residual add follows in
+// its reduction; scratch is a partial-sum buffer that the caller brings.
+template <typename L>
+int run_shared_split(int count, void* const* c, const void* const* b, const void* const* scales, const int* n,
+                     int M, int K, const SharedPlan& pl, L&& launch, const SwigluArgs* sw = nullptr,
+                     float* scratch = nullptr, size_t scratch_bytes = 0, const ResEpi* ep = nullptr) {
+    if (sw && !(count == 2 && n[0] == n[1] && pl.S[0] > 1 && pl.S[1] == pl.S[0])) return 1;
+    long long cols = 0;
+    for (int i = 0; i < count; ++i)
+        if (pl.S[i] > 1) cols += static_cast<long long>(pl.S[i]) * n[i];
+    // Each product's region starts on 16 bytes: up to 3 floats of padding each.
+    if (cols > 0 && count > 1) cols += 4;
+    NG_REQUIRE(cols < (1ll << 31), "ng_gemm_int8_shared_a: too many rows of B");
+    const hipStream_t st = stream();
     float* part = nullptr;
     std::unique_lock<std::mutex> lock(g_mu, std::defer_lock);
-    if (S > 1 && partial_buffer(s, S, M, N, K, scratch, scratch_bytes, lock, &part) != 0) return -1;
-    gemm_i8w_prefill_kernel<TM, TN, WM, WN><<<dim3(static_cast<unsigned>(tiles * S)), dim3(WM * WN * kWave), 0, s>>>(
-        c, a, b, scale, part, M, N, K, tiles_m, tiles_n, S, cps);
-    NG_CHECK_LAUNCH("cuda_gemm_int8");
-    if (S > 1) return launch_reduce(s, c, part, scale, M, N, S, ep);
-    return ep ? cuda_add(ep->out, c, ep->res, static_cast<size_t>(M) * N) : 0;
+    if (cols > 0 && partial_buffer(st, 1, M, static_cast<int>(cols), K, scratch, scratch_bytes, lock, &part) != 0) return -1;
+    SharedSet set{}, rset{};
+    SplitSet sp{};
+    long long blocks = 0, rblocks = 0, off = 0;
+    bool vec4_all = true, vec4_any = false;
+    for (int i = 0; i < kMaxShared; ++i) {
+        const int j = i < count ? i : 0;  // unused slots repeat product 0 and are never selected
+        set.c[i] = rset.c[i] = static_cast<uint16_t*>(c[j]);
+        set.b[i] = rset.b[i] = static_cast<const int8_t*>(b[j]);
+        set.scale[i] = rset.scale[i] = static_cast<const float*>(scales[j]);
+        set.n[i] = rset.n[i] = n[j];
+        sp.S[i] = pl.S[j];
+        sp.tiles[i] = pl.tn[j];
+        sp.cps[i] = pl.cps[j];
+        sp.TT[i] = pl.tm[j];
+        sp.part[i] = nullptr;
+        set.first[i] = i < count ? static_cast<int>(blocks) : INT_MAX;
+        rset.first[i] = i < count ? static_cast<int>(rblocks) : INT_MAX;
+        if (i >= count) continue;
+        blocks += pl.blocks[i];
+        if (pl.S[i] > 1) {
+            sp.part[i] = part + off;
+            off += (static_cast<long long>(pl.S[i]) * M * n[i] + 3) / 4 * 4;
+            const bool v4 = n[i] % 4 == 0 && aligned16(scales[i]) && aligned8(c[i]);
+            vec4_all = vec4_all && v4;
+            vec4_any = vec4_any || v4;
+            const long long mn = static_cast<long long>(M) * n[i];
+            rblocks += v4 ? (mn / 4 + 255) / 256 : (mn + 255) / 256;
+        }
+        NG_REQUIRE(blocks < (1ll << 31) && rblocks < (1ll << 31), "ng_gemm_int8_shared_a: too many rows of B");
+    }
+    launch(set, sp, static_cast<unsigned>(blocks), st);
+    NG_CHECK_LAUNCH("ng_gemm_int8_shared_a");
+    if (sw) {
+        const bool v4 = n[0] % 4 == 0 && aligned16(sw->sg) && aligned16(sw->su) && aligned8(sw->gate) &&
+                        aligned8(sw->up) && aligned8(sw->out);
+        const long long mn = static_cast<long long>(M) * n[0];
+        const unsigned sb = static_cast<unsigned>(v4 ? (mn / 4 + 255) / 256 : (mn + 255) / 256);
+        if (v4)
+            split_reduce_swiglu_kernel<true><<<dim3(sb), dim3(256), 0, st>>>(*sw, sp.part[0], sp.part[1], M, n[0],
+                                                                             pl.S[0]);
+        else
+            split_reduce_swiglu_kernel<false><<<dim3(sb), dim3(256), 0, st>>>(*sw, sp.part[0], sp.part[1], M, n[0],
+                                                                              pl.S[0]);
+        NG_CHECK_LAUNCH("ng_gemm_int8_silu_mul");
+        return 0;
+    }
+    if (rblocks == 0) return 0;
+    if (ep) return launch_reduce(st, static_cast<uint16_t*>(c[0]), part, set.scale[0], M, n[0], pl.S[0], ep);
+    if (vec4_all || !vec4_any) {
+        if (vec4_all)
+            split_reduce_shared_kernel<true><<<dim3(static_cast<unsigned>(rblocks)), dim3(256), 0, st>>>(rset, sp, M);
+        else
+            split_reduce_shared_kernel<false><<<dim3(static_cast<unsigned>(rblocks)), dim3(256), 0, st>>>(rset, sp, M);
+        NG_CHECK_LAUNCH("ng_gemm_int8_shared_a");
+        return 0;
+    }
+    // Products whose reductions take different forms: one reduction each.
+    for (int i = 0; i < count; ++i)
+        if (pl.S[i] > 1 && launch_reduce(st, static_cast<uint16_t*>(c[i]), sp.part[i],
+                                         static_cast<const float*>(scales[i]), M, n[i], pl.S[i]) != 0)
+            return -1;
+    return 0;
 }
 
-// Tile shape by the number of tiles (see the prefill kernel): 256 x 256
-// when that gives at least 192 tiles (three quarters of the CUs), otherwise
-// 128 x 128 with K slices.
-bool prefill_wide_tiles(int M, int N) {
-    return static_cast<long long>((M + 255) / 256) * ((N + 255) / 256) >= 192;
+// Tile shapes of the prefill kernel, <BM, BN, WM, WN, NST>, and the time of a
+// step of 64 k in us on MI355X: lo with up to 96 blocks on the GPU, hi with 256
+// (the clock falls as the matrix cores fill). Fitted to launches of 96 to 1792
+// tiles at K = 4096 and 14336: 256 x 256 at 2048 x 4096 (128 tiles) 95.6 us, at
+// 4096 x 4096 (256 tiles) 122; 128 x 256 54.4 us at 1024 x 4096 (128), 71.4 at
+// 2048 x 4096 (256); 128 x 128 29.4 us at 333 x 4096 (96), 40.4 at 1024 x 4096
+// (256), 251 at 1024 x 28672 (1792); 64 x 128 27.3 us at 333 x 4096 (192).
+// Also measured and slower than the best of these wherever they could be
+// taken: 256 x 128, 64 x 256, and 128 x 128 with 4 waves or 6 stages.
+struct TileShape {
+    int BM, BN;
+    double lo, hi;
+};
+constexpr TileShape kTileShapes[] = {{256, 256, 1.38, 1.84}, {128, 256, 0.78, 1.08}, {128, 128, 0.40, 0.57},
+                                     {64, 128, 0.32, 0.38}};
+constexpr int kTileShapeCount = 4;
+
+// Time of a launch of `blocks` blocks whose steps add up to `steps`, the
+// longest taking `longest`: 6 us, then a round of steps for each 256 blocks.
+double tile_time(const TileShape& ts, long long blocks, long long steps, int longest) {
+    const double fill = blocks < 96 ? 0.0 : blocks > 256 ? 1.0 : (blocks - 96) / 160.0;
+    const double rounds = static_cast<double>((blocks + 255) / 256) * (static_cast<double>(steps) / blocks);
+    return 6.0 + (ts.lo + (ts.hi - ts.lo) * fill) * (rounds > longest ? rounds : longest);
 }
 
-// With ep, the residual add after the product follows, in the split-K
-// reduction's epilogue where the launch slices K, else as cuda_add.
+long long tile_blocks(const TileShape& ts, int M, int N, int S) {
+    return ((static_cast<long long>(M) + ts.BM - 1) / ts.BM) * ((static_cast<long long>(N) + ts.BN - 1) / ts.BN) * S;
+}
+
+// K slices of a product on the prefill kernel: a function of M, N and K alone,
+// so that a product has the same bits in every launch that it is part of.
+// The S <= 8 of least time over the tile shapes, each slice of 8 steps or more
+// and the partial sums within the fixed array of ng_gemm_int8_noalloc, the
+// reduction counted as 4 us and its bytes at 5 TB/s; more than one only where
+// it saves 5% (333 x 4096 x 14336: 62 us with two slices, 95 with one; 130 x
+// 4096 x 4096 20.7 us with slices, 26.8 with one).
+void prefill_slices(int M, int N, int K, int& S, int& cps) {
+    const int nk = (K + kPfBK - 1) / kPfBK;
+    double one = 0.0, best = 0.0;
+    S = 1;
+    cps = nk;
+    for (int s = 1; s <= 8; ++s) {
+        const int per = (nk + s - 1) / s, ss = (nk + per - 1) / per;
+        const double bytes = static_cast<double>(ss) * M * N * sizeof(float);
+        if (s > 1 && (per < 8 || ss < s || bytes > static_cast<double>(kNoAllocScratchBytes))) continue;
+        double t = 0.0;
+        for (const TileShape& ts : kTileShapes) {
+            const long long blocks = tile_blocks(ts, M, N, ss);
+            const double v = tile_time(ts, blocks, blocks / ss * nk, per);
+            if (t == 0.0 || v < t) t = v;
+        }
+        if (ss > 1) t += 4.0 + 2.0 * bytes / 5e6;
+        if (s == 1) one = best = t;
+        if (s > 1 && t < 0.95 * one && t < best) {
+            best = t;
+            S = ss;
+            cps = per;
+        }
+    }
+}
+
+template <int BM, int BN, int WM, int WN, int NST>
+int launch_tiles(int count, void* const* c, const uint16_t* a, const void* const* b, const void* const* scales,
+                 const int* n, int M, int K, SharedPlan& pl, float* scratch, size_t scratch_bytes, const ResEpi* ep,
+                 const SwigluArgs* sw) {
+    const dim3 block(WM * WN * kWave);
+    if (sw && pl.S[0] == 1) {
+        const int tm = (M + BM - 1) / BM, tn = (n[0] + BN / 2 - 1) / (BN / 2);
+        gemm_i8w_tile_swiglu_kernel<BM, BN, WM, WN, NST><<<dim3(static_cast<unsigned>(tm) * tn), block, 0, stream()>>>(
+            *sw, a, M, n[0], K, tm, tn, pl.cps[0]);
+        NG_CHECK_LAUNCH("ng_gemm_int8_silu_mul");
+        return 0;
+    }
+    for (int i = 0; i < count; ++i) {
+        pl.tm[i] = (M + BM - 1) / BM;
+        pl.tn[i] = (n[i] + BN - 1) / BN;
+        pl.blocks[i] = static_cast<long long>(pl.tm[i]) * pl.tn[i] * pl.S[i];
+    }
+    const TileEpi te{ep && pl.S[0] == 1 ? ep->out : nullptr, ep && pl.S[0] == 1 ? ep->res : nullptr};
+    return run_shared_split(count, c, b, scales, n, M, K, pl,
+                            [&](const SharedSet& set, const SplitSet& sp, unsigned blocks, hipStream_t st) {
+                                gemm_i8w_tile_kernel<BM, BN, WM, WN, NST>
+                                    <<<dim3(blocks), block, 0, st>>>(set, sp, a, M, K, te);
+                            },
+                            sw, scratch, scratch_bytes, ep);
+}
+
+// Products that share A on the prefill kernel, in one launch (plus one of the
+// reduction where a product has K slices), on the tile shape of least time for
+// all of them. ep (a product alone): the residual add after it. sw (gate and
+// up): SwiGLU after them.
+int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, const void* const* scales,
+               const int* n, int M, int K, float* scratch = nullptr, size_t scratch_bytes = 0,
+               const ResEpi* ep = nullptr, const SwigluArgs* sw = nullptr) {
+    const auto* ap = static_cast<const uint16_t*>(a);
+    SharedPlan pl{};
+    const int nk = (K + kPfBK - 1) / kPfBK;
+    int longest = 0;
+    for (int i = 0; i < count; ++i) {
+        prefill_slices(M, n[i], K, pl.S[i], pl.cps[i]);
+        longest = max(longest, pl.cps[i]);
+    }
+    int shape = 0;
+    double least = 0.0;
+    for (int k = 0; k < kTileShapeCount; ++k) {
+        long long blocks = 0, steps = 0;
+        for (int i = 0; i < count; ++i) {
+            const long long bl = tile_blocks(kTileShapes[k], M, n[i], pl.S[i]);
+            blocks += bl;
+            steps += bl / pl.S[i] * nk;
+        }
+        const double t = tile_time(kTileShapes[k], blocks, steps, longest);
+        if (k == 0 || t < least) {
+            least = t;
+            shape = k;
+        }
+    }
+    switch (shape) {
+        case 0: return launch_tiles<256, 256, 2, 4, 3>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
+        case 1: return launch_tiles<128, 256, 2, 4, 4>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
+        case 2: return launch_tiles<128, 128, 2, 4, 3>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
+        default: return launch_tiles<64, 128, 2, 4, 4>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
+    }
+}
+
 int gemm_prefill(void* c, const void* a, const void* b, const void* scale, int M, int K, int N,
                  float* scratch = nullptr, size_t scratch_bytes = 0, const ResEpi* ep = nullptr) {
-    auto* cp = static_cast<uint16_t*>(c);
-    auto* ap = static_cast<const uint16_t*>(a);
-    auto* bp = static_cast<const int8_t*>(b);
-    auto* sp = static_cast<const float*>(scale);
-    if (prefill_wide_tiles(M, N))
-        return launch_prefill<4, 4, 4, 4>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
-    return launch_prefill<4, 4, 2, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
+    return gemm_tiles(1, &c, a, &b, &scale, &N, M, K, scratch, scratch_bytes, ep);
 }
 
 // The weight-streaming path takes transpose_b, M <= kMaxFusedM, 16-byte aligned
@@ -2070,96 +2447,6 @@ extern "C" int ng_gemm_int8_noalloc(void* c, const void* a, const void* b, const
     return gemm_prefill(c, a, b, scale, M, K, N, part, kNoAllocScratchBytes);
 }
 
-// Per-product plan of a shared split-K launch: K slices, batches per slice,
-// tiles along N and along M (the split kernel: token tiles), and blocks.
-struct SharedPlan {
-    int S[kMaxShared], cps[kMaxShared], tn[kMaxShared], tm[kMaxShared];
-    long long blocks[kMaxShared];
-};
-
-// Products that share A on one split-K kernel shape: one launch of the kernel
-// (`launch(set, sp, blocks, stream)`), then one of the reduction for the products with
-// more than one slice of K, each product with its own slices and its own
-// region of the stream's partial-sum buffer (the lock is held until both
-// kernels are enqueued, as in launch_split).
-// With sw (gate and up, both with several K slices, as count 2), the
-// reduction is split_reduce_swiglu_kernel's; otherwise it returns 1 before
-// launching anything.
-template <typename L>
-int run_shared_split(int count, void* const* c, const void* const* b, const void* const* scales, const int* n,
-                     int M, int K, const SharedPlan& pl, L&& launch, const SwigluArgs* sw = nullptr) {
-    if (sw && !(count == 2 && n[0] == n[1] && pl.S[0] > 1 && pl.S[1] == pl.S[0])) return 1;
-    long long cols = 0;
-    for (int i = 0; i < count; ++i)
-        if (pl.S[i] > 1) cols += static_cast<long long>(pl.S[i]) * n[i];
-    NG_REQUIRE(cols < (1ll << 31), "ng_gemm_int8_shared_a: too many rows of B");
-    const hipStream_t st = stream();
-    float* part = nullptr;
-    std::unique_lock<std::mutex> lock(g_mu, std::defer_lock);
-    if (cols > 0 && partial_buffer(st, 1, M, static_cast<int>(cols), K, nullptr, 0, lock, &part) != 0) return -1;
-    SharedSet set{}, rset{};
-    SplitSet sp{};
-    long long blocks = 0, rblocks = 0, off = 0;
-    bool vec4_all = true, vec4_any = false;
-    for (int i = 0; i < kMaxShared; ++i) {
-        const int j = i < count ? i : 0;  // unused slots repeat product 0 and are never selected
-        set.c[i] = rset.c[i] = static_cast<uint16_t*>(c[j]);
-        set.b[i] = rset.b[i] = static_cast<const int8_t*>(b[j]);
-        set.scale[i] = rset.scale[i] = static_cast<const float*>(scales[j]);
-        set.n[i] = rset.n[i] = n[j];
-        sp.S[i] = pl.S[j];
-        sp.tiles[i] = pl.tn[j];
-        sp.cps[i] = pl.cps[j];
-        sp.TT[i] = pl.tm[j];
-        sp.part[i] = nullptr;
-        set.first[i] = i < count ? static_cast<int>(blocks) : INT_MAX;
-        rset.first[i] = i < count ? static_cast<int>(rblocks) : INT_MAX;
-        if (i >= count) continue;
-        blocks += pl.blocks[i];
-        if (pl.S[i] > 1) {
-            sp.part[i] = part + off;
-            off += static_cast<long long>(pl.S[i]) * M * n[i];
-            const bool v4 = n[i] % 4 == 0 && aligned16(scales[i]) && aligned8(c[i]);
-            vec4_all = vec4_all && v4;
-            vec4_any = vec4_any || v4;
-            const long long mn = static_cast<long long>(M) * n[i];
-            rblocks += v4 ? (mn / 4 + 255) / 256 : (mn + 255) / 256;
-        }
-        NG_REQUIRE(blocks < (1ll << 31) && rblocks < (1ll << 31), "ng_gemm_int8_shared_a: too many rows of B");
-    }
-    launch(set, sp, static_cast<unsigned>(blocks), st);
-    NG_CHECK_LAUNCH("ng_gemm_int8_shared_a");
-    if (sw) {
-        const bool v4 = n[0] % 4 == 0 && aligned16(sw->sg) && aligned16(sw->su) && aligned8(sw->gate) &&
-                        aligned8(sw->up) && aligned8(sw->out);
-        const long long mn = static_cast<long long>(M) * n[0];
-        const unsigned sb = static_cast<unsigned>(v4 ? (mn / 4 + 255) / 256 : (mn + 255) / 256);
-        if (v4)
-            split_reduce_swiglu_kernel<true><<<dim3(sb), dim3(256), 0, st>>>(*sw, sp.part[0], sp.part[1], M, n[0],
-                                                                             pl.S[0]);
-        else
-            split_reduce_swiglu_kernel<false><<<dim3(sb), dim3(256), 0, st>>>(*sw, sp.part[0], sp.part[1], M, n[0],
-                                                                              pl.S[0]);
-        NG_CHECK_LAUNCH("ng_gemm_int8_silu_mul");
-        return 0;
-    }
-    if (rblocks == 0) return 0;
-    if (vec4_all || !vec4_any) {
-        if (vec4_all)
-            split_reduce_shared_kernel<true><<<dim3(static_cast<unsigned>(rblocks)), dim3(256), 0, st>>>(rset, sp, M);
-        else
-            split_reduce_shared_kernel<false><<<dim3(static_cast<unsigned>(rblocks)), dim3(256), 0, st>>>(rset, sp, M);
-        NG_CHECK_LAUNCH("ng_gemm_int8_shared_a");
-        return 0;
-    }
-    // Products whose reductions take different forms: one reduction each.
-    for (int i = 0; i < count; ++i)
-        if (pl.S[i] > 1 && launch_reduce(st, static_cast<uint16_t*>(c[i]), sp.part[i],
-                                         static_cast<const float*>(scales[i]), M, n[i], pl.S[i]) != 0)
-            return -1;
-    return 0;
-}
-
 // The split kernel's shared form: slices and blocks as launch_split.
 template <int MT, int W, int G>
 int launch_split_shared(int count, void* const* c, const uint16_t* a, const void* const* b,
@@ -2180,28 +2467,8 @@ int launch_split_shared(int count, void* const* c, const uint16_t* a, const void
                             }, sw);
 }
 
-// The prefill kernel's shared form: tiles and slices as launch_prefill.
-template <int TM, int TN, int WM, int WN>
-int launch_prefill_shared(int count, void* const* c, const uint16_t* a, const void* const* b,
-                          const void* const* scales, const int* n, int M, int K) {
-    constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    SharedPlan pl{};
-    for (int i = 0; i < count; ++i) {
-        pl.tm[i] = (M + BM - 1) / BM;
-        pl.tn[i] = (n[i] + BN - 1) / BN;
-        prefill_slices(pl.tm[i] * pl.tn[i], BM * BN, K, pl.S[i], pl.cps[i]);
-        pl.blocks[i] = static_cast<long long>(pl.tm[i]) * pl.tn[i] * pl.S[i];
-    }
-    return run_shared_split(count, c, b, scales, n, M, K, pl,
-                            [&](const SharedSet& set, const SplitSet& sp, unsigned blocks, hipStream_t st) {
-                                gemm_i8w_prefill_shared_kernel<TM, TN, WM, WN>
-                                    <<<dim3(blocks), dim3(WM * WN * kWave), 0, st>>>(set, sp, a, M, K);
-                            });
-}
-
-// Launch shapes of the fused prefill kernel for ng_gemm_int8_shared_a: 128 x 128
-// tiles with K slices, or 256 x 256 tiles.
-constexpr int kPathPrefill128 = 40, kPathPrefill256 = 41;
+// ng_gemm_int8_shared_a's path of the products on the prefill kernel.
+constexpr int kPathPrefill = 40;
 
 // One group of products that take the same launch shape `path` (see
 // shared_path), in one launch of that kernel's shared form; shapes without a
@@ -2221,8 +2488,7 @@ int shared_group(int path, int count, void* const* c, const void* a, const void*
             case 10 + kSplit242: return launch_split_shared<2, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
             case 10 + kSplit442: return launch_split_shared<4, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
             case 10 + kSplit842: return launch_split_shared<8, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
-            case kPathPrefill128: return launch_prefill_shared<4, 4, 2, 2>(count, c, ap, b, scales, n, M, K);
-            case kPathPrefill256: return launch_prefill_shared<4, 4, 4, 4>(count, c, ap, b, scales, n, M, K);
+            case kPathPrefill: return gemm_tiles(count, c, ap, b, scales, n, M, K);
             default: break;
         }
     }
@@ -2277,9 +2543,8 @@ extern "C" int ng_gemm_int8_shared_a(int count, void* const* c, const void* a, c
         NG_REQUIRE(n[i] > 0, "ng_gemm_int8_shared_a: n[%d]=%d must be > 0", i, n[i]);
         // cuda_gemm_int8's fused prefill kernel runs below kLtMinM rows of A
         path[i] = use_i8w(a, b[i], M, K, n[i], true) ? shared_path(M, K, n[i])
-                  : M < kLtMinM && use_prefill(a, b[i], M, K, n[i], true)
-                      ? (prefill_wide_tiles(M, n[i]) ? kPathPrefill256 : kPathPrefill128)
-                      : 0;
+                  : M < kLtMinM && use_prefill(a, b[i], M, K, n[i], true) ? kPathPrefill
+                                                                          : 0;
     }
     bool done[kMaxShared] = {};
     for (int i = 0; i < count; ++i) {
@@ -2516,6 +2781,13 @@ extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void
         int r = swiglu_split(sa, static_cast<const uint16_t*>(a), M, K, N);
         if (r == 1) r = swiglu_sliced(sa, static_cast<const uint16_t*>(a), M, K, N);
         if (r <= 0) return r;
+    } else if (path < 1 && apart && M < kLtMinM && use_prefill(a, b_gate, M, K, N, true) &&
+               use_prefill(a, b_up, M, K, N, true) && !use_i8w(a, b_gate, M, K, N, true)) {
+        void* c[2] = {gate, up};
+        const void* b[2] = {b_gate, b_up};
+        const void* sc[2] = {scale_gate, scale_up};
+        const int n[2] = {N, N};
+        return gemm_tiles(2, c, a, b, sc, n, M, K, nullptr, 0, nullptr, &sa);
     }
     if (path < 1 || !apart) {
         void* c[2] = {gate, up};

@@ -472,3 +472,66 @@ def test_reference_kat_gemm_transpose(lib):
     B = _ref_uniform(K * N).reshape(K, N)
     got = f16val(gemm_fp16(lib, f16bits(A), f16bits(B), M, K, N, True, False))
     assert np.abs(got - _cpu_matmul(A.T, B)).max() < 0.1
+
+
+# The prefill kernel at the edges of its tiles (64, 128 and 256 rows of A, 128
+# and 256 of B), of its stages (fewer steps of 64 k than stages, a partial last
+# step after none, one or more whole ones), with K slices, with N that no 16-byte
+# store divides and with C off 16 bytes. Inputs whose sums are exact in fp32, so
+# every tile shape and slice count has to give the same bits.
+TILE_EDGES = [(129, 16, 1), (129, 64, 127), (191, 80, 129), (192, 128, 128), (193, 192, 255), (255, 208, 257),
+              (257, 256, 300), (384, 320, 4097), (385, 336, 4100), (511, 1024, 14344), (1025, 2048, 8200),
+              (130, 14336, 512), (333, 11008, 1000), (200, 8208, 66)]
+
+
+@pytest.mark.parametrize("M,K,N", TILE_EDGES)
+def test_int8_prefill_tile_edges(lib, M, K, N):
+    banner(f"gemm_int8 prefill tile edges M={M} K={K} N={N}")
+    a = exact_activations(M, K)
+    q = codes((N, K))
+    scale = RNG.uniform(1e-3, 1e-2, N).astype(np.float16).astype(np.float32)
+    want = ((f16val(a) @ q.astype(np.float64).T).astype(np.float32) * scale[None, :]).astype(np.float16)
+    assert_bits_equal(gemm_int8(lib, a, q, scale, M, K, N, True), want.view(np.uint16), "C")
+    ab, qb, sb, cb = dev(a), dev(q), dev(scale), empty(M * N * 2 + 2)
+    ok(lib.cuda_gemm_int8(cb.offset(2), ab.vp, qb.vp, sb.vp, M, K, N, True), "C off 16 bytes")
+    assert_bits_equal(get(cb, np.uint16, (M * N + 1,))[1:].reshape(M, N), want.view(np.uint16), "C off 16 bytes")
+
+
+@pytest.mark.parametrize("M,K,N,off", [(333, 1024, 4096, 0), (1000, 4096, 14336, 0), (200, 1040, 1002, 0),
+                                       (257, 128, 257, 2)])
+def test_int8_prefill_epilogues(lib, M, K, N, off):
+    """SwiGLU and the residual add in the prefill kernel's epilogue give the bits
+    of the calls they replace, also with out in place and off 16 bytes."""
+    banner(f"gemm_int8 prefill epilogues M={M} K={K} N={N} off={off}")
+    a, res = f16bits(RNG.standard_normal((M, K))), f16bits(RNG.standard_normal((M, N)))
+    qg, qu = codes((N, K)), codes((N, K))
+    sg, su = (RNG.uniform(1e-4, 1e-3, N).astype(np.float32) for _ in range(2))
+    ab, rb, gb, ub, sgb, sub = (dev(x) for x in (a, res, qg, qu, sg, su))
+    g = gemm_int8(lib, a, qg, sg, M, K, N, True)
+    u = gemm_int8(lib, a, qu, su, M, K, N, True)
+    gd, ud, od = dev(g), dev(u), empty(2 * M * N)
+    ok(lib.cuda_silu_mul(od.vp, gd.vp, ud.vp, M * N))
+    act = get(od, np.uint16, (M, N))
+    ok(lib.cuda_add(od.vp, gd.vp, rb.vp, M * N))
+    total = get(od, np.uint16, (M, N))
+
+    def fresh():
+        return empty(2 * M * N + off)
+
+    def read(b):
+        return get(b, np.uint8, (2 * M * N + off,))[off:].view(np.uint16).reshape(M, N)
+
+    o, gate, up = fresh(), fresh(), fresh()
+    ok(lib.ng_gemm_int8_silu_mul(o.offset(off), gate.offset(off), up.offset(off), ab.vp, gb.vp, sgb.vp, ub.vp, sub.vp,
+                                 M, K, N))
+    for got, want, what in ((read(gate), g, "gate"), (read(up), u, "up"), (read(o), act, "silu * up")):
+        assert_bits_equal(got, want, what)
+    ok(lib.ng_gemm_int8_silu_mul(gate.offset(off), gate.offset(off), up.offset(off), ab.vp, gb.vp, sgb.vp, ub.vp,
+                                 sub.vp, M, K, N))
+    assert_bits_equal(read(gate), act, "silu * up in gate")
+    o, c = fresh(), fresh()
+    ok(lib.ng_gemm_int8_add(o.offset(off), c.offset(off), ab.vp, gb.vp, sgb.vp, rb.vp, M, K, N))
+    assert_bits_equal(read(c), g, "C")
+    assert_bits_equal(read(o), total, "C + residual")
+    ok(lib.ng_gemm_int8_add(rb.vp, c.offset(off), ab.vp, gb.vp, sgb.vp, rb.vp, M, K, N))
+    assert_bits_equal(get(rb, np.uint16, (M, N)), total, "C + residual in the residual")
