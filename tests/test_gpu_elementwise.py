@@ -143,3 +143,38 @@ def test_softmax_close(lib, ora):
     xb, ob = dev(x), empty(x.nbytes)
     ok(lib.cuda_softmax(ob.vp, xb.vp, 33, 1000))
     assert_close16(get(ob, np.uint16, x.shape), ora.softmax(x), "f16", "softmax")
+
+
+# Rows in registers at the edges of their vectors per thread, rows too long for
+# that, rows that no 16-byte vector divides, and rows off 16 bytes. Bound: the
+# rounding to fp16 (half an ulp, 2^-25 below 2^-14) and 2^-16 of the value: the
+# exponential's and the quotient's last bits and a sum of at most cols / 1024 + 20
+# rounded additions a thread (2^-24 each).
+@pytest.mark.parametrize("rows,cols,off", [(3, 8, 0), (2, 512, 0), (2, 520, 0), (5, 2048, 0), (3, 2056, 0), (2, 8192, 0),
+                                           (2, 8200, 0), (2, 16392, 0), (64, 32000, 0), (2, 65536, 0), (2, 65544, 0),
+                                           (1, 131080, 0), (2, 1001, 0), (3, 4096, 1)])
+def test_softmax_rows(lib, rows, cols, off):
+    banner(f"softmax {rows}x{cols} off {off}")
+    x = bits(RNG.standard_normal((rows, cols)) * 4, "f16")
+    x[0, cols // 2] = 0xFC00                    # -inf: probability 0
+    x[-1, cols - 1] = 0x4B00                    # the last element is the maximum (14)
+    xb, ob = dev(np.concatenate([np.zeros(off, np.uint16), x.ravel()])), empty(x.nbytes + 2 * off)
+    ok(lib.cuda_softmax(ob.offset(2 * off), xb.offset(2 * off), rows, cols))
+    got = get(ob, np.uint16, (x.size + off,))[off:].view(np.float16).astype(np.float64).reshape(x.shape)
+    v = x.view(np.float16).astype(np.float64)
+    e = np.exp(v - v.max(1, keepdims=True))
+    want = e / e.sum(1, keepdims=True)
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(want, 2.0 ** -14))) - 10)
+    assert (np.abs(got - want) <= 0.5 * ulp + want * 2.0 ** -16).all()
+
+
+@pytest.mark.parametrize("cols", [1000, 4096, 70000])
+def test_softmax_nonfinite_rows(lib, cols):
+    """A NaN or +inf anywhere, or nothing but -inf, makes the whole row NaN."""
+    banner(f"softmax non-finite rows of {cols}")
+    x = bits(RNG.standard_normal((4, cols)), "f16")
+    x[0, 5], x[1, cols - 2], x[2] = 0x7E00, 0x7C00, 0xFC00
+    xb, ob = dev(x), empty(x.nbytes)
+    ok(lib.cuda_softmax(ob.vp, xb.vp, 4, cols))
+    got = get(ob, np.uint16, x.shape).view(np.float16)
+    assert np.isnan(got[:3]).all() and np.isfinite(got[3]).all()
