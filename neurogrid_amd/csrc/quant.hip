@@ -14,7 +14,9 @@
 // the caller's scale word itself: zero it, atomicMax the fp16 magnitude
 // patterns into it, quantise, then overwrite it with the scale - four
 // launches in stream order, no allocation, no host synchronisation.
-// Per-column quantisation uses the caller's scales[N] the same way.
+// Per-column quantisation in its vector form passes its partial maxima through
+// the output buffer, which its last launch fills with the codes; the
+// element-wise form uses the caller's scales[N] as the per-tensor path does.
 #include "ng_common.hpp"
 
 namespace ng {
@@ -113,67 +115,179 @@ __global__ void tensor_scale_finalize_kernel(float* scale) {
 }
 
 // ---- per column of [K, N] ------------------------------------------------------
-// Thread = one column (scalar) or one group of 8 columns (vector), over a
-// chunk of rows; the chunk maximum is folded into colmax[N] with atomicMax.
-__global__ __launch_bounds__(kQThreads) void col_absmax_kernel(uint32_t* colmax, const uint16_t* x, int K, int N,
-                                                               int rows_per_chunk, int vec) {
-    const int r0 = blockIdx.y * rows_per_chunk;
-    const int r1 = min(K, r0 + rows_per_chunk);
-    if (vec) {
-        const int cv = blockIdx.x * kQThreads + threadIdx.x;
-        if (cv >= N / 8) return;
-        uint32_t m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int r = r0; r < r1; ++r) {
-            const u32x4 v = ld16(x + static_cast<size_t>(r) * N + cv * 8);
+// Vector form (N % 8 == 0, aligned pointers, K >= kColMinRows): three launches.
+//   1. The matrix is cut into chunks of `rows` rows x 512 columns, a block each:
+//      lane l of a wave owns 8 neighbouring columns (16-byte loads, 1 KiB per
+//      instruction), the 4 waves take every fourth row, kColLoads rows requested
+//      before any is folded. The maxima are taken on packed magnitude patterns
+//      and stored, 16 bits per column and chunk, in the output buffer: chunks N
+//      2 <= K N bytes, as a chunk holds 16 rows or more. No atomics and nothing
+//      to clear first.
+//   2. One thread group per 8 columns folds the chunks and writes the scales.
+//   3. The same chunks are quantised (the codes overwrite the partial maxima),
+//      the 8 scales and reciprocals of a thread computed once per chunk.
+// Bound by HBM: the matrix is read twice (the second time partly from the
+// Infinity Cache) and the codes are written. At 4096 x 14336 on MI355X the three
+// launches take 21.1 + 5.0 + 27.8 us; with a thread per 8 columns and 64 rows
+// and an atomicMax per column, and a scale pair computed for every vector
+// quantised, the four took 5.1 + 55.4 + 55.2 + 5.2. The codes are stored with the
+// default policy: non-temporal stores made the third launch 25.2 us but a
+// dequantisation that follows 38.6 instead of 25.3.
+constexpr int kColCols = 8 * kWave;   // columns of a chunk
+constexpr int kColLoads = 4;          // rows in flight per wave
+constexpr int kColMinRows = 16;       // rows of a chunk, at least
+
+// Largest magnitude pattern per half; patterns above inf's are NaNs.
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ bool has_nan_pattern(uint32_t m) {
+    return (m & 0xffffu) > kInfBits<f16> || (m >> 16) > kInfBits<f16>;
+}
+
+__global__ __launch_bounds__(kQThreads) void col_absmax_kernel(uint16_t* part, const uint16_t* x, int K, int N,
+                                                               int rows) {
+    constexpr int kWaves = kQThreads / kWave;
+    __shared__ u32x4 s_max[kWaves][kWave];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = blockIdx.x * kColCols + 8 * lane;
+    const bool in = c < N;
+    const uint16_t* xc = x + (in ? c : 0);
+    const int r1 = min(K, static_cast<int>(blockIdx.y + 1) * rows);
+    const int r0 = blockIdx.y * rows + wave;
+    u32x4 m = {0u, 0u, 0u, 0u};
+    for (int r = r0; r < r1; r += kColLoads * kWaves) {
+        u32x4 v[kColLoads];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t b = absbits_nonan<f16>(lane16(v, e));
-                m[e] = m[e] > b ? m[e] : b;
+        for (int u = 0; u < kColLoads; ++u)  // rows past the chunk repeat its last one
+            v[u] = ld16(xc + static_cast<size_t>(min(r + u * kWaves, r1 - 1)) * N);
+#pragma unroll
+        for (int u = 0; u < kColLoads; ++u)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) m[d] = pk_max_u16(m[d], v[u][d] & 0x7fff7fffu);
+    }
+    bool nan = false;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) nan = nan || has_nan_pattern(m[d]);
+    if (nan) {  // rare: the maximum over the non-NaN elements
+        uint32_t e[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int r = r0; r < r1; r += kWaves) {
+            const u32x4 v = ld16(xc + static_cast<size_t>(r) * N);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t b = absbits_nonan<f16>(lane16(v, i));
+                e[i] = e[i] > b ? e[i] : b;
             }
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) atomicMax(colmax + cv * 8 + e, m[e]);
-    } else {
-        const int c = blockIdx.x * kQThreads + threadIdx.x;
-        if (c >= N) return;
-        uint32_t m = 0;
-        for (int r = r0; r < r1; ++r) {
-            const uint32_t b = absbits_nonan<f16>(x[static_cast<size_t>(r) * N + c]);
-            m = m > b ? m : b;
+        for (int d = 0; d < 4; ++d) m[d] = e[2 * d] | (e[2 * d + 1] << 16);
+    }
+    s_max[wave][lane] = m;
+    __syncthreads();
+    if (wave != 0 || !in) return;
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) m[d] = pk_max_u16(m[d], s_max[w][lane][d]);
+    u32x2* o = reinterpret_cast<u32x2*>(part + static_cast<size_t>(blockIdx.y) * N + c);  // 8-byte aligned
+    o[0] = u32x2{m[0], m[1]};
+    o[1] = u32x2{m[2], m[3]};
+}
+
+// scales[c] from the partial maxima: 8 threads share 8 columns' chunks.
+__global__ __launch_bounds__(kQThreads) void col_scale_kernel(float* scales, const uint16_t* part, int chunks, int N) {
+    constexpr int kShare = 8;
+    const int g = threadIdx.x & (kShare - 1);
+    const int c = 8 * static_cast<int>(blockIdx.x * (kQThreads / kShare) + threadIdx.x / kShare);
+    u32x4 m = {0u, 0u, 0u, 0u};
+    if (c < N) {
+#pragma unroll 4
+        for (int k = g; k < chunks; k += kShare) {
+            const u32x2* p = reinterpret_cast<const u32x2*>(part + static_cast<size_t>(k) * N + c);
+            const u32x2 lo = p[0], hi = p[1];
+            m[0] = pk_max_u16(m[0], lo[0]);
+            m[1] = pk_max_u16(m[1], lo[1]);
+            m[2] = pk_max_u16(m[2], hi[0]);
+            m[3] = pk_max_u16(m[3], hi[1]);
         }
-        atomicMax(colmax + c, m);
+    }
+#pragma unroll
+    for (int off = 1; off < kShare; off <<= 1)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) m[d] = pk_max_u16(m[d], __shfl_xor(m[d], off, kWave));
+    if (c < N) scales[c + g] = scale_from_bits((m[g >> 1] >> (16 * (g & 1))) & 0xffffu);
+}
+
+__global__ __launch_bounds__(kQThreads) void col_quant_kernel(int8_t* q, const uint16_t* x, const float* scales, int K,
+                                                              int N, int rows) {
+    constexpr int kWaves = kQThreads / kWave;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = blockIdx.x * kColCols + 8 * lane;
+    if (c >= N) return;
+    float sc[8], inv[8];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        sc[e] = scales[c + e];
+        inv[e] = 1.0f / sc[e];
+        finite = finite && __builtin_isfinite(sc[e]);
+    }
+    const int r1 = min(K, static_cast<int>(blockIdx.y + 1) * rows);
+    for (int r = blockIdx.y * rows + wave; r < r1; r += kColLoads * kWaves) {
+        u32x4 v[kColLoads];
+#pragma unroll
+        for (int u = 0; u < kColLoads; ++u)
+            v[u] = ld16_stream(x + static_cast<size_t>(min(r + u * kWaves, r1 - 1)) * N + c);
+#pragma unroll
+        for (int u = 0; u < kColLoads; ++u) {
+            if (r + u * kWaves >= r1) break;
+            const uint32_t m = pk_max_u16(pk_max_u16(v[u][0] & 0x7fff7fffu, v[u][1] & 0x7fff7fffu),
+                                          pk_max_u16(v[u][2] & 0x7fff7fffu, v[u][3] & 0x7fff7fffu));
+            u32x2 o = {0u, 0u};
+            if (finite && !has_nan_pattern(m)) {
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const uint32_t b0 = qcode_bits<f16, 0>(v[u][d], inv[2 * d], -sc[2 * d]);
+                    const uint32_t b1 = qcode_bits<f16, 1>(v[u][d], inv[2 * d + 1], -sc[2 * d + 1]);
+                    o[d >> 1] |= __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) << (16 * (d & 1));
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    o[e >> 2] |= (static_cast<uint32_t>(qcode(to_f32<f16>(lane16(v[u], e)), sc[e], inv[e])) & 0xffu)
+                                 << ((e & 3) * 8);
+            }
+            *reinterpret_cast<u32x2*>(q + static_cast<size_t>(r + u * kWaves) * N + c) = o;
+        }
     }
 }
 
-__global__ __launch_bounds__(kQThreads) void col_quant_kernel(int8_t* q, const uint16_t* x, const uint32_t* colmax,
-                                                              int K, int N, int vec) {
-    if (vec) {
-        const int cv = blockIdx.x * kQThreads + threadIdx.x;
-        if (cv >= N / 8) return;
-        float sc[8], inv[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            sc[e] = scale_from_bits(colmax[cv * 8 + e]);
-            inv[e] = 1.0f / sc[e];
-        }
-        for (int r = blockIdx.y; r < K; r += gridDim.y) {
-            float f[8];
-            unpack8<f16>(ld16(x + static_cast<size_t>(r) * N + cv * 8), f);
-            uint32_t c[2] = {0, 0};
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                c[e >> 2] |= (static_cast<uint32_t>(qcode(f[e], sc[e], inv[e])) & 0xffu) << ((e & 3) * 8);
-            *reinterpret_cast<u32x2*>(q + static_cast<size_t>(r) * N + cv * 8) = u32x2{c[0], c[1]};
-        }
-    } else {
-        const int c = blockIdx.x * kQThreads + threadIdx.x;
-        if (c >= N) return;
-        const float sc = scale_from_bits(colmax[c]);
-        const float inv = 1.0f / sc;
-        for (int r = blockIdx.y; r < K; r += gridDim.y) {
-            const size_t i = static_cast<size_t>(r) * N + c;
-            q[i] = static_cast<int8_t>(qcode(to_f32<f16>(x[i]), sc, inv));
-        }
+// Element-wise form: a thread is one column over a chunk of rows, the chunk
+// maxima are folded into colmax[N] with atomicMax.
+__global__ __launch_bounds__(kQThreads) void col_absmax_scalar_kernel(uint32_t* colmax, const uint16_t* x, int K, int N,
+                                                                      int rows_per_chunk) {
+    const int r0 = blockIdx.y * rows_per_chunk;
+    const int r1 = min(K, r0 + rows_per_chunk);
+    const int c = blockIdx.x * kQThreads + threadIdx.x;
+    if (c >= N) return;
+    uint32_t m = 0;
+    for (int r = r0; r < r1; ++r) {
+        const uint32_t b = absbits_nonan<f16>(x[static_cast<size_t>(r) * N + c]);
+        m = m > b ? m : b;
+    }
+    atomicMax(colmax + c, m);
+}
+
+__global__ __launch_bounds__(kQThreads) void col_quant_scalar_kernel(int8_t* q, const uint16_t* x,
+                                                                     const uint32_t* colmax, int K, int N) {
+    const int c = blockIdx.x * kQThreads + threadIdx.x;
+    if (c >= N) return;
+    const float sc = scale_from_bits(colmax[c]);
+    const float inv = 1.0f / sc;
+    for (int r = blockIdx.y; r < K; r += gridDim.y) {
+        const size_t i = static_cast<size_t>(r) * N + c;
+        q[i] = static_cast<int8_t>(qcode(to_f32<f16>(x[i]), sc, inv));
     }
 }
 
@@ -354,20 +468,38 @@ extern "C" int cuda_dequantize_per_tensor(void* output, const void* input, const
 extern "C" int cuda_quantize_weights(void* output, void* scales, const void* input, int K, int N) {
     NG_REQUIRE(output && scales && input, "cuda_quantize_weights: null pointer");
     NG_REQUIRE(K > 0 && N > 0, "cuda_quantize_weights: K=%d N=%d must be > 0", K, N);
-    uint32_t* colmax = static_cast<uint32_t*>(scales);
     const uint16_t* x = static_cast<const uint16_t*>(input);
-    const int vec = N % 8 == 0 && aligned16(input) && aligned8(output);
-    const int cols_per_thread = vec ? 8 : 1;
-    const unsigned gx = static_cast<unsigned>((N / cols_per_thread + kQThreads - 1) / kQThreads);
+    int8_t* q = static_cast<int8_t*>(output);
+    if (N % 8 == 0 && K >= kColMinRows && aligned16(input) && aligned8(output)) {
+        // Rows per chunk: 64, or fewer down to 16 while that leaves under
+        // 1024 chunks (four blocks per CU).
+        const unsigned gx = static_cast<unsigned>((N + kColCols - 1) / kColCols);
+        int rows = 64;
+        while (rows > kColMinRows && static_cast<long long>(gx) * ((K + rows - 1) / rows) < 1024) rows /= 2;
+        while ((K + rows - 1) / rows > 65535) rows *= 2;  // grid limit
+        const int chunks = (K + rows - 1) / rows;
+        uint16_t* part = static_cast<uint16_t*>(output);
+        float* sc = static_cast<float*>(scales);
+        const dim3 grid(gx, static_cast<unsigned>(chunks));
+        col_absmax_kernel<<<grid, dim3(kQThreads), 0, stream()>>>(part, x, K, N, rows);
+        NG_CHECK_LAUNCH("cuda_quantize_weights");
+        col_scale_kernel<<<dim3(static_cast<unsigned>((N + kQThreads - 1) / kQThreads)), dim3(kQThreads), 0, stream()>>>(
+            sc, part, chunks, N);
+        NG_CHECK_LAUNCH("cuda_quantize_weights");
+        col_quant_kernel<<<grid, dim3(kQThreads), 0, stream()>>>(q, x, sc, K, N, rows);
+        NG_CHECK_LAUNCH("cuda_quantize_weights");
+        return 0;
+    }
+    uint32_t* colmax = static_cast<uint32_t*>(scales);
+    const unsigned gx = static_cast<unsigned>((N + kQThreads - 1) / kQThreads);
     fill_u32_kernel<<<dim3((N + 255) / 256), dim3(256), 0, stream()>>>(colmax, static_cast<size_t>(N), 0u);
     NG_CHECK_LAUNCH("cuda_quantize_weights");
     const int rows_per_chunk = 64;
     const unsigned chunks = static_cast<unsigned>((K + rows_per_chunk - 1) / rows_per_chunk);
-    col_absmax_kernel<<<dim3(gx, chunks), dim3(kQThreads), 0, stream()>>>(colmax, x, K, N, rows_per_chunk, vec);
+    col_absmax_scalar_kernel<<<dim3(gx, chunks), dim3(kQThreads), 0, stream()>>>(colmax, x, K, N, rows_per_chunk);
     NG_CHECK_LAUNCH("cuda_quantize_weights");
     const unsigned gy = static_cast<unsigned>(K < 4096 ? K : 4096);
-    col_quant_kernel<<<dim3(gx, gy), dim3(kQThreads), 0, stream()>>>(static_cast<int8_t*>(output), x, colmax, K, N,
-                                                                     vec);
+    col_quant_scalar_kernel<<<dim3(gx, gy), dim3(kQThreads), 0, stream()>>>(q, x, colmax, K, N);
     NG_CHECK_LAUNCH("cuda_quantize_weights");
     col_scale_finalize_kernel<<<dim3((N + 255) / 256), dim3(256), 0, stream()>>>(static_cast<float*>(scales), N);
     NG_CHECK_LAUNCH("cuda_quantize_weights");

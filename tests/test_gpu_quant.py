@@ -208,6 +208,23 @@ def test_per_tensor_quant_with_nan_and_inf(lib, ora, n):
     assert_bits_equal(get(qb2, np.int8, (n,)), qw, "codes")
 
 
+# The vector form: fewest rows, chunks and columns of a chunk that end early,
+# more chunks than threads that fold them, and back to the element-wise form.
+@pytest.mark.parametrize("K,N", [(16, 8), (17, 520), (63, 512), (65, 1032), (129, 4104), (4099, 1016), (15, 64),
+                                 (200, 36)])
+def test_per_column_quant_chunks(lib, ora, K, N):
+    banner(f"per-column quant chunks {K}x{N}")
+    x = f16(RNG.standard_normal((K, N)) * RNG.uniform(0.01, 10, (1, N)))
+    x[:, 0] = 0                                  # a zero column
+    x[K - 1, N - 1] = 0x7BFF                     # the last element is its column's maximum
+    x[::3, 1], x[K // 2, 2], x[K // 2, 3] = 0x7E01, 0x7C00, 0xFC00
+    xb, qb, sb = dev(x), empty(x.size), empty(4 * N)
+    ok(lib.cuda_quantize_weights(qb.vp, sb.vp, xb.vp, K, N), "quant cols")
+    qw, sw = ora.quant_cols(x)
+    assert_bits_equal(get(sb, np.float32, (N,)).view(np.uint32), sw.view(np.uint32), "scales")
+    assert_bits_equal(get(qb, np.int8, (K, N)), qw, "codes")
+
+
 @pytest.mark.parametrize("K,N", [(128, 64), (100, 33)])
 def test_per_column_quant_with_nan_and_inf(lib, ora, K, N):
     banner(f"per-column quant with NaN {K}x{N}")
