@@ -16,15 +16,16 @@
 // fp16 first and sums those; the two differ by at most 2^-11 of
 // sum_k |A[m, k] * q[n, k] * scale[n]| plus the accumulation error.
 //
-// Three kernels, by M, K and N (see gemm_i8w):
+// Four kernels, by M, K and N (see gemm_i8w):
 //   M <= 2, and M <= 4 with K, N < 8192: gemv_i8w_kernel, dot-product
 //       instructions, each load reads 1 KiB contiguous of one row of B;
 //   4 < M <= 16 with K, N < 8192: gemm_i8w_kernel, matrix cores, A read from
 //       L2, waves split K within the block;
-//   otherwise, up to M = 128: gemm_i8w_split_kernel, matrix cores, A staged
+//   otherwise, up to M = 32: gemm_i8w_split_kernel, matrix cores, A staged
 //       in LDS, K split between wave groups of a block and between blocks
-//       (slices whose sums a second kernel adds), A cut into token tiles
-//       for few rows of B.
+//       (slices whose sums a second kernel adds);
+//   32 < M <= 128: gemm_i8w_ring_kernel, A and B straight into LDS several
+//       steps ahead, K split likewise.
 // Above 128 rows of A (prefill) the product is bound by the matrix cores:
 // gemm_i8w_tile_kernel, a tiled GEMM that loads A and the codes of B straight
 // into LDS and converts the codes on their way to the matrix cores (see the
@@ -62,6 +63,7 @@
 #include <mutex>
 #include <set>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -853,13 +855,14 @@ int launch_gemv(uint16_t* c, const uint16_t* a, const int8_t* b, const float* sc
 }
 
 // ---- split-K variant --------------------------------------------------------
-// For more than a few rows of A the kernel above reads A from L2 once per
-// 16 rows of B: at M = 64 that is 8 bytes of A per weight byte. Here a block
-// of W waves owns 16 W rows of B and one of S slices of K; the A columns of
-// each 128-k batch are staged once in LDS and shared by the block's waves
-// (2M / (16 W) bytes of A per weight byte). W = 4, or 8 for K >= 8192 (the
-// down projection: 22.5 vs 25.2 us at M = 64, 34.5 vs 40.1 us at M = 128;
-// 8 waves were slower at K = 4096, and 2 slower everywhere but N = 1024).
+// Up to 32 rows of A. For more than a few rows the kernel above reads A from L2
+// once per 16 rows of B: at M = 32 that is 4 bytes of A per weight byte. Here a
+// block of W waves owns 16 W rows of B and one of S slices of K; the A columns
+// of each 128-k batch are staged once in LDS and shared by the block's waves
+// (2M / (16 W) bytes of A per weight byte). W = 4, or 8 for K >= 8192 above 16
+// rows (the down projection); 8 waves were slower at K = 4096, and 2 slower
+// everywhere but N = 1024. The kernel of 33 to 128 rows does not pay here: its
+// smallest tile is 32 rows, and at 8 rows gate/up took it 25.8 against 24.9 us.
 //
 // B is read in whole 128-byte lines: each load instruction of a wave covers
 // 8 rows x 128 codes (8 lanes per row), two instructions a wave's 16 rows.
@@ -886,7 +889,7 @@ int launch_gemv(uint16_t* c, const uint16_t* a, const int8_t* b, const float* sc
 // sums in memory and no second launch.
 constexpr int kBatch = 128;  // k per batch
 
-// SW (ng_gemm_int8_silu_mul, one K slice, no token tiles): the block's first
+// SW (ng_gemm_int8_silu_mul, one K slice): the block's first
 // W/2 waves of each group take rows of the gate product and the last W/2 the
 // same rows of the up product (8 W row pairs per block instead of 16 W rows of
 // one product). A wave's sums depend only on its own 16 rows of B, which start
@@ -896,18 +899,12 @@ constexpr int kBatch = 128;  // k per batch
 template <int MT, int W, int G, bool SW = false>
 __device__ __forceinline__ void gemm_i8w_split_block(
     uint16_t* __restrict__ c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b,
-    const float* __restrict__ scale, float* __restrict__ part, int M, int N, int K, int S, int tiles, int cps,
-    int TT, int blk, const SwigluArgs* sw = nullptr) {
+    const float* __restrict__ scale, float* __restrict__ part, int M, int N, int K, int S, int cps, int blk,
+    const SwigluArgs* sw = nullptr) {
     static_assert(!SW || W % 2 == 0, "SW splits the waves of a group in two");
-    // A batch of A in LDS. From 4 tiles of A on: 256 bytes per row, 16-byte
-    // piece q of row m stored at piece q xor (m mod 16), so the MFMA reads
-    // (16 rows, one piece each per lane group) are conflict-free; padded rows
-    // (16, 32 or 64 bytes) leave two-way conflicts, unpadded unswizzled rows
-    // eight-way ones. With 1 or 2 tiles the rows are padded by 32 bytes
-    // instead: measured 6% faster there (gate/up at M = 17-32), while the
-    // swizzle is 2-11% faster at M = 64-128.
-    constexpr bool kSwizzleA = MT >= 4;
-    constexpr int kRowBytes = kSwizzleA ? kBatch * 2 : kBatch * 2 + 32;
+    // A batch of A in LDS: 256 bytes per row, padded by 32 (6% faster at 17-32
+    // rows than an xor swizzle without conflicts).
+    constexpr int kRowBytes = kBatch * 2 + 32;
     constexpr int kPieces = 16 * MT * 16;       // 16-byte pieces of A per batch
     constexpr int kThreads = G * W * kWave;
     static_assert((G * kPieces) % kThreads == 0, "A pieces must divide among the threads");
@@ -916,26 +913,8 @@ __device__ __forceinline__ void gemm_i8w_split_block(
     __shared__ __align__(16) uint8_t lds_a[2][G][16 * MT * kRowBytes];
     __shared__ __align__(16) u32x4 lds_b[G * W][2 * kWave];
 
-    // With TT > 1 token tiles, block b takes rows 16 MT ty .. of A for unit u
-    // (a tile and slice), with the TT blocks of a unit on one XCD (ids u + 8 j
-    // apart), so that they read its rows of B from one L2.
-    int unit = blk, ty = 0;
-    if (TT > 1) {
-        const int i = blk / 8;
-        ty = i % TT;
-        unit = (i / TT) * 8 + blk % 8;
-        if (unit >= tiles * S) return;
-    }
-    const int Mall = M;
-    {
-        const int m0 = 16 * MT * ty;
-        a += static_cast<size_t>(m0) * K;
-        c += static_cast<size_t>(m0) * N;
-        part += static_cast<size_t>(m0) * N;
-        M = min(16 * MT, M - m0);
-    }
-    const int sl = unit % S;
-    const int tile = unit / S;
+    const int sl = blk % S;
+    const int tile = blk / S;
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -1021,7 +1000,7 @@ __device__ __forceinline__ void gemm_i8w_split_block(
             const int pc = j * kThreads + tid;
             const int g = pc / kPieces;
             const int row = (pc % kPieces) / 16;
-            *reinterpret_cast<u32x4*>(lds_a[buf][g] + row * kRowBytes + 16 * (kSwizzleA ? (pc % 16) ^ (row & 15) : pc % 16)) = ar[j];
+            *reinterpret_cast<u32x4*>(lds_a[buf][g] + row * kRowBytes + 16 * (pc % 16)) = ar[j];
         }
     };
     auto multiply = [&](int buf, const u32x4 (&bv)[2], int first) {
@@ -1052,8 +1031,8 @@ __device__ __forceinline__ void gemm_i8w_split_block(
                 // pieces 8 st + 2 grp and the next one of row 16 t + col
                 const uint8_t* ap = lds_a[buf][kg] + (16 * t + col) * kRowBytes;
                 const int q0 = 8 * st + 2 * grp;
-                a0[t] = *reinterpret_cast<const u32x4*>(ap + 16 * (kSwizzleA ? q0 ^ col : q0));
-                a1[t] = *reinterpret_cast<const u32x4*>(ap + 16 * (kSwizzleA ? (q0 + 1) ^ col : q0 + 1));
+                a0[t] = *reinterpret_cast<const u32x4*>(ap + 16 * q0);
+                a1[t] = *reinterpret_cast<const u32x4*>(ap + 16 * (q0 + 1));
             }
 #pragma unroll
             for (int t = 0; t < MT; ++t)
@@ -1151,7 +1130,7 @@ __device__ __forceinline__ void gemm_i8w_split_block(
         return;
     }
     if (n < N) {
-        float* mine = part + static_cast<size_t>(sl) * Mall * N;
+        float* mine = part + static_cast<size_t>(sl) * M * N;
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -1165,9 +1144,8 @@ __device__ __forceinline__ void gemm_i8w_split_block(
 template <int MT, int W, int G>
 __global__ __launch_bounds__(G * W * kWave) void gemm_i8w_split_kernel(
     uint16_t* __restrict__ c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b,
-    const float* __restrict__ scale, float* __restrict__ part, int M, int N, int K, int S, int tiles, int cps,
-    int TT) {
-    gemm_i8w_split_block<MT, W, G>(c, a, b, scale, part, M, N, K, S, tiles, cps, TT, blockIdx.x);
+    const float* __restrict__ scale, float* __restrict__ part, int M, int N, int K, int S, int cps) {
+    gemm_i8w_split_block<MT, W, G>(c, a, b, scale, part, M, N, K, S, cps, blockIdx.x);
 }
 
 // gate/up and SwiGLU on the split kernel (ng_gemm_int8_silu_mul from 3 rows):
@@ -1176,8 +1154,7 @@ template <int MT, int W, int G>
 __global__ __launch_bounds__(G * W * kWave) void gemm_i8w_split_swiglu_kernel(SwigluArgs sa,
                                                                                const uint16_t* __restrict__ a,
                                                                                int M, int N, int K, int cps) {
-    gemm_i8w_split_block<MT, W, G, true>(nullptr, a, nullptr, nullptr, nullptr, M, N, K, 1, 0, cps, 1, blockIdx.x,
-                                         &sa);
+    gemm_i8w_split_block<MT, W, G, true>(nullptr, a, nullptr, nullptr, nullptr, M, N, K, 1, cps, blockIdx.x, &sa);
 }
 
 // Products that share A on one split-kernel shape (ng_gemm_int8_shared_a):
@@ -1190,9 +1167,7 @@ __global__ __launch_bounds__(G * W * kWave) void gemm_i8w_split_shared_kernel(Sh
     shared_dispatch(s, [&](uint16_t* c, const int8_t* b, const float* scale, int n, int blk, int p) {
         gemm_i8w_split_block<MT, W, G>(c, a, b, scale, pick4(p, sp.part[0], sp.part[1], sp.part[2], sp.part[3]), M,
                                        n, K, pick4(p, sp.S[0], sp.S[1], sp.S[2], sp.S[3]),
-                                       pick4(p, sp.tiles[0], sp.tiles[1], sp.tiles[2], sp.tiles[3]),
-                                       pick4(p, sp.cps[0], sp.cps[1], sp.cps[2], sp.cps[3]),
-                                       pick4(p, sp.TT[0], sp.TT[1], sp.TT[2], sp.TT[3]), blk);
+                                       pick4(p, sp.cps[0], sp.cps[1], sp.cps[2], sp.cps[3]), blk);
     });
 }
 
@@ -1412,6 +1387,54 @@ struct TileEpi {
     const uint16_t* res;  // residual add
 };
 
+// Whether rows of C (and of what else the epilogue touches) are whole 16-byte pieces.
+template <bool SW>
+__device__ __forceinline__ bool out_vec(const uint16_t* c, int N, const TileEpi& ep, const SwigluArgs* sw) {
+    const auto on16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    return N % 8 == 0 && on16(SW ? sw->gate : c) && (!SW || on16(sw->up)) && (ep.out == nullptr || on16(ep.out)) &&
+           (ep.res == nullptr || on16(ep.res));
+}
+
+// Elements o .. o + 7 of C (n_ok of them in the row) with what follows: v as
+// rounded to fp16 (SW: gate, with up in u). out may be an operand itself: each
+// element is read and written by one thread, out last.
+template <bool SW>
+__device__ __forceinline__ void store_out8(uint16_t* c, size_t o, int n_ok, const u32x4& v, const u32x4& u, bool vec,
+                                           const TileEpi& ep, const SwigluArgs* sw) {
+    const auto store = [&](uint16_t* p, const u32x4& x) {
+        if (vec) {
+            st16(p + o, x);
+        } else {
+            for (int e = 0; e < 8; ++e)
+                if (e < n_ok) p[o + e] = lane16(x, e);
+        }
+    };
+    u32x4 y;
+    if constexpr (SW) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            y[h] = pack2<f16>(swiglu_f32(el_get<f16, 0>(v[h]), el_get<f16, 0>(u[h])),
+                              swiglu_f32(el_get<f16, 1>(v[h]), el_get<f16, 1>(u[h])));
+        store(sw->gate, v);
+        store(sw->up, u);
+        store(ep.out, y);
+    } else if (ep.out == nullptr) {
+        store(c, v);
+    } else {
+        u32x4 x;
+        if (vec) {
+            x = ld16(ep.res + o);
+        } else {
+            for (int h = 0; h < 4; ++h)
+                x[h] = (2 * h < n_ok ? ep.res[o + 2 * h] : 0u) | ((2 * h + 1 < n_ok ? ep.res[o + 2 * h + 1] : 0u) << 16);
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) y[h] = pack2<f16>(el_add<f16, 0>(v[h], x[h]), el_add<f16, 1>(v[h], x[h]));
+        store(c, v);
+        store(ep.out, y);
+    }
+}
+
 template <int BM, int BN, int WM, int WN, int NST, bool SW>
 __device__ __forceinline__ void gemm_i8w_tile_block(
     uint16_t* c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b, const float* __restrict__ scale,
@@ -1479,6 +1502,7 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
         const uint32_t base = lds0 + static_cast<uint32_t>(st * kStage);
         const uint32_t k0 = static_cast<uint32_t>(step * kPfBK);
         // Pieces past K of a partial last step fetch the step's first piece.
+        // (Selects: with a branch for whole steps the loop was 4-7% slower.)
         const bool part_step = krem != 0 && step == nk - 1;
 #pragma unroll
         for (int j = 0; j < kAI; ++j) {
@@ -1567,9 +1591,11 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
     // 1024 x 28672, K = 4096: 206 against 215 us; one by one between all
     // columns: 210).
     constexpr int kThird = (kLoads + 2) / 3, kEarly = TN > 1 ? 1 : 0;
-    for (int i = 0; i < full; ++i) {
+    // STEADY: steps whose loads all exist, without a branch in the body.
+    const auto step = [&](int i, auto steady) {
+        constexpr bool STEADY = decltype(steady)::value;
         const int nx = st + 1 == NST ? 0 : st + 1, prev = st == 0 ? NST - 1 : st - 1;
-        const bool more = i > 0 && i - 1 + NST < n;  // loads left of step i - 1 + NST
+        const bool more = STEADY || (i > 0 && i - 1 + NST < n);  // loads left of step i - 1 + NST
         read_a(st, 1, fa[1]);
         read_b(st, 1, cb[1]);
         columns(fa[0], cb[0], 0, cb[0], 1, 0, 1);
@@ -1583,16 +1609,20 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
         columns(fa[0], cb[1], 0, cb[1], 1, 0, TN);
         // Step i + 1 is in LDS once every wave has waited for its own loads of
         // it; stage st is free once every wave has read its last fragments.
-        if (i + NST <= n) wait_vmem<(NST - 2) * kLoads>();
+        if (STEADY || i + NST <= n) wait_vmem<(NST - 2) * kLoads>();
         else wait_vmem<0>();
         lds_read_barrier();
         columns(fa[1], cb[1], 1, cb[0], 0, 0, kEarly);
         read_b(nx, 0, cb[0]);
         read_a(nx, 0, fa[0]);
-        if (i + NST < n) load(c0 + i + NST, st, 0, kThird);
+        if (STEADY || i + NST < n) load(c0 + i + NST, st, 0, kThird);
         columns(fa[1], cb[1], 1, cb[0], 0, kEarly, TN);
         st = nx;
-    }
+    };
+    int i0 = 0;
+    if (full > 0) step(i0++, std::false_type{});
+    for (; i0 + NST < n && i0 < full; ++i0) step(i0, std::true_type{});
+    for (; i0 < full; ++i0) step(i0, std::false_type{});
     if (full < n) {
         // The partial last step: k past K zeroed in both operands.
 #pragma unroll
@@ -1659,53 +1689,15 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
         }
     __syncthreads();
     constexpr int kPieces = BNC / 8;  // 16-byte pieces of a row of one matrix C
-    const auto store = [&](uint16_t* p, size_t o, int n_ok, const u32x4& v, bool vec) {
-        if (vec) {
-            st16(p + o, v);
-        } else {
-            for (int e = 0; e < 8; ++e)
-                if (e < n_ok) p[o + e] = lane16(v, e);
-        }
-    };
-    const auto on16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    const bool vec = N % 8 == 0 && on16(SW ? sw->gate : c) && (!SW || on16(sw->up)) &&
-                     (ep.out == nullptr || on16(ep.out)) && (ep.res == nullptr || on16(ep.res));
+    const bool vec = out_vec<SW>(c, N, ep, sw);
     for (int p = tid; p < BM * kPieces; p += NW * kWave) {
         const int r = p / kPieces, q = p % kPieces;
         const int m = m0 + r, nn = n0 + 8 * q;
         if (m >= M || nn >= N) continue;
-        const size_t o = static_cast<size_t>(m) * N + nn;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * kRow + 16 * q);
-        if constexpr (SW) {
-            const u32x4 u = *reinterpret_cast<const u32x4*>(lds + r * kRow + 2 * BNC + 16 * q);
-            u32x4 y;
-#pragma unroll
-            for (int h = 0; h < 4; ++h)
-                y[h] = pack2<f16>(swiglu_f32(el_get<f16, 0>(v[h]), el_get<f16, 0>(u[h])),
-                                  swiglu_f32(el_get<f16, 1>(v[h]), el_get<f16, 1>(u[h])));
-            store(sw->gate, o, N - nn, v, vec);
-            store(sw->up, o, N - nn, u, vec);
-            store(ep.out, o, N - nn, y, vec);
-        } else {
-            if (ep.out == nullptr) {
-                store(c, o, N - nn, v, vec);
-            } else {
-                u32x4 x;
-                if (vec) {
-                    x = ld16(ep.res + o);
-                } else {
-                    for (int h = 0; h < 4; ++h)
-                        x[h] = (2 * h < N - nn ? ep.res[o + 2 * h] : 0u) |
-                               ((2 * h + 1 < N - nn ? ep.res[o + 2 * h + 1] : 0u) << 16);
-                }
-                u32x4 y;
-#pragma unroll
-                for (int h = 0; h < 4; ++h)
-                    y[h] = pack2<f16>(el_add<f16, 0>(v[h], x[h]), el_add<f16, 1>(v[h], x[h]));
-                store(c, o, N - nn, v, vec);
-                store(ep.out, o, N - nn, y, vec);
-            }
-        }
+        const uint8_t* row = lds + r * kRow + 16 * q;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(row);
+        const u32x4 u = *reinterpret_cast<const u32x4*>(row + (SW ? 2 * BNC : 0));
+        store_out8<SW>(c, static_cast<size_t>(m) * N + nn, N - nn, v, u, vec, ep, sw);
     }
 }
 
@@ -1739,6 +1731,279 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_swiglu_kerne
     const TileEpi ep{sa.out, nullptr};
     gemm_i8w_tile_block<BM, BN, WM, WN, NST, true>(nullptr, a, nullptr, nullptr, nullptr, M, N, K, tiles_m, tiles_n, 1,
                                                    cps, blockIdx.x, ep, &sa);
+}
+
+// ---- 33 to 128 rows of A ------------------------------------------------------
+// Here the weights still have to be read once, but a block that streams its
+// rows of B also reads its K slice of A from L2, and both have to be in flight
+// ahead of the matrix cores. One tile of all rows of A x BN rows of B per block:
+//   * stages of WK x 64 k, NST of them, go straight into LDS as in the prefill
+//     kernel, NST - 1 steps ahead: 64 to 96 KiB in flight per CU and one barrier
+//     per step (the kernel this replaces staged both through registers one step
+//     ahead);
+//   * the WK groups of WN waves multiply different 64 k of a stage, each wave
+//     all rows of A by 32 rows of B, so a fragment of A feeds as many MFMAs as
+//     the tile is wide and B is converted once; the groups' sums meet in LDS at
+//     the end, in group order;
+//   * B is loaded, and lies in LDS, in 128-byte pieces of rows (128 k, two
+//     groups): whole lines; 16-byte piece q of row r at q xor ((r / 2) mod 8), as
+//     for A;
+//   * S slices of K (a function of N and K) where one slice leaves most CUs
+//     idle, added in slice order by the reduction; with one slice the epilogues
+//     of the prefill kernel. Gate and up with SwiGLU load B non-temporally (at 64
+//     rows 29.2 against 31.2 us); with K slices that was 2-8% slower.
+// Measured on MI355X against that kernel, reductions included: q/k/v of
+// Mistral-7B at 64 rows 16.0 against 22.7 us, o 11.2 against 12.0, gate/up with
+// SwiGLU 32.4 against 39.0; at 128 rows 21.7 against 29.7, 14.1 against 17.1, 46.3
+// against 67.3, down 31.2 against 32.1; gate/up of TinyLlama at 64 rows 11.2
+// against 18.1. Slower are k/v alone (N = 1024: 8.3 against 7.6 us at 64 rows) and
+// three products of 4096 rows of B at 33 - 48 rows (23.1 against 20.2 at 33).
+// Bound at 64 rows: gate/up move 117 MB of weights in 32 us (3.7 TB/s) and A 224
+// times from L2 (as much again); 8 or 16 us calls are launch, first loads and the
+// reduction.
+__device__ __forceinline__ void load_lds16_nt(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff),
+                 "s"(r), "s"(soff)
+                 : "memory");
+}
+
+template <int BM, int BN, int WN, int WK, int NST, bool SW>
+__device__ __forceinline__ void gemm_i8w_ring_block(uint16_t* c, const uint16_t* __restrict__ a,
+                                                    const int8_t* __restrict__ b, const float* __restrict__ scale,
+                                                    float* __restrict__ part, int Mall, int N, int K, int S,
+                                                    int tiles, int cps, int TT, int blk, const TileEpi& ep,
+                                                    const SwigluArgs* sw = nullptr) {
+    constexpr int NW = WN * WK;
+    constexpr int TM = BM / 32;
+    constexpr int kA64 = BM * 128, kB128 = BN * 128;  // bytes of A of 64 k, of B of 128 k
+    constexpr int kABytes = WK * kA64, kStage = kABytes + WK / 2 * kB128;
+    constexpr int kAI = kABytes / 1024 / NW, kBI = WK / 2 * kB128 / 1024 / NW, kLoads = kAI + kBI;
+    constexpr int kRow = BN * 4 + 16;  // a row of a group's fp32 sums in LDS, padded
+    constexpr int kSums = WK * BM * kRow;
+    constexpr int BNC = SW ? BN / 2 : BN;
+    static_assert(BN == 32 * WN && WK % 2 == 0 && BM % 32 == 0, "tile shape");
+    static_assert(kAI * NW * 1024 == kABytes && kBI * NW * 2048 == WK * kB128, "loads must divide among the waves");
+    __shared__ __align__(1024) uint8_t lds[NST * kStage > kSums ? NST * kStage : kSums];
+    const uint32_t lds0 =
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
+    // With TT > 1 row tiles, the TT blocks of a unit (a tile and slice) sit on
+    // one XCD (ids 8 apart), so that they read its rows of B from one L2.
+    int unit = blk, m0 = 0;
+    if (TT > 1) {
+        const int i = blk / 8;
+        m0 = BM * (i % TT);
+        unit = i / TT * 8 + blk % 8;
+        if (unit >= tiles * S) return;
+    }
+    const int M = Mall - m0;  // rows from this tile's first on
+    const int sl = unit % S, n0 = unit / S * BNC;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int kg = wave / WN, wn = wave % WN;
+    const int grp = lane >> 5;
+
+    const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(a + static_cast<size_t>(m0) * K), 0, static_cast<int>(min(static_cast<long long>(M) * K * 2, 0x7fffffffll)), 0x00020000);
+    const auto rsrc_b = [&](const int8_t* p) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<int8_t*>(p + static_cast<size_t>(n0) * K), 0,
+            static_cast<int>(min(static_cast<long long>(N - n0) * K, 0x7fffffffll)), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rsb = rsrc_b(SW ? sw->bg : b), rsu = rsrc_b(SW ? sw->bu : b);
+    // Load j of a step: 8 rows of A of one group's 64 k, or 8 rows of B of two
+    // groups' 128 k; lane l row l / 8, slot l % 8. Rows past M or N repeat the last.
+    const auto a_group = [&](int j) { return (wave * kAI + j) / (BM / 8); };
+    const auto b_pair = [&](int j) { return (wave * kBI + j) / (BN / 8); };
+    const auto a_row = [&](int j) { return (wave * kAI + j) % (BM / 8) * 8 + (lane >> 3); };
+    const auto b_row = [&](int j) { return (wave * kBI + j) % (BN / 8) * 8 + (lane >> 3); };
+    const auto piece = [&](int r) { return (lane & 7) ^ ((r >> 1) & 7); };
+    uint32_t av[kAI], bv[kBI];
+#pragma unroll
+    for (int j = 0; j < kAI; ++j)
+        av[j] = static_cast<uint32_t>(min(a_row(j), M - 1) * K * 2 + 128 * a_group(j) + 16 * piece(a_row(j)));
+#pragma unroll
+    for (int j = 0; j < kBI; ++j)
+        bv[j] = static_cast<uint32_t>(min(SW ? b_row(j) % BNC : b_row(j), N - 1 - n0) * K + 128 * b_pair(j) +
+                                      16 * piece(b_row(j)));
+    const int nk = (K + 64 * WK - 1) / (64 * WK);
+    const int kparts = K / 64 - (nk - 1) * WK;  // 64-k parts of the last step (K % 64 == 0)
+    const auto load = [&](int step, int st) {
+        const uint32_t base = lds0 + static_cast<uint32_t>(st * kStage);
+        const uint32_t k0 = static_cast<uint32_t>(step * 64 * WK);
+        // Parts past K of the last step fetch the step's first part.
+        const bool cut = kparts < WK && step == nk - 1;
+#pragma unroll
+        for (int j = 0; j < kBI; ++j) {
+            const int in_pair = piece(b_row(j)) >> 2;
+            const uint32_t v =
+                cut && 2 * b_pair(j) + in_pair >= kparts ? bv[j] - 128 * b_pair(j) - 64 * in_pair : bv[j];
+            const bool up = SW && (wave * kBI + j) % (BN / 8) * 8 >= BNC;
+            const uint32_t to = base + static_cast<uint32_t>(kABytes + (wave * kBI + j) * 1024);
+            if (SW) load_lds16_nt(up ? rsu : rsb, to, v, k0);
+            else load_lds16(rsb, to, v, k0);
+        }
+#pragma unroll
+        for (int j = 0; j < kAI; ++j) {
+            const uint32_t v = cut && a_group(j) >= kparts ? av[j] - 128 * a_group(j) : av[j];
+            load_lds16(rsa, base + static_cast<uint32_t>((wave * kAI + j) * 1024), v, 2 * k0);
+        }
+    };
+
+    f32x16 acc[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+    const int ar = lane & 31, br = wn * 32 + (lane & 31);
+    const uint32_t aoff = static_cast<uint32_t>(kg * kA64 + ar * 128 + (((2 * grp) ^ ((ar >> 1) & 7)) << 4));
+    const uint32_t boff = static_cast<uint32_t>(kABytes + kg / 2 * kB128 + br * 128 +
+                                                (((4 * (kg & 1) + grp) ^ ((br >> 1) & 7)) << 4));
+
+    const int c0 = sl * cps, c1 = min(nk, c0 + cps), n = c1 - c0;
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+        if (s < n) load(c0 + s, s);
+    // MFMA (P, j) of the group's 64 k as in the prefill kernel: fragments of A
+    // for q = 2 P + j, codes of B for both j.
+    u32x4 fa[4][TM], cb[2];
+    const auto read = [&](int st) {
+        const uint8_t* base = lds + st * kStage;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q % 2 == 0) cb[q / 2] = *reinterpret_cast<const u32x4*>(base + (boff ^ (q << 4)));
+            const uint8_t* p = base + (aoff ^ ((4 * (q >> 1) + (q & 1)) << 4));
+#pragma unroll
+            for (int m = 0; m < TM; ++m) fa[q][m] = *reinterpret_cast<const u32x4*>(p + m * 32 * 128);
+        }
+    };
+    const auto multiply = [&]() {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f16x8 w = codes8_to_operand(cb[q >> 1][2 * (q & 1)], cb[q >> 1][2 * (q & 1) + 1]);
+#pragma unroll
+            for (int m = 0; m < TM; ++m)
+                acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, __builtin_bit_cast(f16x8, fa[q][m]), acc[m], 0, 0, 0);
+        }
+    };
+    // Whole steps; a last one that not every group has a part of follows the
+    // loop (a branch around the loop's MFMAs cost gate at 64 rows 3 of 23 us).
+    const int full = c1 == nk && kparts < WK ? n - 1 : n;
+    int st = 0;
+    const auto step = [&](int i, auto steady) {
+        constexpr bool STEADY = decltype(steady)::value;
+        // This wave's loads of step i have landed; after the barrier every
+        // wave's have, and every wave has read step i - 1, whose stage the
+        // loads of step i + NST - 1 then take.
+        if (STEADY || i + NST - 1 <= n) wait_vmem<(NST - 2) * kLoads>();
+        else wait_vmem<0>();
+        lds_read_barrier();
+        read(st);
+        __builtin_amdgcn_sched_barrier(0);
+        if (STEADY || i + NST - 1 < n) load(c0 + i + NST - 1, st == 0 ? NST - 1 : st - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply();
+        __builtin_amdgcn_sched_barrier(0);
+        st = st + 1 == NST ? 0 : st + 1;
+    };
+    int i0 = 0;
+    for (; i0 + NST - 1 < n && i0 < full; ++i0) step(i0, std::true_type{});
+    for (; i0 < full; ++i0) step(i0, std::false_type{});
+    if (full < n) {
+        wait_vmem<0>();
+        lds_read_barrier();
+        if (kg < kparts) {
+            read(st);
+            multiply();
+        }
+    }
+    lds_read_barrier();  // the stages are free (their last loads were waited for)
+
+    // acc[i][4 q + e] is this group's sum for row 32 i + l % 32, column 32 wn + 8 q + 4 (l / 32) + e.
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4*>(lds + (kg * BM + 32 * i + (lane & 31)) * kRow + 4 * (32 * wn + 8 * q + 4 * grp)) =
+                f32x4{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+    __syncthreads();
+    // Eight columns from `col` of row r, groups added in order.
+    const auto sums8 = [&](int r, int col, float (&v)[8]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            f32x4 x = *reinterpret_cast<const f32x4*>(lds + r * kRow + 4 * col + 16 * h);
+#pragma unroll
+            for (int g = 1; g < WK; ++g) x += *reinterpret_cast<const f32x4*>(lds + (g * BM + r) * kRow + 4 * col + 16 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * h + e] = x[e];
+        }
+    };
+    constexpr int kPieces = BNC / 8;
+    const bool vec = S > 1 ? N % 4 == 0 : out_vec<SW>(c, N, ep, sw);
+    for (int p = tid; p < BM * kPieces; p += NW * kWave) {
+        const int r = p / kPieces, q = p % kPieces, nn = n0 + 8 * q;
+        if (r >= M || nn >= N) continue;
+        float v[8];
+        sums8(r, 8 * q, v);
+        if (S > 1) {
+            float* o = part + (static_cast<size_t>(sl) * Mall + m0 + r) * N + nn;
+            if (vec) {
+                *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
+                if (nn + 4 < N) *reinterpret_cast<f32x4*>(o + 4) = f32x4{v[4], v[5], v[6], v[7]};
+            } else {
+                for (int e = 0; e < 8; ++e)
+                    if (nn + e < N) o[e] = v[e];
+            }
+            continue;
+        }
+        const auto scaled = [&](const float* sc) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] *= sc[min(nn + e, N - 1)];
+            return pack8<f16>(v);
+        };
+        const u32x4 x = scaled(SW ? sw->sg : scale);
+        u32x4 u = x;
+        if constexpr (SW) {
+            sums8(r, BNC + 8 * q, v);
+            u = scaled(sw->su);
+        }
+        store_out8<SW>(c, static_cast<size_t>(m0 + r) * N + nn, N - nn, x, u, vec, ep, sw);
+    }
+}
+
+// A product alone: plain arguments, which are in registers when its waves
+// start (o at 64 rows 9.6 us without its reduction, 10.0 through the argument sets
+// of the shared form).
+template <int BM, int BN, int WN, int WK, int NST>
+__global__ __launch_bounds__(WN * WK * kWave, 1) void gemm_i8w_ring_kernel(
+    uint16_t* c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b, const float* __restrict__ scale,
+    float* __restrict__ part, int M, int N, int K, int S, int tiles, int cps, int TT, TileEpi ep) {
+    gemm_i8w_ring_block<BM, BN, WN, WK, NST, false>(c, a, b, scale, part, M, N, K, S, tiles, cps, TT, blockIdx.x, ep);
+}
+
+// Products that share A, as gemm_i8w_tile_kernel.
+template <int BM, int BN, int WN, int WK, int NST>
+__global__ __launch_bounds__(WN * WK * kWave, 1) void gemm_i8w_ring_shared_kernel(SharedSet s, SplitSet sp,
+                                                                                  const uint16_t* __restrict__ a,
+                                                                                  int M, int K) {
+    shared_dispatch(s, [&](uint16_t* c, const int8_t* b, const float* scale, int n, int blk, int p) {
+        gemm_i8w_ring_block<BM, BN, WN, WK, NST, false>(
+            c, a, b, scale, pick4(p, sp.part[0], sp.part[1], sp.part[2], sp.part[3]), M, n, K,
+            pick4(p, sp.S[0], sp.S[1], sp.S[2], sp.S[3]), pick4(p, sp.tiles[0], sp.tiles[1], sp.tiles[2], sp.tiles[3]),
+            pick4(p, sp.cps[0], sp.cps[1], sp.cps[2], sp.cps[3]), pick4(p, sp.TT[0], sp.TT[1], sp.TT[2], sp.TT[3]),
+            blk, TileEpi{nullptr, nullptr});
+    });
+}
+
+// gate, up and SwiGLU with one K slice, as gemm_i8w_tile_swiglu_kernel.
+template <int BM, int BN, int WN, int WK, int NST>
+__global__ __launch_bounds__(WN * WK * kWave, 1) void gemm_i8w_ring_swiglu_kernel(SwigluArgs sa,
+                                                                                  const uint16_t* __restrict__ a,
+                                                                                  int M, int N, int K, int tiles,
+                                                                                  int cps, int TT) {
+    const TileEpi ep{sa.out, nullptr};
+    gemm_i8w_ring_block<BM, BN, WN, WK, NST, true>(nullptr, a, nullptr, nullptr, nullptr, M, N, K, 1, tiles, cps, TT,
+                                                   blockIdx.x, ep, &sa);
 }
 
 // ---- hipBLASLt path ----------------------------------------------------------
@@ -1979,14 +2244,14 @@ int launch_reduce(hipStream_t s, uint16_t* c, const float* part, const float* sc
     return 0;
 }
 
-// Slices of K for a split launch of `tiles` tiles of B (and TT token tiles):
+// Slices of K for a split launch of `tiles` tiles of B:
 // enough for about 256 blocks (512 for K >= 8192; with G groups in the
 // block, 192 blocks of twice the waves), at most 8, each of at least two
 // turns, none empty; cps batches of 128 k per slice.
-void split_slices(int tiles, int TT, int G, int K, int& S, int& cps) {
+void split_slices(int tiles, int G, int K, int& S, int& cps) {
     const int nbatch = (K + kBatch - 1) / kBatch;
     const int target = G > 1 ? 192 : K >= 8192 ? 512 : 256;
-    S = (target + tiles * TT - 1) / (tiles * TT);
+    S = (target + tiles - 1) / tiles;
     S = max(1, min(S, min(8, nbatch / (2 * G))));
     cps = (nbatch + S - 1) / S;
     S = (nbatch + cps - 1) / cps;
@@ -1994,10 +2259,10 @@ void split_slices(int tiles, int TT, int G, int K, int& S, int& cps) {
 
 template <int MT, int W, int G>
 int launch_split(uint16_t* c, const uint16_t* a, const int8_t* b, const float* scale, int M, int N, int K,
-                 float* scratch, size_t scratch_bytes, int TT = 1, const ResEpi* ep = nullptr) {
+                 float* scratch, size_t scratch_bytes, const ResEpi* ep = nullptr) {
     const int tiles = (N + 16 * W - 1) / (16 * W);
     int S = 0, cps = 0;
-    split_slices(tiles, TT, G, K, S, cps);
+    split_slices(tiles, G, K, S, cps);
     // With S > 1 the partial-sum buffer is this stream's: the lock is held
     // until both kernels are enqueued, so calls from other host threads on the
     // same stream cannot slip a launch between them.
@@ -2005,10 +2270,8 @@ int launch_split(uint16_t* c, const uint16_t* a, const int8_t* b, const float* s
     float* part = nullptr;
     std::unique_lock<std::mutex> lock(g_mu, std::defer_lock);
     if (S > 1 && partial_buffer(s, S, M, N, K, scratch, scratch_bytes, lock, &part) != 0) return -1;
-    const int units = tiles * S;
-    const int blocks = TT > 1 ? (units + 7) / 8 * 8 * TT : units;
-    gemm_i8w_split_kernel<MT, W, G><<<dim3(static_cast<unsigned>(blocks)), dim3(G * W * kWave), 0, s>>>(
-        c, a, b, scale, part, M, N, K, S, tiles, cps, TT);
+    gemm_i8w_split_kernel<MT, W, G><<<dim3(static_cast<unsigned>(tiles * S)), dim3(G * W * kWave), 0, s>>>(
+        c, a, b, scale, part, M, N, K, S, cps);
     NG_CHECK_LAUNCH("cuda_gemm_int8");
     if (S > 1) return launch_reduce(s, c, part, scale, M, N, S, ep);
     return ep ? cuda_add(ep->out, c, ep->res, static_cast<size_t>(M) * N) : 0;
@@ -2025,31 +2288,31 @@ int gemv_shape(int M, int K, int N) {
     return M == 1 ? 1 : M == 2 ? 2 : 3;
 }
 
-// The split kernel's launch shape <MT, W, G> that gemm_i8w takes when the
-// GEMV kernel does not, or kSmallM for the small-M MFMA kernel:
-//   K >= 8192 (down): 8 waves per block;
+// The split kernel's launch shape <MT, W, G> that gemm_i8w takes up to 32
+// rows of A when the GEMV kernel does not, or kSmallM for the small-M MFMA kernel:
+//   K >= 8192 (down): 8 waves per block above 16 rows;
 //   N >= 12288 at smaller K (gate/up): 192 or more tiles of 64 rows fill the
 //   GPU with one slice of K, split between two groups of 4 waves per block;
-//   few rows of B (k/v: N = 1024 gives 16 tiles) and M > 32: blocks of 32
-//   rows of A each (token tiles sharing B through one XCD's L2) instead of
-//   one block for all of A: 7-16% faster at M = 64-128 (k/v: 9.0 vs 10.5 us
-//   at M = 96); for larger N, and with 16-row token tiles, slower;
 //   M <= 16 with K and N below 8192: the small-M MFMA kernel.
-enum SplitConfig {
-    kSmallM, kSplitTokenTiles, kSplit881, kSplit842, kSplit841, kSplit481, kSplit442, kSplit441, kSplit281,
-    kSplit242, kSplit241, kSplit142, kSplit141
-};
+enum SplitConfig { kSmallM, kSplit281, kSplit242, kSplit241, kSplit142, kSplit141 };
 SplitConfig split_config(int M, int K, int N) {
     const bool big = K >= 8192 || N >= 8192;
     const bool deep = K >= 8192;
     const bool wide = !deep && N >= 12288;
-    if (!deep && N <= 2048 && M > 32) return kSplitTokenTiles;
-    if (M > 64) return deep ? kSplit881 : wide ? kSplit842 : kSplit841;
-    if (M > 32) return deep ? kSplit481 : wide ? kSplit442 : kSplit441;
     if (M > 16) return deep ? kSplit281 : wide ? kSplit242 : kSplit241;
     if (big) return wide ? kSplit142 : kSplit141;
     return kSmallM;
 }
+
+// ng_gemm_int8_shared_a's paths of the products on the prefill kernel and on
+// the 33 - 128 row kernel.
+constexpr int kPathPrefill = 40, kPathRing2 = 41, kPathRing4 = 42;
+constexpr int kRingMinM = 33;
+
+void ring_slices(int M, int N, int K, int& wk, int& S, int& cps);
+int gemm_ring(int count, void* const* c, const void* a, const void* const* b, const void* const* scales, const int* n,
+              int M, int K, float* scratch = nullptr, size_t scratch_bytes = 0, const ResEpi* ep = nullptr,
+              const SwigluArgs* sw = nullptr);
 
 // The launch shape gemm_i8w takes for a product on the weight-streaming
 // path, for ng_gemm_int8_shared_a: the GEMV shapes 1-3 above, 4 for the
@@ -2058,6 +2321,11 @@ SplitConfig split_config(int M, int K, int N) {
 int shared_path(int M, int K, int N) {
     const int gv = gemv_shape(M, K, N);
     if (gv != 0) return gv;
+    if (M >= kRingMinM) {
+        int wk = 0, S = 0, cps = 0;
+        ring_slices(M, N, K, wk, S, cps);
+        return wk == 2 ? kPathRing2 : kPathRing4;
+    }
     const SplitConfig sc = split_config(M, K, N);
     return sc == kSmallM ? 4 : 10 + static_cast<int>(sc);
 }
@@ -2067,9 +2335,8 @@ int shared_path(int M, int K, int N) {
 // the GEMV kernel up to M = 4 (8 rows of B per block for M <= 2, 4 for M = 3,
 // 4: 23-33% faster than the MFMA kernels at M = 1), the split kernel from
 // M = 17 on and from M = 3 on with K or N of 8192 or more (at M = 4: 13.4 vs
-// 14.8 us for gate/up, 13.7 vs 15.5 us for down), with token tiles of 32 rows
-// of A for N <= 2048 from M = 33 on, otherwise the MFMA kernel that reads A
-// from L2 directly.
+// 14.8 us for gate/up, 13.7 vs 15.5 us for down), the ring kernel from M = 33
+// on, otherwise the MFMA kernel that reads A from L2 directly.
 // With ep, the residual add after the product follows: in the split-K
 // reduction's epilogue where the launch has several K slices, else as
 // cuda_add.
@@ -2088,19 +2355,13 @@ int gemm_i8w(void* c, const void* a, const void* b, const void* scale, int M, in
         case 3: return then_add(launch_gemv<4, 4>(cp, ap, bp, sp, M, N, K));
         default: break;
     }
+    if (M >= kRingMinM) return gemm_ring(1, &c, a, &b, &scale, &N, M, K, scratch, scratch_bytes, ep);
     switch (split_config(M, K, N)) {
-        case kSplitTokenTiles: return launch_split<2, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, (M + 31) / 32, ep);
-        case kSplit881: return launch_split<8, 8, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit842: return launch_split<8, 4, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit841: return launch_split<8, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit481: return launch_split<4, 8, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit442: return launch_split<4, 4, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit441: return launch_split<4, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit281: return launch_split<2, 8, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit242: return launch_split<2, 4, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit241: return launch_split<2, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit142: return launch_split<1, 4, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
-        case kSplit141: return launch_split<1, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, 1, ep);
+        case kSplit281: return launch_split<2, 8, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
+        case kSplit242: return launch_split<2, 4, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
+        case kSplit241: return launch_split<2, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
+        case kSplit142: return launch_split<1, 4, 2>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
+        case kSplit141: return launch_split<1, 4, 1>(cp, ap, bp, sp, M, N, K, scratch, scratch_bytes, ep);
         default: return then_add(launch_i8w<1, 1, 8, 4>(cp, ap, bp, sp, M, N, K));
     }
 }
@@ -2189,7 +2450,7 @@ int run_shared_split(int count, void* const* c, const void* const* b, const void
         return 0;
     }
     if (rblocks == 0) return 0;
-    if (ep) return launch_reduce(st, static_cast<uint16_t*>(c[0]), part, set.scale[0], M, n[0], pl.S[0], ep);
+    if (count == 1) return launch_reduce(st, set.c[0], part, set.scale[0], M, n[0], pl.S[0], ep);
     if (vec4_all || !vec4_any) {
         if (vec4_all)
             split_reduce_shared_kernel<true><<<dim3(static_cast<unsigned>(rblocks)), dim3(256), 0, st>>>(rset, sp, M);
@@ -2331,6 +2592,100 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
     }
 }
 
+// The 33 - 128 row kernel's 64-k groups of a block and K slices of a product,
+// by its M, N and K alone (they show in the bits; tile sizes do not): one slice
+// for wide products (gate/up) and for short K; otherwise slices for about 128
+// blocks of 64 rows of B, twice that for K >= 8192 (four times above 64 rows),
+// each of 1024 k or more. Two groups above 64 rows, where four leave room for
+// two stages only, and for wide products, whose tiles are 128 wide; else four
+// (at 64 rows o 11.8 against 12.3 us, down 20.4 against 21.4, q/k/v 13.7 against
+// 14.6).
+constexpr int kRingWideN = 10240;
+
+void ring_slices(int M, int N, int K, int& wk, int& S, int& cps) {
+    const int tiles = (N + 63) / 64;
+    const bool wide = N >= kRingWideN;
+    wk = M > 64 || wide ? 2 : 4;
+    const int nk = (K + 64 * wk - 1) / (64 * wk);
+    const int target = K >= 8192 ? (M > 64 ? 512 : 256) : 128;
+    S = wide || K <= 2048 ? 1 : max(1, min(min(target / tiles, K / 1024), 8));
+    cps = (nk + S - 1) / S;
+    S = (nk + cps - 1) / cps;
+}
+
+template <int BM, int BN, int WK, int NST>
+int launch_ring(int count, void* const* c, const uint16_t* a, const void* const* b, const void* const* scales,
+                const int* n, int M, int K, SharedPlan& pl, float* scratch, size_t scratch_bytes, const ResEpi* ep,
+                const SwigluArgs* sw) {
+    constexpr int WN = BN / 32;
+    const dim3 block(WN * WK * kWave);
+    const int TT = (M + BM - 1) / BM;
+    const auto blocks_of = [&](long long units) { return TT > 1 ? (units + 7) / 8 * 8 * TT : units; };
+    if (sw && pl.S[0] == 1) {
+        const int tiles = (n[0] + BN / 2 - 1) / (BN / 2);
+        gemm_i8w_ring_swiglu_kernel<BM, BN, WN, WK, NST>
+            <<<dim3(static_cast<unsigned>(blocks_of(tiles))), block, 0, stream()>>>(*sw, a, M, n[0], K, tiles,
+                                                                                    pl.cps[0], TT);
+        NG_CHECK_LAUNCH("ng_gemm_int8_silu_mul");
+        return 0;
+    }
+    for (int i = 0; i < count; ++i) {
+        pl.tm[i] = TT;
+        pl.tn[i] = (n[i] + BN - 1) / BN;
+        pl.blocks[i] = blocks_of(static_cast<long long>(pl.tn[i]) * pl.S[i]);
+    }
+    const TileEpi te{ep && pl.S[0] == 1 ? ep->out : nullptr, ep && pl.S[0] == 1 ? ep->res : nullptr};
+    return run_shared_split(count, c, b, scales, n, M, K, pl,
+                            [&](const SharedSet& set, const SplitSet& sp, unsigned blocks, hipStream_t st) {
+                                if (count == 1)
+                                    gemm_i8w_ring_kernel<BM, BN, WN, WK, NST><<<dim3(blocks), block, 0, st>>>(
+                                        set.c[0], a, set.b[0], set.scale[0], sp.part[0], M, set.n[0], K, sp.S[0],
+                                        sp.tiles[0], sp.cps[0], TT, te);
+                                else
+                                    gemm_i8w_ring_shared_kernel<BM, BN, WN, WK, NST>
+                                        <<<dim3(blocks), block, 0, st>>>(set, sp, a, M, K);
+                            },
+                            sw, scratch, scratch_bytes, ep);
+}
+
+// Products that share A at 33 to 128 rows and take the same groups; other
+// arguments as gemm_tiles. Tile by the number of blocks: wide enough to share A
+// where there are enough of them for the CUs, narrow where not (one product of
+// 4096 rows of B at 64 rows: 11.8 us on tiles of 32, 12.8 on 64; gate alone 19.3
+// on 64, 24.1 on 128), and rows of A cut into tiles of 64 or 32 where even
+// those leave the GPU idle.
+int gemm_ring(int count, void* const* c, const void* a, const void* const* b, const void* const* scales, const int* n,
+              int M, int K, float* scratch, size_t scratch_bytes, const ResEpi* ep, const SwigluArgs* sw) {
+    const auto* ap = static_cast<const uint16_t*>(a);
+    SharedPlan pl{};
+    int wk = 0;
+    long long b64 = 0, b128 = 0;
+    for (int i = 0; i < count; ++i) {
+        ring_slices(M, n[i], K, wk, pl.S[i], pl.cps[i]);
+        b64 += (static_cast<long long>(n[i]) + 63) / 64 * pl.S[i];
+        b128 += (static_cast<long long>(n[i]) + 127) / 128 * pl.S[i];
+    }
+#define NG_RING(BM, BN, WK, NST) \
+    return launch_ring<BM, BN, WK, NST>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw)
+    if (wk == 4) {
+        if (b64 > 128) NG_RING(64, 64, 4, 3);
+        NG_RING(64, 32, 4, 4);
+    }
+    if (M <= 64) {
+        if (b128 >= 128) NG_RING(64, 128, 2, 4);
+        NG_RING(64, 64, 2, 6);
+    }
+    if (b64 <= 64) NG_RING(32, 64, 2, 8);
+    if (b64 <= 128) NG_RING(64, 64, 2, 6);
+    if (b128 >= 160) {
+        if (M <= 96) NG_RING(96, 128, 2, 3);
+        NG_RING(128, 128, 2, 3);
+    }
+    if (M <= 96) NG_RING(96, 64, 2, 5);
+    NG_RING(128, 64, 2, 4);
+#undef NG_RING
+}
+
 int gemm_prefill(void* c, const void* a, const void* b, const void* scale, int M, int K, int N,
                  float* scratch = nullptr, size_t scratch_bytes = 0, const ResEpi* ep = nullptr) {
     return gemm_tiles(1, &c, a, &b, &scale, &N, M, K, scratch, scratch_bytes, ep);
@@ -2450,15 +2805,13 @@ extern "C" int ng_gemm_int8_noalloc(void* c, const void* a, const void* b, const
 // The split kernel's shared form: slices and blocks as launch_split.
 template <int MT, int W, int G>
 int launch_split_shared(int count, void* const* c, const uint16_t* a, const void* const* b,
-                        const void* const* scales, const int* n, int M, int K, int TT,
+                        const void* const* scales, const int* n, int M, int K,
                         const SwigluArgs* sw = nullptr) {
     SharedPlan pl{};
     for (int i = 0; i < count; ++i) {
         pl.tn[i] = (n[i] + 16 * W - 1) / (16 * W);
-        pl.tm[i] = TT;
-        split_slices(pl.tn[i], TT, G, K, pl.S[i], pl.cps[i]);
-        const long long units = static_cast<long long>(pl.tn[i]) * pl.S[i];
-        pl.blocks[i] = TT > 1 ? (units + 7) / 8 * 8 * TT : units;
+        split_slices(pl.tn[i], G, K, pl.S[i], pl.cps[i]);
+        pl.blocks[i] = static_cast<long long>(pl.tn[i]) * pl.S[i];
     }
     return run_shared_split(count, c, b, scales, n, M, K, pl,
                             [&](const SharedSet& set, const SplitSet& sp, unsigned blocks, hipStream_t st) {
@@ -2466,9 +2819,6 @@ int launch_split_shared(int count, void* const* c, const uint16_t* a, const void
                                     <<<dim3(blocks), dim3(G * W * kWave), 0, st>>>(set, sp, a, M, K);
                             }, sw);
 }
-
-// ng_gemm_int8_shared_a's path of the products on the prefill kernel.
-constexpr int kPathPrefill = 40;
 
 // One group of products that take the same launch shape `path` (see
 // shared_path), in one launch of that kernel's shared form; shapes without a
@@ -2478,16 +2828,12 @@ int shared_group(int path, int count, void* const* c, const void* a, const void*
     const auto* ap = static_cast<const uint16_t*>(a);
     if (count > 1) {
         switch (path) {
-            case 10 + kSplitTokenTiles:
-                return launch_split_shared<2, 4, 1>(count, c, ap, b, scales, n, M, K, (M + 31) / 32);
-            case 10 + kSplit141: return launch_split_shared<1, 4, 1>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit241: return launch_split_shared<2, 4, 1>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit441: return launch_split_shared<4, 4, 1>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit841: return launch_split_shared<8, 4, 1>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit142: return launch_split_shared<1, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit242: return launch_split_shared<2, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit442: return launch_split_shared<4, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
-            case 10 + kSplit842: return launch_split_shared<8, 4, 2>(count, c, ap, b, scales, n, M, K, 1);
+            case 10 + kSplit141: return launch_split_shared<1, 4, 1>(count, c, ap, b, scales, n, M, K);
+            case 10 + kSplit241: return launch_split_shared<2, 4, 1>(count, c, ap, b, scales, n, M, K);
+            case 10 + kSplit142: return launch_split_shared<1, 4, 2>(count, c, ap, b, scales, n, M, K);
+            case 10 + kSplit242: return launch_split_shared<2, 4, 2>(count, c, ap, b, scales, n, M, K);
+            case kPathRing2:
+            case kPathRing4: return gemm_ring(count, c, ap, b, scales, n, M, K);
             case kPathPrefill: return gemm_tiles(count, c, ap, b, scales, n, M, K);
             default: break;
         }
@@ -2720,7 +3066,7 @@ template <int MT, int W, int G>
 int launch_split_swiglu(const SwigluArgs& sa, const uint16_t* a, int M, int N, int K) {
     const int tn = (N + 16 * W - 1) / (16 * W);  // tiles of one product's own launch
     int S = 0, cps = 0;
-    split_slices(tn, 1, G, K, S, cps);
+    split_slices(tn, G, K, S, cps);
     if (S != 1) return 1;
     const unsigned blocks = static_cast<unsigned>((N + 8 * W - 1) / (8 * W));
     gemm_i8w_split_swiglu_kernel<MT, W, G><<<dim3(blocks), dim3(G * W * kWave), 0, stream()>>>(sa, a, M, N, K, cps);
@@ -2736,18 +3082,14 @@ static int swiglu_sliced(const SwigluArgs& sa, const uint16_t* a, int M, int K, 
     const void* sc[2] = {sa.sg, sa.su};
     const int n[2] = {N, N};
     switch (shared_path(M, K, N)) {
-        case 10 + kSplit141: return launch_split_shared<1, 4, 1>(2, c, a, b, sc, n, M, K, 1, &sa);
-        case 10 + kSplit241: return launch_split_shared<2, 4, 1>(2, c, a, b, sc, n, M, K, 1, &sa);
-        case 10 + kSplit441: return launch_split_shared<4, 4, 1>(2, c, a, b, sc, n, M, K, 1, &sa);
-        case 10 + kSplit841: return launch_split_shared<8, 4, 1>(2, c, a, b, sc, n, M, K, 1, &sa);
+        case 10 + kSplit141: return launch_split_shared<1, 4, 1>(2, c, a, b, sc, n, M, K, &sa);
+        case 10 + kSplit241: return launch_split_shared<2, 4, 1>(2, c, a, b, sc, n, M, K, &sa);
         default: return 1;
     }
 }
 
 static int swiglu_split(const SwigluArgs& sa, const uint16_t* a, int M, int K, int N) {
     switch (split_config(M, K, N)) {
-        case kSplit842: return launch_split_swiglu<8, 4, 2>(sa, a, M, N, K);
-        case kSplit442: return launch_split_swiglu<4, 4, 2>(sa, a, M, N, K);
         case kSplit242: return launch_split_swiglu<2, 4, 2>(sa, a, M, N, K);
         case kSplit142: return launch_split_swiglu<1, 4, 2>(sa, a, M, N, K);
         default: return 1;
@@ -2778,6 +3120,13 @@ extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void
                         static_cast<const int8_t*>(b_gate), static_cast<const int8_t*>(b_up),
                         static_cast<const float*>(scale_gate), static_cast<const float*>(scale_up)};
     if (path < 1 && apart && use_i8w(a, b_gate, M, K, N, true) && use_i8w(a, b_up, M, K, N, true)) {
+        if (M >= kRingMinM) {
+            void* c[2] = {gate, up};
+            const void* b[2] = {b_gate, b_up};
+            const void* sc[2] = {scale_gate, scale_up};
+            const int n[2] = {N, N};
+            return gemm_ring(2, c, a, b, sc, n, M, K, nullptr, 0, nullptr, &sa);
+        }
         int r = swiglu_split(sa, static_cast<const uint16_t*>(a), M, K, N);
         if (r == 1) r = swiglu_sliced(sa, static_cast<const uint16_t*>(a), M, K, N);
         if (r <= 0) return r;

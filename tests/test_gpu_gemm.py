@@ -479,7 +479,14 @@ def test_reference_kat_gemm_transpose(lib):
 # step after none, one or more whole ones), with K slices, with N that no 16-byte
 # store divides and with C off 16 bytes. Inputs whose sums are exact in fp32, so
 # every tile shape and slice count has to give the same bits.
-TILE_EDGES = [(129, 16, 1), (129, 64, 127), (191, 80, 129), (192, 128, 128), (193, 192, 255), (255, 208, 257),
+# Likewise the kernel of 33 to 128 rows: each tile of 32, 64, 96 and 128 rows by
+# 32, 64 and 128, row tiles that end early, two and four groups, one and several
+# K slices, 64-k parts past K, fewer steps than stages.
+TILE_EDGES = [(33, 64, 1), (33, 128, 127), (64, 192, 129), (65, 320, 130), (96, 448, 10300), (97, 2048, 300),
+              (128, 4160, 1000), (127, 64, 10240), (64, 8256, 257), (100, 11008, 132), (128, 14336, 4099),
+              (64, 4160, 9000), (50, 2112, 10300), (34, 192, 20500), (70, 4160, 5000), (66, 4288, 9000),
+              (90, 192, 20500), (128, 192, 20500), (110, 4160, 9000),
+              (129, 16, 1), (129, 64, 127), (191, 80, 129), (192, 128, 128), (193, 192, 255), (255, 208, 257),
               (257, 256, 300), (384, 320, 4097), (385, 336, 4100), (511, 1024, 14344), (1025, 2048, 8200),
               (130, 14336, 512), (333, 11008, 1000), (200, 8208, 66)]
 
@@ -498,10 +505,12 @@ def test_int8_prefill_tile_edges(lib, M, K, N):
 
 
 @pytest.mark.parametrize("M,K,N,off", [(333, 1024, 4096, 0), (1000, 4096, 14336, 0), (200, 1040, 1002, 0),
-                                       (257, 128, 257, 2)])
+                                       (257, 128, 257, 2), (40, 4096, 14336, 0), (100, 192, 10250, 0),
+                                       (128, 4096, 1000, 0), (64, 1024, 10241, 2)])
 def test_int8_prefill_epilogues(lib, M, K, N, off):
-    """SwiGLU and the residual add in the prefill kernel's epilogue give the bits
-    of the calls they replace, also with out in place and off 16 bytes."""
+    """SwiGLU and the residual add in the epilogue (one K slice) or the reduction
+    of the kernels above 32 rows give the bits of the calls they replace, also with
+    out in place and off 16 bytes."""
     banner(f"gemm_int8 prefill epilogues M={M} K={K} N={N} off={off}")
     a, res = f16bits(RNG.standard_normal((M, K))), f16bits(RNG.standard_normal((M, N)))
     qg, qu = codes((N, K)), codes((N, K))
