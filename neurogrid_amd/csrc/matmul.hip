@@ -57,6 +57,7 @@
 
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <map>
@@ -1435,7 +1436,10 @@ __device__ __forceinline__ void store_out8(uint16_t* c, size_t o, int n_ok, cons
     }
 }
 
-template <int BM, int BN, int WM, int WN, int NST, bool SW>
+// SERIAL: a block takes all K slices of its tile (S = 1; cps: a slice's steps),
+// one after the other, and adds each sum to those before it as the reduction
+// does: the bits of a launch with a block per slice, without its partial sums.
+template <int BM, int BN, int WM, int WN, int NST, bool SW, bool SERIAL = false>
 __device__ __forceinline__ void gemm_i8w_tile_block(
     uint16_t* c, const uint16_t* __restrict__ a, const int8_t* __restrict__ b, const float* __restrict__ scale,
     float* __restrict__ part, int M, int N, int K, int tiles_m, int tiles_n, int S, int cps, int blk,
@@ -1571,7 +1575,7 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    const int c0 = sl * cps, c1 = min(nk, c0 + cps);
+    const int c0 = SERIAL ? 0 : sl * cps, c1 = SERIAL ? nk : min(nk, c0 + cps);
     const int n = c1 - c0;                            // steps of this block
     const int full = c1 == nk && krem ? n - 1 : n;    // of them whole ones
     u32x4 fa[2][TM], cb[2][TN];
@@ -1621,6 +1625,21 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
     };
     int i0 = 0;
     if (full > 0) step(i0++, std::false_type{});
+    [[maybe_unused]] f32x16 sum[SERIAL ? TM : 1][SERIAL ? TN : 1] = {};  // of the slices before
+    if constexpr (SERIAL) {
+        for (int end = cps; end < n; end += cps) {
+            const int stop = min(end, full);
+            for (; i0 + NST < n && i0 < stop; ++i0) step(i0, std::true_type{});
+            for (; i0 < stop; ++i0) step(i0, std::false_type{});
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = f32x16{};
+                }
+        }
+    }
     for (; i0 + NST < n && i0 < full; ++i0) step(i0, std::true_type{});
     for (; i0 < full; ++i0) step(i0, std::false_type{});
     if (full < n) {
@@ -1645,6 +1664,12 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
         }
     }
 
+    if constexpr (SERIAL) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j] + acc[i][j];
+    }
     // acc[i][j][4 q + e] is C[m0 + wm TM 32 + 32 i + l % 32][n0 + wn TN 32 + 32 j + 8 q + 4 (l / 32) + e].
     if (S > 1) {
         float* mine = part + static_cast<size_t>(sl) * M * N;
@@ -1706,12 +1731,12 @@ __device__ __forceinline__ void gemm_i8w_tile_block(
 // product's tiles along N and `TT` its tiles along M. ep follows the product of
 // a launch of one with one K slice (out may be c or res itself: each element
 // is read and written by one thread, out last).
-template <int BM, int BN, int WM, int WN, int NST>
+template <int BM, int BN, int WM, int WN, int NST, bool SERIAL>
 __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_kernel(SharedSet s, SplitSet sp,
                                                                            const uint16_t* __restrict__ a, int M,
                                                                            int K, TileEpi ep) {
     shared_dispatch(s, [&](uint16_t* c, const int8_t* b, const float* scale, int n, int blk, int p) {
-        gemm_i8w_tile_block<BM, BN, WM, WN, NST, false>(
+        gemm_i8w_tile_block<BM, BN, WM, WN, NST, false, SERIAL>(
             c, a, b, scale, pick4(p, sp.part[0], sp.part[1], sp.part[2], sp.part[3]), M, n, K,
             pick4(p, sp.TT[0], sp.TT[1], sp.TT[2], sp.TT[3]),
             pick4(p, sp.tiles[0], sp.tiles[1], sp.tiles[2], sp.tiles[3]),
@@ -2467,29 +2492,39 @@ int run_shared_split(int count, void* const* c, const void* const* b, const void
     return 0;
 }
 
-// Tile shapes of the prefill kernel, <BM, BN, WM, WN, NST>, and the time of a
-// step of 64 k in us on MI355X: lo with up to 96 blocks on the GPU, hi with 256
-// (the clock falls as the matrix cores fill). Fitted to launches of 96 to 1792
-// tiles at K = 4096 and 14336: 256 x 256 at 2048 x 4096 (128 tiles) 95.6 us, at
-// 4096 x 4096 (256 tiles) 122; 128 x 256 54.4 us at 1024 x 4096 (128), 71.4 at
-// 2048 x 4096 (256); 128 x 128 29.4 us at 333 x 4096 (96), 40.4 at 1024 x 4096
-// (256), 251 at 1024 x 28672 (1792); 64 x 128 27.3 us at 333 x 4096 (192).
-// Also measured and slower than the best of these wherever they could be
-// taken: 256 x 128, 64 x 256, and 128 x 128 with 4 waves or 6 stages.
+// Tile shapes of the prefill kernel, <BM, BN, 2, 4, NST>, and the time of a
+// launch on each on MI355X, in us: fixed, plus for each step of 64 k of a block
+// lo with few blocks on the GPU, rising from a share `knee` of the 256 CUs to hi
+// at one block for each (the clock falls as the matrix cores fill), and more for
+// every full round of a launch of several. Fitted to 544 launches of
+// M = 130 - 3000 at N = 1024 - 28672, K = 2048 - 14336 with 1 - 8 slices on every
+// shape; taken by it a launch is at most 10% (0.5% on average) above the fastest
+// of all shapes and slices. The 192 row tiles are for M that 128 and 256 divide
+// badly (gate/up of 333 rows, 4096 -> 2 x 14336: 90 us, 107 on 256 x 256; of 190
+// rows 57, 70 on 128 x 256) and in slices for down (900 x 4096 x 14336: 116 us
+// in three, 138 on 128 x 256). Also measured and slower than the best of these
+// wherever they could be taken: 64 x 256, 64 x 64, 128 x 128 with 4 waves or 6
+// stages, and 4 x 2 waves on 256 x 128.
 struct TileShape {
     int BM, BN;
-    double lo, hi;
+    double fixed, lo, hi, knee, more;
 };
-constexpr TileShape kTileShapes[] = {{256, 256, 1.38, 1.84}, {128, 256, 0.78, 1.08}, {128, 128, 0.40, 0.57},
-                                     {64, 128, 0.32, 0.38}};
-constexpr int kTileShapeCount = 4;
+constexpr TileShape kTileShapes[] = {
+    {256, 256, 9.1, 1.097, 1.534, 0.49, 1.694}, {192, 256, 8.4, 0.899, 1.236, 0.56, 1.353},
+    {256, 128, 7.3, 0.653, 0.906, 0.47, 0.994}, {128, 256, 7.3, 0.714, 0.969, 0.61, 1.025},
+    {192, 128, 6.4, 0.507, 0.732, 0.45, 0.792}, {128, 128, 5.3, 0.425, 0.587, 0.54, 0.527},
+    {64, 128, 4.4, 0.324, 0.398, 0.58, 0.349}};
+constexpr int kTileShapeCount = 7, kTileSerialFirst = 2;
 
-// Time of a launch of `blocks` blocks whose steps add up to `steps`, the
-// longest taking `longest`: 6 us, then a round of steps for each 256 blocks.
-double tile_time(const TileShape& ts, long long blocks, long long steps, int longest) {
-    const double fill = blocks < 96 ? 0.0 : blocks > 256 ? 1.0 : (blocks - 96) / 160.0;
-    const double rounds = static_cast<double>((blocks + 255) / 256) * (static_cast<double>(steps) / blocks);
-    return 6.0 + (ts.lo + (ts.hi - ts.lo) * fill) * (rounds > longest ? rounds : longest);
+// Time of a launch of `blocks` blocks whose steps add up to `steps`.
+double tile_time(const TileShape& ts, long long blocks, long long steps) {
+    const long long full = blocks / 256;
+    const double rest = static_cast<double>(blocks % 256) / 256.0;
+    double step;
+    if (full == 0) step = ts.lo + (rest > ts.knee ? (ts.hi - ts.lo) * (rest - ts.knee) / (1.0 - ts.knee) : 0.0);
+    else if (rest == 0.0) step = full == 1 ? ts.hi : ts.more * full;
+    else step = ts.more * full + ts.lo + (ts.more - ts.lo) * rest;
+    return ts.fixed + step * (static_cast<double>(steps) / blocks);
 }
 
 long long tile_blocks(const TileShape& ts, int M, int N, int S) {
@@ -2500,9 +2535,9 @@ long long tile_blocks(const TileShape& ts, int M, int N, int S) {
 // so that a product has the same bits in every launch that it is part of.
 // The S <= 8 of least time over the tile shapes, each slice of 8 steps or more
 // and the partial sums within the fixed array of ng_gemm_int8_noalloc, the
-// reduction counted as 4 us and its bytes at 5 TB/s; more than one only where
-// it saves 5% (333 x 4096 x 14336: 62 us with two slices, 95 with one; 130 x
-// 4096 x 4096 20.7 us with slices, 26.8 with one).
+// reduction counted as 3 us and 0.3 us a MB of partial sums; more than one only
+// where it saves 2% (333 x 4096 x 14336: 57 us with four slices, 83 with one;
+// 130 x 4096 x 4096 19 us with two, 25 with one).
 void prefill_slices(int M, int N, int K, int& S, int& cps) {
     const int nk = (K + kPfBK - 1) / kPfBK;
     double one = 0.0, best = 0.0;
@@ -2515,12 +2550,12 @@ void prefill_slices(int M, int N, int K, int& S, int& cps) {
         double t = 0.0;
         for (const TileShape& ts : kTileShapes) {
             const long long blocks = tile_blocks(ts, M, N, ss);
-            const double v = tile_time(ts, blocks, blocks / ss * nk, per);
+            const double v = tile_time(ts, blocks, blocks / ss * nk);
             if (t == 0.0 || v < t) t = v;
         }
-        if (ss > 1) t += 4.0 + 2.0 * bytes / 5e6;
+        if (ss > 1) t += 3.0 + 0.3e-6 * bytes;
         if (s == 1) one = best = t;
-        if (s > 1 && t < 0.95 * one && t < best) {
+        if (s > 1 && t < 0.98 * one && t < best) {
             best = t;
             S = ss;
             cps = per;
@@ -2528,7 +2563,7 @@ void prefill_slices(int M, int N, int K, int& S, int& cps) {
     }
 }
 
-template <int BM, int BN, int WM, int WN, int NST>
+template <int BM, int BN, int WM, int WN, int NST, bool SERIAL = false>
 int launch_tiles(int count, void* const* c, const uint16_t* a, const void* const* b, const void* const* scales,
                  const int* n, int M, int K, SharedPlan& pl, float* scratch, size_t scratch_bytes, const ResEpi* ep,
                  const SwigluArgs* sw) {
@@ -2548,7 +2583,7 @@ int launch_tiles(int count, void* const* c, const uint16_t* a, const void* const
     const TileEpi te{ep && pl.S[0] == 1 ? ep->out : nullptr, ep && pl.S[0] == 1 ? ep->res : nullptr};
     return run_shared_split(count, c, b, scales, n, M, K, pl,
                             [&](const SharedSet& set, const SplitSet& sp, unsigned blocks, hipStream_t st) {
-                                gemm_i8w_tile_kernel<BM, BN, WM, WN, NST>
+                                gemm_i8w_tile_kernel<BM, BN, WM, WN, NST, SERIAL>
                                     <<<dim3(blocks), block, 0, st>>>(set, sp, a, M, K, te);
                             },
                             sw, scratch, scratch_bytes, ep);
@@ -2558,6 +2593,13 @@ int launch_tiles(int count, void* const* c, const uint16_t* a, const void* const
 // reduction where a product has K slices), on the tile shape of least time for
 // all of them. ep (a product alone): the residual add after it. sw (gate and
 // up): SwiGLU after them.
+// Of several products narrow ones have slices that pay alone but not beside a
+// wide one, whose blocks fill the GPU meanwhile: there a block takes all slices
+// of its tile, with the same bits, where that is the faster estimate, on the
+// shapes whose second set of sums fits in registers (q/k/v of 4096, 1024 and
+// 1024 rows, K = 4096, with k and v in 4 slices: 512 rows 38 against 48 us, 700
+// rows 45 against 55; with 8 slices at 190 rows a block per slice stays faster,
+// 26 against 27).
 int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, const void* const* scales,
                const int* n, int M, int K, float* scratch = nullptr, size_t scratch_bytes = 0,
                const ResEpi* ep = nullptr, const SwigluArgs* sw = nullptr) {
@@ -2565,31 +2607,61 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
     SharedPlan pl{};
     const int nk = (K + kPfBK - 1) / kPfBK;
     int longest = 0;
+    double reduce = 0.0;
     for (int i = 0; i < count; ++i) {
         prefill_slices(M, n[i], K, pl.S[i], pl.cps[i]);
         longest = max(longest, pl.cps[i]);
+        if (pl.S[i] > 1) reduce += (reduce == 0.0 ? 3.0 : 0.0) + 0.3e-6 * sizeof(float) * pl.S[i] * M * n[i];
     }
-    int shape = 0;
+    // The shape of least time, with a block per slice and with all slices in one.
+    const auto best = [&](bool serial, int first, double& least) {
+        int shape = first;
+        for (int k = first; k < kTileShapeCount; ++k) {
+            long long blocks = 0, steps = 0;
+            for (int i = 0; i < count; ++i) {
+                const long long bl = tile_blocks(kTileShapes[k], M, n[i], serial ? 1 : pl.S[i]);
+                blocks += bl;
+                steps += serial ? bl * nk : bl / pl.S[i] * nk;
+            }
+            double t = tile_time(kTileShapes[k], blocks, steps);
+            if (!serial) t = reduce + std::max(t, kTileShapes[k].fixed + kTileShapes[k].lo * longest);
+            if (k == first || t < least) {
+                least = t;
+                shape = k;
+            }
+        }
+        return shape;
+    };
     double least = 0.0;
-    for (int k = 0; k < kTileShapeCount; ++k) {
-        long long blocks = 0, steps = 0;
-        for (int i = 0; i < count; ++i) {
-            const long long bl = tile_blocks(kTileShapes[k], M, n[i], pl.S[i]);
-            blocks += bl;
-            steps += bl / pl.S[i] * nk;
-        }
-        const double t = tile_time(kTileShapes[k], blocks, steps, longest);
-        if (k == 0 || t < least) {
-            least = t;
-            shape = k;
+    const int shape = best(false, 0, least);
+    if (count > 1 && !sw && reduce > 0.0) {
+        double least_serial = 0.0;
+        const int serial = best(true, kTileSerialFirst, least_serial);
+        if (1.02 * least_serial < least) {
+            for (int i = 0; i < count; ++i) pl.S[i] = 1;
+#define NG_TILES(BM, BN, NST) return launch_tiles<BM, BN, 2, 4, NST, true>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw)
+            switch (serial) {
+                case 2: NG_TILES(256, 128, 3);
+                case 3: NG_TILES(128, 256, 4);
+                case 4: NG_TILES(192, 128, 3);
+                case 5: NG_TILES(128, 128, 3);
+                default: NG_TILES(64, 128, 4);
+            }
+#undef NG_TILES
         }
     }
+#define NG_TILES(BM, BN, NST) \
+    return launch_tiles<BM, BN, 2, 4, NST>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw)
     switch (shape) {
-        case 0: return launch_tiles<256, 256, 2, 4, 3>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
-        case 1: return launch_tiles<128, 256, 2, 4, 4>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
-        case 2: return launch_tiles<128, 128, 2, 4, 3>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
-        default: return launch_tiles<64, 128, 2, 4, 4>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
+        case 0: NG_TILES(256, 256, 3);
+        case 1: NG_TILES(192, 256, 3);
+        case 2: NG_TILES(256, 128, 3);
+        case 3: NG_TILES(128, 256, 4);
+        case 4: NG_TILES(192, 128, 3);
+        case 5: NG_TILES(128, 128, 3);
+        default: NG_TILES(64, 128, 4);
     }
+#undef NG_TILES
 }
 
 // The 33 - 128 row kernel's 64-k groups of a block and K slices of a product,

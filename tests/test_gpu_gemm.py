@@ -488,7 +488,8 @@ TILE_EDGES = [(33, 64, 1), (33, 128, 127), (64, 192, 129), (65, 320, 130), (96, 
               (90, 192, 20500), (128, 192, 20500), (110, 4160, 9000),
               (129, 16, 1), (129, 64, 127), (191, 80, 129), (192, 128, 128), (193, 192, 255), (255, 208, 257),
               (257, 256, 300), (384, 320, 4097), (385, 336, 4100), (511, 1024, 14344), (1025, 2048, 8200),
-              (130, 14336, 512), (333, 11008, 1000), (200, 8208, 66)]
+              (130, 14336, 512), (333, 11008, 1000), (200, 8208, 66), (255, 528, 8200), (257, 528, 14340),
+              (257, 528, 28700), (769, 528, 14340), (255, 1040, 20500), (640, 1040, 8200), (900, 8256, 4090)]
 
 
 @pytest.mark.parametrize("M,K,N", TILE_EDGES)

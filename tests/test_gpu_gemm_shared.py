@@ -134,6 +134,20 @@ def separate(lib, a, qs, scales, M, K):
     return out
 
 
+# Narrow products beside a wide one at prefill lengths, sliced along K alone:
+# in the set a block takes all slices of its tile, on each tile shape that does
+# so, with a partial last step and N off the tiles.
+@pytest.mark.parametrize("M,K,ns", [(333, 2064, [2048, 256, 250]), (512, 4096, [4096, 1024, 1024]),
+                                    (700, 4112, [4096, 1000, 1024]), (1025, 4160, [4096, 1024, 1000]),
+                                    (600, 8208, [8200, 1000, 77]), (256, 4112, [30000, 600]),
+                                    (300, 8208, [7000, 500, 66])])
+def test_shared_a_prefill_slices_bit_for_bit(lib, M, K, ns):
+    banner(f"gemm_int8_shared_a prefill slices M={M} K={K} n={ns}")
+    a, qs, scales = problem(M, K, ns, exact=False)
+    for g, w in zip(shared(lib, a, qs, scales, M, K), separate(lib, a, qs, scales, M, K)):
+        assert_bits_equal(g, w)
+
+
 @pytest.mark.parametrize("M,K,ns", SETS)
 def test_shared_a_is_cuda_gemm_int8_bit_for_bit(lib, M, K, ns):
     banner(f"gemm_int8_shared_a random M={M} K={K} n={ns}")
