@@ -2252,6 +2252,19 @@ int partial_buffer(hipStream_t s, int S, int M, int N, int K, float* scratch, si
     return 0;
 }
 
+// Whether partial_buffer can give `need` bytes on stream s: not when they would
+// have to be allocated while it is captured.
+bool partial_room(hipStream_t s, size_t need) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        if (need <= g_buffers[{dev, s}].part_bytes) return true;
+    }
+    bool cap = false;
+    return capturing(s, &cap) == 0 && !cap;
+}
+
 // C = fp16(scale[n] * sum of the S slices of part), slices added in order.
 int launch_reduce(hipStream_t s, uint16_t* c, const float* part, const float* scale, int M, int N, int S,
                   const ResEpi* ep = nullptr) {
@@ -2598,8 +2611,9 @@ int launch_tiles(int count, void* const* c, const uint16_t* a, const void* const
 // of its tile, with the same bits, where that is the faster estimate, on the
 // shapes whose second set of sums fits in registers (q/k/v of 4096, 1024 and
 // 1024 rows, K = 4096, with k and v in 4 slices: 512 rows 38 against 48 us, 700
-// rows 45 against 55; with 8 slices at 190 rows a block per slice stays faster,
-// 26 against 27).
+// rows 45 against 55; with slices of 2, 8 and 8 at 190 rows 27 against 26). A
+// launch under capture that finds no buffer for its partial sums does the same
+// (not with sw: 1 is returned before launching anything).
 int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, const void* const* scales,
                const int* n, int M, int K, float* scratch = nullptr, size_t scratch_bytes = 0,
                const ResEpi* ep = nullptr, const SwigluArgs* sw = nullptr) {
@@ -2607,12 +2621,16 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
     SharedPlan pl{};
     const int nk = (K + kPfBK - 1) / kPfBK;
     int longest = 0;
-    double reduce = 0.0;
+    size_t cols = 0;  // of partial sums
     for (int i = 0; i < count; ++i) {
         prefill_slices(M, n[i], K, pl.S[i], pl.cps[i]);
         longest = max(longest, pl.cps[i]);
-        if (pl.S[i] > 1) reduce += (reduce == 0.0 ? 3.0 : 0.0) + 0.3e-6 * sizeof(float) * pl.S[i] * M * n[i];
+        if (pl.S[i] > 1) cols += static_cast<size_t>(pl.S[i]) * n[i];
     }
+    const size_t part_bytes = sizeof(float) * cols * M;
+    const double reduce = cols > 0 ? 3.0 + 0.3e-6 * part_bytes : 0.0;
+    const bool room = cols == 0 || scratch != nullptr || partial_room(stream(), part_bytes + 4 * sizeof(float) * M);
+    if (sw && !room) return 1;
     // The shape of least time, with a block per slice and with all slices in one.
     const auto best = [&](bool serial, int first, double& least) {
         int shape = first;
@@ -2634,10 +2652,10 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
     };
     double least = 0.0;
     const int shape = best(false, 0, least);
-    if (count > 1 && !sw && reduce > 0.0) {
+    if (!sw && cols > 0 && (count > 1 || !room)) {
         double least_serial = 0.0;
         const int serial = best(true, kTileSerialFirst, least_serial);
-        if (1.02 * least_serial < least) {
+        if (!room || 1.02 * least_serial < least) {
             for (int i = 0; i < count; ++i) pl.S[i] = 1;
 #define NG_TILES(BM, BN, NST) return launch_tiles<BM, BN, 2, 4, NST, true>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw)
             switch (serial) {
@@ -3208,7 +3226,8 @@ extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void
         const void* b[2] = {b_gate, b_up};
         const void* sc[2] = {scale_gate, scale_up};
         const int n[2] = {N, N};
-        return gemm_tiles(2, c, a, b, sc, n, M, K, nullptr, 0, nullptr, &sa);
+        const int r = gemm_tiles(2, c, a, b, sc, n, M, K, nullptr, 0, nullptr, &sa);
+        if (r <= 0) return r;
     }
     if (path < 1 || !apart) {
         void* c[2] = {gate, up};

@@ -341,3 +341,46 @@ def test_capture_survives_buffer_growth(lib, inp, capture_stream):
     finally:
         for b in (a, w, sc, big):
             b.free()
+
+
+# Products with K slices at prefill lengths, captured on a stream that holds no
+# buffer for their partial sums: a block takes all slices of its tile, same bits.
+@pytest.mark.parametrize("M,K,N", [(900, 8256, 4096), (333, 11008, 4099)])
+def test_capture_prefill_without_warmup(lib, capture_stream, M, K, N):
+    hip, stream = capture_stream
+    banner(f"graph capture without an eager call: prefill M={M} K={K} N={N}")
+    rng = np.random.Generator(np.random.PCG64(5))
+    a = dev(f16_bits(rng.standard_normal((M, K)).astype(np.float32)))
+    w = [dev(rng.integers(-127, 128, (N, K)).astype(np.int8)) for _ in range(2)]
+    sc = dev(rng.uniform(1e-5, 1e-4, N).astype(np.float32))
+    res = dev(f16_bits(rng.standard_normal((M, N)).astype(np.float32)))
+    outs = [empty(M * N * 2) for _ in range(6)]
+    y, s, c, g, u, o = [b.vp for b in outs]
+
+    def calls():
+        ok(lib.cuda_gemm_int8(y, a.vp, w[0].vp, sc.vp, M, K, N, True), "gemm")
+        ok(lib.ng_gemm_int8_add(s, c, a.vp, w[0].vp, sc.vp, res.vp, M, K, N), "add")
+        ok(lib.ng_gemm_int8_silu_mul(o, g, u, a.vp, w[0].vp, sc.vp, w[1].vp, sc.vp, M, K, N), "silu_mul")
+
+    try:
+        graph, ex = hip.capture(stream, calls)
+        try:
+            got = []
+            for _ in range(3):
+                for b in outs:
+                    b.upload(np.zeros(M * N, np.uint16))
+                hip.launch(ex, stream)
+                got.append([get(b, np.uint16, (M, N)) for b in outs])
+            for b in outs:
+                b.upload(np.zeros(M * N, np.uint16))
+            calls()
+            hip.check(hip.h.hipStreamSynchronize(stream), "hipStreamSynchronize")
+            want = [get(b, np.uint16, (M, N)) for b in outs]
+        finally:
+            hip.destroy(graph, ex)
+        for rep in got:
+            for name, x, v in zip(("gemm", "add", "c", "gate", "up", "out"), rep, want):
+                assert_bits_equal(x, v, name)
+    finally:
+        for b in (a, sc, res, *w, *outs):
+            b.free()
