@@ -877,8 +877,8 @@ def shared_a_extras(L, hip, stream):
         grp.free()
     out["note"] = ("us: one ng_gemm_int8_shared_a call (one launch per group of products with the same launch "
                    "shape: the GEMV kernel at 1-2 tokens, the small-M MFMA kernel for q/k/v at 8, the split kernel "
-                   "and its reduction up to 128 tokens (at 64 q alone and k/v together), the fused prefill kernel "
-                   "and its reduction above); separate_us: one cuda_gemm_int8 call per projection")
+                   "up to 32 tokens, the 33-128 row kernel up to 128, the fused prefill kernel above, each with its "
+                   "reduction); separate_us: one cuda_gemm_int8 call per projection")
     return out
 
 
@@ -952,9 +952,9 @@ def norm_shared_extras(L, hip, stream):
 def silu_mul_gemm_extras(L, hip, stream, K=4096, N=14336):
     """The gate/up projections and SwiGLU (layer.cu:575-588) at M = 1, 2, 4, 8
     and 64 tokens, Mistral-7B's by default (N = 11008: Llama-2-7B's). us:
-    ng_gemm_int8_silu_mul (the GEMV kernel at M <= 2 here; from 3 rows the
-    split kernel's SwiGLU form, or with K slices (N = 11008) one shared split
-    launch and the reduction's SwiGLU form);
+    ng_gemm_int8_silu_mul (the GEMV kernel at M <= 2 here; above, the
+    fused kernels' SwiGLU forms, or with K slices (N = 11008 up to 32 rows) one
+    shared launch and the reduction's SwiGLU form);
     two_calls_us: ng_gemm_int8_shared_a, then cuda_silu_mul. Both give the same bits; weight pools keep the codes
     cache-cold."""
     rng = np.random.Generator(np.random.PCG64(8))
@@ -1000,9 +1000,9 @@ def silu_mul_gemm_extras(L, hip, stream, K=4096, N=14336):
 def gemm_add_extras(L, hip, stream, K=14336, N=4096):
     """Mistral-7B's down projection and the layer's final residual add
     (layer.cu:593-598) at M = 1, 2, 4, 8, 64, 512 and 2048 tokens. us:
-    ng_gemm_int8_add (one launch on the GEMV kernel's shapes, M <= 2 here; from
-    3 tokens the split kernel, and from 129 the prefill kernel, with the add in
-    the reduction of their K slices); two_calls_us: cuda_gemm_int8, then
+    ng_gemm_int8_add (one launch on the GEMV kernel's shapes, M <= 2 here; above,
+    the other fused kernels with the add in the reduction of their K slices or
+    in their epilogue); two_calls_us: cuda_gemm_int8, then
     cuda_add. Both give the same bits; weight pools keep
     the codes cache-cold."""
     rng = np.random.Generator(np.random.PCG64(9))

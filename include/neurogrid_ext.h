@@ -187,10 +187,10 @@ int ng_rmsnorm_qkv_rope_int8(void* normed, void* q, void* k, void* v, const void
  * for bit. With no output overlapping an input or another output (out may
  * be gate or up itself, as the engine's in-place call), one launch computes
  * all three when both products take the GEMV kernel (M <= 4, aligned
- * pointers) or, up to 128 rows, the split kernel with one K slice (wide
+ * pointers) or, up to 4095 rows, another fused kernel with one K slice (wide
  * products, e.g. Mistral-7B's gate/up); with several K slices (e.g.
- * Llama-2-7B's gate/up) one shared split launch and one reduction that also
- * writes SwiGLU; otherwise this is the two calls. B is [N, K] (transpose_b).
+ * Llama-2-7B's gate/up at 3 to 32 rows) one shared launch and one reduction
+ * that also writes SwiGLU; otherwise this is the two calls. B is [N, K] (transpose_b).
  * Returns 0 or -1. */
 int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void* a, const void* b_gate,
                           const void* scale_gate, const void* b_up, const void* scale_up, int M, int K, int N);
@@ -200,9 +200,9 @@ int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void* a, const 
  * true), then cuda_add(out, c, residual, M N), bit for bit. With no output
  * overlapping an input or the other output (out may be c or residual
  * itself): on the GEMV kernel's shapes (M <= 4, aligned pointers) one launch
- * writes both; on the split-K kernel (up to 128 rows) and the prefill kernel
- * (up to 4095) the add runs in the reduction of their K slices. Otherwise
- * this is the two calls. Returns 0 or -1. */
+ * writes both; up to 4095 rows the add runs in the reduction of the K slices
+ * or, from 33 rows with one slice, in the product's launch. Otherwise this is
+ * the two calls. Returns 0 or -1. */
 int ng_gemm_int8_add(void* out, void* c, const void* a, const void* b, const void* scale,
                      const void* residual, int M, int K, int N);
 

@@ -134,7 +134,7 @@ struct SharedSet {
 
 // Per-product split-K parameters (gemm_i8w_split_shared_kernel): the
 // product's partial-sum region, its slice count, tiles of B, batches per
-// slice and token tiles.
+// slice and row tiles.
 struct SplitSet {
     float* part[kMaxShared];
     int S[kMaxShared];
@@ -2354,8 +2354,8 @@ int gemm_ring(int count, void* const* c, const void* a, const void* const* b, co
 
 // The launch shape gemm_i8w takes for a product on the weight-streaming
 // path, for ng_gemm_int8_shared_a: the GEMV shapes 1-3 above, 4 for the
-// small-M MFMA kernel, 10 + c for split shape c (10-22; the prefill kernel's
-// shapes are kPathPrefill128 and kPathPrefill256).
+// small-M MFMA kernel, 10 + c for split shape c, kPathRing2 or kPathRing4 by the
+// groups of the 33 - 128 row kernel.
 int shared_path(int M, int K, int N) {
     const int gv = gemv_shape(M, K, N);
     if (gv != 0) return gv;
@@ -2376,8 +2376,8 @@ int shared_path(int M, int K, int N) {
 // 14.8 us for gate/up, 13.7 vs 15.5 us for down), the ring kernel from M = 33
 // on, otherwise the MFMA kernel that reads A from L2 directly.
 // With ep, the residual add after the product follows: in the split-K
-// reduction's epilogue where the launch has several K slices, else as
-// cuda_add.
+// reduction's epilogue where the launch has several K slices, in the ring
+// kernel's where it has one, else as cuda_add.
 int gemm_i8w(void* c, const void* a, const void* b, const void* scale, int M, int K, int N,
              float* scratch = nullptr, size_t scratch_bytes = 0, const ResEpi* ep = nullptr) {
     auto* cp = static_cast<uint16_t*>(c);
@@ -2411,7 +2411,7 @@ bool use_prefill(const void* a, const void* b, int M, int K, int N, bool transpo
 }
 
 // Per-product plan of a shared split-K launch: K slices, batches per slice,
-// tiles along N and along M (the split kernel: token tiles), and blocks.
+// tiles along N and along M, and blocks.
 struct SharedPlan {
     int S[kMaxShared], cps[kMaxShared], tn[kMaxShared], tm[kMaxShared];
     long long blocks[kMaxShared];
@@ -2873,7 +2873,7 @@ extern "C" int cuda_gemm_int8(void* c, const void* a, const void* b, const void*
 // fused prefill kernel, where cuda_gemm_int8 runs the dequantize + hipBLASLt
 // composition. Every call on a device shares that device's
 // array: calls that overlap on one GPU (other streams, other host threads)
-// race on it. The split kernel writes every partial sum before the reduction
+// race on it. The kernels write every partial sum before the reduction
 // reads it, so nothing needs clearing between calls.
 extern "C" int ng_gemm_int8_noalloc(void* c, const void* a, const void* b, const void* scale, int M, int K, int N,
                                     bool transpose_b) {
@@ -3189,10 +3189,10 @@ static int swiglu_split(const SwigluArgs& sa, const uint16_t* a, int M, int K, i
 // gate/up (cuda_gemm_int8 on one A, as ng_gemm_int8_shared_a) and SwiGLU
 // (cuda_silu_mul), when no output overlaps an input or another output (out
 // may be gate or up exactly): one launch of gemv_i8w_swiglu_kernel when both
-// products take the GEMV kernel, one of gemm_i8w_split_swiglu_kernel when
-// they take the split kernel with one K slice, the shared split launch and
-// split_reduce_swiglu_kernel when they take a one-group split shape with
-// several K slices; otherwise the two calls. The same bits either way.
+// products take the GEMV kernel, one of gemm_i8w_split_swiglu_kernel (33 to 128
+// rows: _ring_, above and below kLtMinM: _tile_) when they take that kernel with
+// one K slice, its shared launch and split_reduce_swiglu_kernel when they have
+// several; otherwise the two calls. The same bits either way.
 extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void* a, const void* b_gate,
                                      const void* scale_gate, const void* b_up, const void* scale_up, int M, int K,
                                      int N) {
@@ -3256,9 +3256,9 @@ extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void
 // output (out may be c or the residual exactly), one launch of
 // gemv_i8w_add_kernel on the GEMV kernel's shapes, and on cuda_gemm_int8's
 // other fused paths (the weight-streaming kernels up to 128 rows, the prefill
-// kernel below kLtMinM) the add in the split-K reduction (after the product as
-// cuda_add where the launch has one K slice); otherwise the two calls. The
-// same bits either way.
+// kernel below kLtMinM) the add in the split-K reduction, or with one K slice in
+// the epilogue of the 33 - 128 row and the prefill kernel (up to 32 rows after
+// the product as cuda_add); otherwise the two calls. The same bits either way.
 extern "C" int ng_gemm_int8_add(void* out, void* c, const void* a, const void* b, const void* scale,
                                 const void* residual, int M, int K, int N) {
     NG_REQUIRE(out && c && a && b && scale && residual, "ng_gemm_int8_add: null pointer");
@@ -3273,7 +3273,7 @@ extern "C" int ng_gemm_int8_add(void* out, void* c, const void* a, const void* b
     if (path < 1 || !apart) {
         // cuda_gemm_int8's own fused paths (the weight-streaming kernels up to
         // 128 rows of A, the prefill kernel below kLtMinM): the add in the
-        // split-K reduction where the launch has one.
+        // split-K reduction or the epilogue.
         const ResEpi ep{static_cast<uint16_t*>(out), static_cast<const uint16_t*>(residual)};
         if (apart && use_i8w(a, b, M, K, N, true)) return gemm_i8w(c, a, b, scale, M, K, N, nullptr, 0, &ep);
         if (apart && M < kLtMinM && use_prefill(a, b, M, K, N, true))
