@@ -2184,10 +2184,10 @@ int gemm_lt(void* c, const void* a, const void* b, const void* q, const void* sc
 // of the weights in this (device, stream)'s buffer, grown to the largest
 // weight seen (117 MB for a 14336 x 4096 projection), where the reference
 // allocates and frees one per call. Measured on MI355X at M = 4096 for
-// Mistral-7B's projections: 115 us for q/o against 161 us for the fused
-// prefill kernel, 424 against 531 for gate/up, 367 against 467 for down, 48
-// against 59 for k/v; at M = 512 the fused kernel is faster (37 against
-// 42 us for q/o). Between 512 and 4096 rows the composition is not measured,
+// Mistral-7B's projections, eager calls back to back: 108-116 us for q/o against
+// 116-125 us for the fused prefill kernel, 371 against 410 for gate or up, 337
+// against 373 for down, 47 against 42 for k/v (not worth a rule of its own).
+// Between 512 and 4096 rows the composition is not measured,
 // so the fused kernel keeps those sizes. Returns 1 when hipBLASLt has no
 // algorithm for the shape or refuses the call (remembered for the shape),
 // having written nothing but the fp16 buffer: the caller then runs the fused
