@@ -2227,19 +2227,17 @@ int gemm_lt_rows(void* c, const void* a, const void* q, const void* scale, int M
     return 0;
 }
 
-// The fp32 partial-sum buffer [S][M][N] of a split-K launch: `scratch` when
-// the caller brings one (refused when too small), else this (device,
+// The buffer of a split-K launch's `need` bytes of fp32 partial sums: `scratch`
+// when the caller brings one (refused when too small), else this (device,
 // stream)'s buffer, grown on demand with `lock` (g_mu) taken; the caller
 // keeps the lock until both kernels are enqueued, so that calls from other
 // host threads on the same stream cannot slip a launch between them.
-int partial_buffer(hipStream_t s, int S, int M, int N, int K, float* scratch, size_t scratch_bytes,
+int partial_buffer(hipStream_t s, size_t need, float* scratch, size_t scratch_bytes,
                    std::unique_lock<std::mutex>& lock, float** out) {
-    const size_t need = static_cast<size_t>(S) * M * N * sizeof(float);
     if (scratch != nullptr) {
         NG_REQUIRE(need <= scratch_bytes,
-                   "ng_gemm_int8_noalloc: M=%d K=%d N=%d splits K into %d slices whose partial sums need %zu "
-                   "bytes, more than the %zu-byte scratch; call cuda_gemm_int8 instead",
-                   M, K, N, S, need, scratch_bytes);
+                   "ng_gemm_int8_noalloc: the partial sums of the slices of K need %zu bytes, more than the "
+                   "%zu-byte scratch; call cuda_gemm_int8 instead", need, scratch_bytes);
         *out = scratch;
         return 0;
     }
@@ -2307,7 +2305,8 @@ int launch_split(uint16_t* c, const uint16_t* a, const int8_t* b, const float* s
     const hipStream_t s = stream();
     float* part = nullptr;
     std::unique_lock<std::mutex> lock(g_mu, std::defer_lock);
-    if (S > 1 && partial_buffer(s, S, M, N, K, scratch, scratch_bytes, lock, &part) != 0) return -1;
+    const size_t need = static_cast<size_t>(S) * M * N * sizeof(float);
+    if (S > 1 && partial_buffer(s, need, scratch, scratch_bytes, lock, &part) != 0) return -1;
     gemm_i8w_split_kernel<MT, W, G><<<dim3(static_cast<unsigned>(tiles * S)), dim3(G * W * kWave), 0, s>>>(
         c, a, b, scale, part, M, N, K, S, cps);
     NG_CHECK_LAUNCH("cuda_gemm_int8");
@@ -2417,6 +2416,19 @@ struct SharedPlan {
     long long blocks[kMaxShared];
 };
 
+// Floats of partial sums of a launch of `count` products, the regions of those
+// with K slices one after the other, each on 16 bytes; the starts in `at`.
+size_t partial_floats(int count, const int* n, int M, const int* S, size_t* at = nullptr) {
+    size_t end = 0;
+    for (int i = 0; i < count; ++i) {
+        if (S[i] == 1) continue;
+        const size_t start = (end + 3) / 4 * 4;
+        if (at != nullptr) at[i] = start;
+        end = start + static_cast<size_t>(S[i]) * M * n[i];
+    }
+    return end;
+}
+
 // Products that share A on one split-K kernel shape: one launch of the kernel
 // (`launch(set, sp, blocks, stream)`), then one of the reduction for the products with
 // more than one slice of K, each product with its own slices and its own
@@ -2431,19 +2443,15 @@ int run_shared_split(int count, void* const* c, const void* const* b, const void
                      int M, int K, const SharedPlan& pl, L&& launch, const SwigluArgs* sw = nullptr,
                      float* scratch = nullptr, size_t scratch_bytes = 0, const ResEpi* ep = nullptr) {
     if (sw && !(count == 2 && n[0] == n[1] && pl.S[0] > 1 && pl.S[1] == pl.S[0])) return 1;
-    long long cols = 0;
-    for (int i = 0; i < count; ++i)
-        if (pl.S[i] > 1) cols += static_cast<long long>(pl.S[i]) * n[i];
-    // Each product's region starts on 16 bytes: up to 3 floats of padding each.
-    if (cols > 0 && count > 1) cols += 4;
-    NG_REQUIRE(cols < (1ll << 31), "ng_gemm_int8_shared_a: too many rows of B");
+    size_t at[kMaxShared] = {};
+    const size_t floats = partial_floats(count, n, M, pl.S, at);
     const hipStream_t st = stream();
     float* part = nullptr;
     std::unique_lock<std::mutex> lock(g_mu, std::defer_lock);
-    if (cols > 0 && partial_buffer(st, 1, M, static_cast<int>(cols), K, scratch, scratch_bytes, lock, &part) != 0) return -1;
+    if (floats > 0 && partial_buffer(st, floats * sizeof(float), scratch, scratch_bytes, lock, &part) != 0) return -1;
     SharedSet set{}, rset{};
     SplitSet sp{};
-    long long blocks = 0, rblocks = 0, off = 0;
+    long long blocks = 0, rblocks = 0;
     bool vec4_all = true, vec4_any = false;
     for (int i = 0; i < kMaxShared; ++i) {
         const int j = i < count ? i : 0;  // unused slots repeat product 0 and are never selected
@@ -2461,8 +2469,7 @@ int run_shared_split(int count, void* const* c, const void* const* b, const void
         if (i >= count) continue;
         blocks += pl.blocks[i];
         if (pl.S[i] > 1) {
-            sp.part[i] = part + off;
-            off += (static_cast<long long>(pl.S[i]) * M * n[i] + 3) / 4 * 4;
+            sp.part[i] = part + at[i];
             const bool v4 = n[i] % 4 == 0 && aligned16(scales[i]) && aligned8(c[i]);
             vec4_all = vec4_all && v4;
             vec4_any = vec4_any || v4;
@@ -2621,15 +2628,13 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
     SharedPlan pl{};
     const int nk = (K + kPfBK - 1) / kPfBK;
     int longest = 0;
-    size_t cols = 0;  // of partial sums
     for (int i = 0; i < count; ++i) {
         prefill_slices(M, n[i], K, pl.S[i], pl.cps[i]);
         longest = max(longest, pl.cps[i]);
-        if (pl.S[i] > 1) cols += static_cast<size_t>(pl.S[i]) * n[i];
     }
-    const size_t part_bytes = sizeof(float) * cols * M;
-    const double reduce = cols > 0 ? 3.0 + 0.3e-6 * part_bytes : 0.0;
-    const bool room = cols == 0 || scratch != nullptr || partial_room(stream(), part_bytes + 4 * sizeof(float) * M);
+    const size_t part_bytes = sizeof(float) * partial_floats(count, n, M, pl.S);
+    const double reduce = part_bytes > 0 ? 3.0 + 0.3e-6 * part_bytes : 0.0;
+    const bool room = part_bytes == 0 || scratch != nullptr || partial_room(stream(), part_bytes);
     if (sw && !room) return 1;
     // The shape of least time, with a block per slice and with all slices in one.
     const auto best = [&](bool serial, int first, double& least) {
@@ -2652,7 +2657,7 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
     };
     double least = 0.0;
     const int shape = best(false, 0, least);
-    if (!sw && cols > 0 && (count > 1 || !room)) {
+    if (!sw && part_bytes > 0 && (count > 1 || !room)) {
         double least_serial = 0.0;
         const int serial = best(true, kTileSerialFirst, least_serial);
         if (!room || 1.02 * least_serial < least) {

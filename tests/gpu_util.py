@@ -92,14 +92,42 @@ class HipRuntime:
         self.h.hipGraphDestroy.argtypes = [vp]
         self.h.hipStreamSynchronize.argtypes = [vp]
         self.h.hipStreamDestroy.argtypes = [vp]
+        self.h.hipGraphGetNodes.argtypes = [vp, C.POINTER(vp), C.POINTER(C.c_size_t)]
+        self.h.hipGraphNodeGetType.argtypes = [vp, C.POINTER(C.c_int)]
 
     def check(self, rc, what):
         assert rc == 0, f"{what} failed with hipError {rc}"
 
+    handles: set[int] = set()  # of every stream this process got here
+
     def stream(self):
         s = C.c_void_p()
         self.check(self.h.hipStreamCreate(C.byref(s)), "hipStreamCreate")
+        self.handles.add(s.value)
         return s
+
+    def unused_stream(self):
+        """A stream whose handle no earlier stream had: the library keeps its
+        buffers by handle, and the runtime hands handles out again."""
+        seen, tried = set(self.handles), []
+        while not tried or tried[-1].value in seen:
+            assert len(tried) < 64, "no new stream handle"
+            tried.append(self.stream())
+        for s in tried[:-1]:
+            self.h.hipStreamDestroy(s)
+        return tried[-1]
+
+    def kernel_nodes(self, graph):
+        """How many kernels a captured graph launches; every node has to be one."""
+        n = C.c_size_t(0)
+        self.check(self.h.hipGraphGetNodes(graph, None, C.byref(n)), "hipGraphGetNodes")
+        nodes = (C.c_void_p * n.value)()
+        self.check(self.h.hipGraphGetNodes(graph, nodes, C.byref(n)), "hipGraphGetNodes")
+        for node in nodes:
+            kind = C.c_int(-1)
+            self.check(self.h.hipGraphNodeGetType(node, C.byref(kind)), "hipGraphNodeGetType")
+            assert kind.value == 0, f"graph node of type {kind.value}"  # hipGraphNodeTypeKernel
+        return n.value
 
     def capture(self, stream, fn):
         """Capture the launches `fn` makes on `stream` (relaxed mode); returns (graph, exec)."""

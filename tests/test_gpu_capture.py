@@ -343,11 +343,35 @@ def test_capture_survives_buffer_growth(lib, inp, capture_stream):
             b.free()
 
 
+@pytest.fixture()
+def cold_stream(lib):
+    """A stream for which the library holds no buffer yet."""
+    hip = HipRuntime()
+    stream = hip.unused_stream()
+    lib.ng_set_stream(stream)
+    try:
+        yield hip, stream
+    finally:
+        lib.ng_set_stream(None)
+        hip.h.hipStreamDestroy(stream)
+
+
+def kernels_captured(hip, stream, call, label):
+    """Kernel launches that `call` records."""
+    graph, ex = hip.capture(stream, lambda: ok(call(), f"{label} under capture"))
+    try:
+        return hip.kernel_nodes(graph)
+    finally:
+        hip.destroy(graph, ex)
+
+
 # Products with K slices at prefill lengths, captured on a stream that holds no
-# buffer for their partial sums: a block takes all slices of its tile, same bits.
+# buffer for their partial sums: a block takes all slices of its tile, one
+# launch for the product and its add, same bits; after a call of the shape the
+# slices have blocks of their own and the reduction follows, as in the call.
 @pytest.mark.parametrize("M,K,N", [(900, 8256, 4096), (333, 11008, 4099)])
-def test_capture_prefill_without_warmup(lib, capture_stream, M, K, N):
-    hip, stream = capture_stream
+def test_capture_prefill_without_warmup(lib, cold_stream, M, K, N):
+    hip, stream = cold_stream
     banner(f"graph capture without an eager call: prefill M={M} K={K} N={N}")
     rng = np.random.Generator(np.random.PCG64(5))
     a = dev(f16_bits(rng.standard_normal((M, K)).astype(np.float32)))
@@ -357,12 +381,20 @@ def test_capture_prefill_without_warmup(lib, capture_stream, M, K, N):
     outs = [empty(M * N * 2) for _ in range(6)]
     y, s, c, g, u, o = [b.vp for b in outs]
 
+    def gemm():
+        return lib.cuda_gemm_int8(y, a.vp, w[0].vp, sc.vp, M, K, N, True)
+
+    def add():
+        return lib.ng_gemm_int8_add(s, c, a.vp, w[0].vp, sc.vp, res.vp, M, K, N)
+
     def calls():
-        ok(lib.cuda_gemm_int8(y, a.vp, w[0].vp, sc.vp, M, K, N, True), "gemm")
-        ok(lib.ng_gemm_int8_add(s, c, a.vp, w[0].vp, sc.vp, res.vp, M, K, N), "add")
+        ok(gemm(), "gemm")
+        ok(add(), "add")
         ok(lib.ng_gemm_int8_silu_mul(o, g, u, a.vp, w[0].vp, sc.vp, w[1].vp, sc.vp, M, K, N), "silu_mul")
 
     try:
+        assert kernels_captured(hip, stream, gemm, "gemm") == 1
+        assert kernels_captured(hip, stream, add, "add") == 1
         graph, ex = hip.capture(stream, calls)
         try:
             got = []
@@ -373,6 +405,9 @@ def test_capture_prefill_without_warmup(lib, capture_stream, M, K, N):
                 got.append([get(b, np.uint16, (M, N)) for b in outs])
             for b in outs:
                 b.upload(np.zeros(M * N, np.uint16))
+            ok(gemm(), "gemm")
+            assert kernels_captured(hip, stream, gemm, "gemm after a call") == 2
+            assert kernels_captured(hip, stream, add, "add after a call") == 2
             calls()
             hip.check(hip.h.hipStreamSynchronize(stream), "hipStreamSynchronize")
             want = [get(b, np.uint16, (M, N)) for b in outs]
@@ -383,4 +418,32 @@ def test_capture_prefill_without_warmup(lib, capture_stream, M, K, N):
                 assert_bits_equal(x, v, name)
     finally:
         for b in (a, sc, res, *w, *outs):
+            b.free()
+
+
+# Products that share A: the capture after a call of the set records what the
+# call launched (the slices of narrow products as blocks of their own).
+@pytest.mark.parametrize("M,K,ns", [(333, 11008, [1024, 1024, 1024]), (64, 4096, [4096, 1024, 1024]),
+                                    (333, 14336, [999, 1001])])
+def test_capture_of_a_set_after_a_call(lib, cold_stream, M, K, ns):
+    hip, stream = cold_stream
+    banner(f"graph capture of a set after a call M={M} K={K} n={ns}")
+    rng = np.random.Generator(np.random.PCG64(6))
+    a = dev(f16_bits(rng.standard_normal((M, K)).astype(np.float32)))
+    w = [dev(rng.integers(-127, 128, (n, K)).astype(np.int8)) for n in ns]
+    sc = [dev(rng.uniform(1e-5, 1e-4, n).astype(np.float32)) for n in ns]
+    outs = [empty(M * n * 2) for n in ns]
+    p = len(ns)
+    args = ((C.c_void_p * p)(*[b.ptr for b in outs]), (C.c_void_p * p)(*[b.ptr for b in w]),
+            (C.c_void_p * p)(*[b.ptr for b in sc]), (C.c_int * p)(*ns))
+
+    def shared():
+        return lib.ng_gemm_int8_shared_a(p, args[0], a.vp, args[1], args[2], args[3], M, K)
+
+    try:
+        ok(shared(), "set")
+        hip.check(hip.h.hipStreamSynchronize(stream), "hipStreamSynchronize")
+        assert kernels_captured(hip, stream, shared, "set") == 2
+    finally:
+        for b in (a, *w, *sc, *outs):
             b.free()
