@@ -2748,7 +2748,9 @@ int launch_ring(int count, void* const* c, const uint16_t* a, const void* const*
 // where there are enough of them for the CUs, narrow where not (one product of
 // 4096 rows of B at 64 rows: 11.8 us on tiles of 32, 12.8 on 64; gate alone 19.3
 // on 64, 24.1 on 128), and rows of A cut into tiles of 64 or 32 where even
-// those leave the GPU idle.
+// those leave the GPU idle. Several products on a stream under capture whose
+// buffer holds the partial sums of each but not of all of them: one launch each
+// (with sw 1 is returned before launching anything), as separate calls.
 int gemm_ring(int count, void* const* c, const void* a, const void* const* b, const void* const* scales, const int* n,
               int M, int K, float* scratch, size_t scratch_bytes, const ResEpi* ep, const SwigluArgs* sw) {
     const auto* ap = static_cast<const uint16_t*>(a);
@@ -2759,6 +2761,13 @@ int gemm_ring(int count, void* const* c, const void* a, const void* const* b, co
         ring_slices(M, n[i], K, wk, pl.S[i], pl.cps[i]);
         b64 += (static_cast<long long>(n[i]) + 63) / 64 * pl.S[i];
         b128 += (static_cast<long long>(n[i]) + 127) / 128 * pl.S[i];
+    }
+    const size_t floats = partial_floats(count, n, M, pl.S);
+    if (count > 1 && floats > 0 && !partial_room(stream(), floats * sizeof(float))) {
+        if (sw) return 1;
+        for (int i = 0; i < count; ++i)
+            if (gemm_ring(1, c + i, a, b + i, scales + i, n + i, M, K) != 0) return -1;
+        return 0;
     }
 #define NG_RING(BM, BN, WK, NST) \
     return launch_ring<BM, BN, WK, NST>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw)
@@ -3220,11 +3229,13 @@ extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void
             const void* b[2] = {b_gate, b_up};
             const void* sc[2] = {scale_gate, scale_up};
             const int n[2] = {N, N};
-            return gemm_ring(2, c, a, b, sc, n, M, K, nullptr, 0, nullptr, &sa);
+            const int r = gemm_ring(2, c, a, b, sc, n, M, K, nullptr, 0, nullptr, &sa);
+            if (r <= 0) return r;
+        } else {
+            int r = swiglu_split(sa, static_cast<const uint16_t*>(a), M, K, N);
+            if (r == 1) r = swiglu_sliced(sa, static_cast<const uint16_t*>(a), M, K, N);
+            if (r <= 0) return r;
         }
-        int r = swiglu_split(sa, static_cast<const uint16_t*>(a), M, K, N);
-        if (r == 1) r = swiglu_sliced(sa, static_cast<const uint16_t*>(a), M, K, N);
-        if (r <= 0) return r;
     } else if (path < 1 && apart && M < kLtMinM && use_prefill(a, b_gate, M, K, N, true) &&
                use_prefill(a, b_up, M, K, N, true) && !use_i8w(a, b_gate, M, K, N, true)) {
         void* c[2] = {gate, up};

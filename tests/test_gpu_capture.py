@@ -447,3 +447,53 @@ def test_capture_of_a_set_after_a_call(lib, cold_stream, M, K, ns):
     finally:
         for b in (a, *w, *sc, *outs):
             b.free()
+
+
+# A set at 33 - 128 rows whose products were called one by one before: the
+# buffer holds the partial sums of the largest, not of all, and the set is
+# captured as the separate launches.
+@pytest.mark.parametrize("M,K,ns,kernels", [(64, 4096, [4096, 1024, 1024], 6), (128, 4096, [2048, 1024], 4)])
+def test_capture_of_a_set_after_its_products(lib, cold_stream, M, K, ns, kernels):
+    hip, stream = cold_stream
+    banner(f"graph capture of a set after its products M={M} K={K} n={ns}")
+    rng = np.random.Generator(np.random.PCG64(8))
+    a = dev(f16_bits(rng.standard_normal((M, K)).astype(np.float32)))
+    w = [dev(rng.integers(-127, 128, (n, K)).astype(np.int8)) for n in ns]
+    sc = [dev(rng.uniform(1e-5, 1e-4, n).astype(np.float32)) for n in ns]
+    outs = [empty(M * n * 2) for n in ns]
+    p = len(ns)
+    args = ((C.c_void_p * p)(*[b.ptr for b in outs]), (C.c_void_p * p)(*[b.ptr for b in w]),
+            (C.c_void_p * p)(*[b.ptr for b in sc]), (C.c_int * p)(*ns))
+
+    def separate():
+        for c, b, s, n in zip(outs, w, sc, ns):
+            ok(lib.cuda_gemm_int8(c.vp, a.vp, b.vp, s.vp, M, K, n, True), "gemm")
+        hip.check(hip.h.hipStreamSynchronize(stream), "hipStreamSynchronize")
+
+    def shared():
+        return lib.ng_gemm_int8_shared_a(p, args[0], a.vp, args[1], args[2], args[3], M, K)
+
+    def read():
+        return [get(c, np.uint16, (M, n)) for c, n in zip(outs, ns)]
+
+    try:
+        separate()
+        graph, ex = hip.capture(stream, lambda: ok(shared(), "set under capture"))
+        try:
+            assert hip.kernel_nodes(graph) == kernels
+            got = []
+            for _ in range(3):
+                for c, n in zip(outs, ns):
+                    c.upload(np.zeros((M, n), np.uint16))
+                hip.launch(ex, stream)
+                got.append(read())
+            separate()
+            want = read()
+        finally:
+            hip.destroy(graph, ex)
+        for rep in got:
+            for x, v in zip(rep, want):
+                assert_bits_equal(x, v)
+    finally:
+        for b in (a, *w, *sc, *outs):
+            b.free()
