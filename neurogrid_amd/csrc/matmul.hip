@@ -1763,9 +1763,9 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_swiglu_kerne
 // rows of B also reads its K slice of A from L2, and both have to be in flight
 // ahead of the matrix cores. One tile of all rows of A x BN rows of B per block:
 //   * stages of WK x 64 k, NST of them, go straight into LDS as in the prefill
-//     kernel, NST - 1 steps ahead: 64 to 96 KiB in flight per CU and one barrier
-//     per step (the kernel this replaces staged both through registers one step
-//     ahead);
+//     kernel, NST - 1 steps ahead: 80 to 128 KiB in flight per CU (one block, or
+//     two of the small tiles) and one barrier per step (the kernel this replaces
+//     staged both through registers one step ahead);
 //   * the WK groups of WN waves multiply different 64 k of a stage, each wave
 //     all rows of A by 32 rows of B, so a fragment of A feeds as many MFMAs as
 //     the tile is wide and B is converted once; the groups' sums meet in LDS at
@@ -1781,8 +1781,11 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_swiglu_kerne
 // Mistral-7B at 64 rows 16.0 against 22.7 us, o 11.2 against 12.0, gate/up with
 // SwiGLU 32.4 against 39.0; at 128 rows 21.7 against 29.7, 14.1 against 17.1, 46.3
 // against 67.3, down 31.2 against 32.1; gate/up of TinyLlama at 64 rows 11.2
-// against 18.1. Slower are k/v alone (N = 1024: 8.3 against 7.6 us at 64 rows) and
-// three products of 4096 rows of B at 33 - 48 rows (23.1 against 20.2 at 33).
+// against 18.1; k/v alone (N = 1024) 7.2 against 7.5, three products of 4096 rows
+// of B at 33 and 64 rows 18.0 against 20.6 and 21.6 against 25.9. Up to 6% slower at 33 -
+// 64 rows: one wide product of K >= 5120 whose blocks of 64 rows of B take most of
+// the GPU's CUs (13824 x 5120 at 64 rows 25.9 against 24.7), since a CU then runs 4
+// waves; two of them, or one with SwiGLU, are faster.
 // Bound at 64 rows: gate/up move 117 MB of weights in 32 us (3.7 TB/s) and A 224
 // times from L2 (as much again); 8 or 16 us calls are launch, first loads and the
 // reduction.
@@ -1792,7 +1795,10 @@ __device__ __forceinline__ void load_lds16_nt(__amdgpu_buffer_rsrc_t r, uint32_t
                  : "memory");
 }
 
-template <int BM, int BN, int WN, int WK, int NST, bool SW>
+// SERIAL: a block takes both K slices of its tile (S = 1; cps: the first one's
+// steps), one after the other, and adds the second sum to the first as the
+// reduction does: the bits of a launch with a block per slice, without its partial sums.
+template <int BM, int BN, int WN, int WK, int NST, bool SW, bool SERIAL = false>
 __device__ __forceinline__ void gemm_i8w_ring_block(uint16_t* c, const uint16_t* __restrict__ a,
                                                     const int8_t* __restrict__ b, const float* __restrict__ scale,
                                                     float* __restrict__ part, int Mall, int N, int K, int S,
@@ -1885,7 +1891,7 @@ __device__ __forceinline__ void gemm_i8w_ring_block(uint16_t* c, const uint16_t*
     const uint32_t boff = static_cast<uint32_t>(kABytes + kg / 2 * kB128 + br * 128 +
                                                 (((4 * (kg & 1) + grp) ^ ((br >> 1) & 7)) << 4));
 
-    const int c0 = sl * cps, c1 = min(nk, c0 + cps), n = c1 - c0;
+    const int c0 = SERIAL ? 0 : sl * cps, c1 = SERIAL ? nk : min(nk, c0 + cps), n = c1 - c0;
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s)
         if (s < n) load(c0 + s, s);
@@ -1932,6 +1938,19 @@ __device__ __forceinline__ void gemm_i8w_ring_block(uint16_t* c, const uint16_t*
         st = st + 1 == NST ? 0 : st + 1;
     };
     int i0 = 0;
+    [[maybe_unused]] f32x16 first[SERIAL ? TM : 1];  // the first slice's sums
+    const bool two = SERIAL && cps < n;
+    if constexpr (SERIAL) {
+        if (two) {
+            for (; i0 + NST - 1 < n && i0 < cps; ++i0) step(i0, std::true_type{});
+            for (; i0 < cps; ++i0) step(i0, std::false_type{});
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            first[i] = acc[i];
+            acc[i] = f32x16{};
+        }
+    }
     for (; i0 + NST - 1 < n && i0 < full; ++i0) step(i0, std::true_type{});
     for (; i0 < full; ++i0) step(i0, std::false_type{});
     if (full < n) {
@@ -1945,13 +1964,15 @@ __device__ __forceinline__ void gemm_i8w_ring_block(uint16_t* c, const uint16_t*
     lds_read_barrier();  // the stages are free (their last loads were waited for)
 
     // acc[i][4 q + e] is this group's sum for row 32 i + l % 32, column 32 wn + 8 q + 4 (l / 32) + e.
+    if constexpr (!SERIAL) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<f32x4*>(lds + (kg * BM + 32 * i + (lane & 31)) * kRow + 4 * (32 * wn + 8 * q + 4 * grp)) =
-                f32x4{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
-    __syncthreads();
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<f32x4*>(lds + (kg * BM + 32 * i + (lane & 31)) * kRow + 4 * (32 * wn + 8 * q + 4 * grp)) =
+                    f32x4{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+        __syncthreads();
+    }
     // Eight columns from `col` of row r, groups added in order.
     const auto sums8 = [&](int r, int col, float (&v)[8]) {
 #pragma unroll
@@ -1964,12 +1985,38 @@ __device__ __forceinline__ void gemm_i8w_ring_block(uint16_t* c, const uint16_t*
         }
     };
     constexpr int kPieces = BNC / 8;
+    [[maybe_unused]] float head[8];  // of this thread's piece: the first slice
+    if constexpr (SERIAL) {
+        static_assert(BM * kPieces == NW * kWave, "one piece per thread");
+        const auto put = [&](const f32x16 (&x)[TM]) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f32x4*>(lds + (kg * BM + 32 * i + (lane & 31)) * kRow +
+                                              4 * (32 * wn + 8 * q + 4 * grp)) =
+                        f32x4{x[i][4 * q], x[i][4 * q + 1], x[i][4 * q + 2], x[i][4 * q + 3]};
+            __syncthreads();
+        };
+        if (two) {
+            put(first);
+            sums8(tid / kPieces, 8 * (tid % kPieces), head);
+            __syncthreads();
+        }
+        put(acc);
+    }
     const bool vec = S > 1 ? N % 4 == 0 : out_vec<SW>(c, N, ep, sw);
     for (int p = tid; p < BM * kPieces; p += NW * kWave) {
         const int r = p / kPieces, q = p % kPieces, nn = n0 + 8 * q;
         if (r >= M || nn >= N) continue;
         float v[8];
         sums8(r, 8 * q, v);
+        if constexpr (SERIAL) {
+            if (two) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = head[e] + v[e];
+            }
+        }
         if (S > 1) {
             float* o = part + (static_cast<size_t>(sl) * Mall + m0 + r) * N + nn;
             if (vec) {
@@ -2007,12 +2054,12 @@ __global__ __launch_bounds__(WN * WK * kWave, 1) void gemm_i8w_ring_kernel(
 }
 
 // Products that share A, as gemm_i8w_tile_kernel.
-template <int BM, int BN, int WN, int WK, int NST>
+template <int BM, int BN, int WN, int WK, int NST, bool SERIAL>
 __global__ __launch_bounds__(WN * WK * kWave, 1) void gemm_i8w_ring_shared_kernel(SharedSet s, SplitSet sp,
                                                                                   const uint16_t* __restrict__ a,
                                                                                   int M, int K) {
     shared_dispatch(s, [&](uint16_t* c, const int8_t* b, const float* scale, int n, int blk, int p) {
-        gemm_i8w_ring_block<BM, BN, WN, WK, NST, false>(
+        gemm_i8w_ring_block<BM, BN, WN, WK, NST, false, SERIAL>(
             c, a, b, scale, pick4(p, sp.part[0], sp.part[1], sp.part[2], sp.part[3]), M, n, K,
             pick4(p, sp.S[0], sp.S[1], sp.S[2], sp.S[3]), pick4(p, sp.tiles[0], sp.tiles[1], sp.tiles[2], sp.tiles[3]),
             pick4(p, sp.cps[0], sp.cps[1], sp.cps[2], sp.cps[3]), pick4(p, sp.TT[0], sp.TT[1], sp.TT[2], sp.TT[3]),
@@ -2688,27 +2735,40 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
 }
 
 // The 33 - 128 row kernel's 64-k groups of a block and K slices of a product,
-// by its M, N and K alone (they show in the bits; tile sizes do not): one slice
-// for wide products (gate/up) and for short K; otherwise slices for about 128
-// blocks of 64 rows of B, twice that for K >= 8192 (four times above 64 rows),
-// each of 1024 k or more. Two groups above 64 rows, where four leave room for
-// two stages only, and for wide products, whose tiles are 128 wide; else four
-// (at 64 rows o 11.8 against 12.3 us, down 20.4 against 21.4, q/k/v 13.7 against
-// 14.6).
+// by its M, N and K alone (they show in the bits; tile sizes do not). Times in us.
+//   Groups: four up to 64 rows; two for wide products (gate/up), whose tiles are
+//   128 wide, for the longest K, and above 64 rows, where four leave room for two
+//   stages only - but four for short K, on small tiles (K and N of 2048 at 128
+//   rows 5.8, with two 8.9).
+//   Slices: one for wide products and short K, whose reduction costs more than it
+//   gains; else for about 128 blocks of 64 rows of B, at K >= 8192 twice (above 64
+//   rows four times) that. N = 2048 up to K = 4096 two only: three such products
+//   fill the GPU with them (at 33 rows 13.8, with four each 16.5). K of 16384 and
+//   more by 8192 rows of B and more three or four (28672 x 8192 at 64 rows 52.9,
+//   with two on narrower tiles 62). Narrow products (k/v) would leave most of the
+//   GPU idle: slices of 1024 k (above 64 rows and below N = 1024 of 512) up to
+//   about one small tile for each CU (N = 512, K = 4096 at 96 rows 6.8, with four
+//   8.6).
 constexpr int kRingWideN = 10240;
+constexpr int kRingNarrowN = 1024;
 
 void ring_slices(int M, int N, int K, int& wk, int& S, int& cps) {
-    const int tiles = (N + 63) / 64;
-    const bool wide = N >= kRingWideN;
-    wk = M > 64 || wide ? 2 : 4;
+    const int tiles = (N + 63) / 64, rows = (M + 31) / 32;
+    const bool wide = N >= kRingWideN, narrow = N <= kRingNarrowN, shallow = K <= 2048;
+    const bool longest = K >= 16384 && N >= 8192;
+    wk = wide || (M > 64 ? !(shallow && K >= 512 && N <= 4096) : longest) ? 2 : 4;
     const int nk = (K + 64 * wk - 1) / (64 * wk);
-    const int target = K >= 8192 ? (M > 64 ? 512 : 256) : 128;
-    S = wide || K <= 2048 ? 1 : max(1, min(min(target / tiles, K / 1024), 8));
+    if (wide || shallow) S = 1;
+    else if (longest && M <= 64) S = K > 16384 ? 4 : 3;
+    else if (K >= 8192) S = min((M > 64 ? 512 : 256) / tiles, 8);
+    else if (!narrow) S = min(128 / tiles, M > 64 ? K / 1024 : K > 4096 || N > 2048 || N <= 1792 ? 4 : 2);
+    else S = min(min(8, 256 / (rows * (M > 64 ? tiles : (N + 31) / 32))), K / (M > 64 && N < kRingNarrowN ? 512 : 1024));
+    S = max(S, 1);
     cps = (nk + S - 1) / S;
     S = (nk + cps - 1) / cps;
 }
 
-template <int BM, int BN, int WK, int NST>
+template <int BM, int BN, int WK, int NST, bool SERIAL = false>
 int launch_ring(int count, void* const* c, const uint16_t* a, const void* const* b, const void* const* scales,
                 const int* n, int M, int K, SharedPlan& pl, float* scratch, size_t scratch_bytes, const ResEpi* ep,
                 const SwigluArgs* sw) {
@@ -2716,13 +2776,15 @@ int launch_ring(int count, void* const* c, const uint16_t* a, const void* const*
     const dim3 block(WN * WK * kWave);
     const int TT = (M + BM - 1) / BM;
     const auto blocks_of = [&](long long units) { return TT > 1 ? (units + 7) / 8 * 8 * TT : units; };
-    if (sw && pl.S[0] == 1) {
-        const int tiles = (n[0] + BN / 2 - 1) / (BN / 2);
-        gemm_i8w_ring_swiglu_kernel<BM, BN, WN, WK, NST>
-            <<<dim3(static_cast<unsigned>(blocks_of(tiles))), block, 0, stream()>>>(*sw, a, M, n[0], K, tiles,
-                                                                                    pl.cps[0], TT);
-        NG_CHECK_LAUNCH("ng_gemm_int8_silu_mul");
-        return 0;
+    if constexpr (!SERIAL) {
+        if (sw && pl.S[0] == 1) {
+            const int tiles = (n[0] + BN / 2 - 1) / (BN / 2);
+            gemm_i8w_ring_swiglu_kernel<BM, BN, WN, WK, NST>
+                <<<dim3(static_cast<unsigned>(blocks_of(tiles))), block, 0, stream()>>>(*sw, a, M, n[0], K, tiles,
+                                                                                        pl.cps[0], TT);
+            NG_CHECK_LAUNCH("ng_gemm_int8_silu_mul");
+            return 0;
+        }
     }
     for (int i = 0; i < count; ++i) {
         pl.tm[i] = TT;
@@ -2732,54 +2794,82 @@ int launch_ring(int count, void* const* c, const uint16_t* a, const void* const*
     const TileEpi te{ep && pl.S[0] == 1 ? ep->out : nullptr, ep && pl.S[0] == 1 ? ep->res : nullptr};
     return run_shared_split(count, c, b, scales, n, M, K, pl,
                             [&](const SharedSet& set, const SplitSet& sp, unsigned blocks, hipStream_t st) {
-                                if (count == 1)
-                                    gemm_i8w_ring_kernel<BM, BN, WN, WK, NST><<<dim3(blocks), block, 0, st>>>(
-                                        set.c[0], a, set.b[0], set.scale[0], sp.part[0], M, set.n[0], K, sp.S[0],
-                                        sp.tiles[0], sp.cps[0], TT, te);
-                                else
-                                    gemm_i8w_ring_shared_kernel<BM, BN, WN, WK, NST>
-                                        <<<dim3(blocks), block, 0, st>>>(set, sp, a, M, K);
+                                if constexpr (!SERIAL) {
+                                    if (count == 1) {
+                                        gemm_i8w_ring_kernel<BM, BN, WN, WK, NST><<<dim3(blocks), block, 0, st>>>(
+                                            set.c[0], a, set.b[0], set.scale[0], sp.part[0], M, set.n[0], K, sp.S[0],
+                                            sp.tiles[0], sp.cps[0], TT, te);
+                                        return;
+                                    }
+                                }
+                                gemm_i8w_ring_shared_kernel<BM, BN, WN, WK, NST, SERIAL>
+                                    <<<dim3(blocks), block, 0, st>>>(set, sp, a, M, K);
                             },
                             sw, scratch, scratch_bytes, ep);
 }
 
 // Products that share A at 33 to 128 rows and take the same groups; other
-// arguments as gemm_tiles. Tile by the number of blocks: wide enough to share A
-// where there are enough of them for the CUs, narrow where not (one product of
-// 4096 rows of B at 64 rows: 11.8 us on tiles of 32, 12.8 on 64; gate alone 19.3
-// on 64, 24.1 on 128), and rows of A cut into tiles of 64 or 32 where even
-// those leave the GPU idle. Several products on a stream under capture whose
-// buffer holds the partial sums of each but not of all of them: one launch each
-// (with sw 1 is returned before launching anything), as separate calls.
+// arguments as gemm_tiles. Tile by the number of blocks: the widest that still
+// gives every CU one, and rows of A cut into tiles of 32 too where that takes
+// fewer rounds of blocks. Measured in us, four groups: K = 4096 at 64 rows, N =
+// 1024 6.8 on 32 x 32 and 8.3 on 64 x 32, N = 4096 11.4 on 32 x 64 and 13.1 on 64 x
+// 64; slices of 1024 k or less pay too little for that (N = 8192, K = 1024 at 33
+// rows 5.6 on 64 x 32, 6.1 on 32 x 64). Two groups up to 64 rows: 64 x 64, six
+// stages deep or, two blocks per CU, three (N = 11008, K = 4096: 17.4 and 18.3 at 33
+// rows, 19.9 and 19.6 at 64), up to a block for each CU or where nearly two fit it
+// (N = 32000, K = 4096 at 33 rows 33.3, on 64 x 128 36.0), 64 x 128 between and for
+// SwiGLU. Above 64 rows 32 x 64 in one round, or in two of short slices (N = 1024,
+// K = 4096 at 96 rows 7.9, on eight stages of it 8.3), then wider.
+// A set whose sliced products take more than one round has both slices of a tile
+// in one block (SERIAL: three products of 4096 rows of B, K = 4096, at 33, 48 and 64
+// rows 18, 19 and 21; with a block per slice 24, 24 and 26). Several products on a
+// stream under capture whose buffer holds the partial sums of each but not of all
+// of them: one launch each (with sw 1 is returned before launching anything), as
+// separate calls.
 int gemm_ring(int count, void* const* c, const void* a, const void* const* b, const void* const* scales, const int* n,
               int M, int K, float* scratch, size_t scratch_bytes, const ResEpi* ep, const SwigluArgs* sw) {
     const auto* ap = static_cast<const uint16_t*>(a);
     SharedPlan pl{};
     int wk = 0;
-    long long b64 = 0, b128 = 0;
+    const int rows32 = (M + 31) / 32;
+    long long b32 = 0, b64 = 0, b128 = 0;
+    int most = 1, longest = 0;  // slices of a product, steps of a slice
     for (int i = 0; i < count; ++i) {
         ring_slices(M, n[i], K, wk, pl.S[i], pl.cps[i]);
+        most = max(most, pl.S[i]);
+        longest = max(longest, pl.cps[i]);
+        b32 += (static_cast<long long>(n[i]) + 31) / 32 * pl.S[i];
         b64 += (static_cast<long long>(n[i]) + 63) / 64 * pl.S[i];
         b128 += (static_cast<long long>(n[i]) + 127) / 128 * pl.S[i];
     }
-    const size_t floats = partial_floats(count, n, M, pl.S);
+    const bool serial = count > 1 && !sw && M <= 64 && wk == 4 && most == 2 && b64 > 256;
+    const size_t floats = serial ? 0 : partial_floats(count, n, M, pl.S);
     if (count > 1 && floats > 0 && !partial_room(stream(), floats * sizeof(float))) {
         if (sw) return 1;
         for (int i = 0; i < count; ++i)
             if (gemm_ring(1, c + i, a, b + i, scales + i, n + i, M, K) != 0) return -1;
         return 0;
     }
+    const auto rounds = [](long long blocks) { return (blocks + 255) / 256; };  // at a block per CU
 #define NG_RING(BM, BN, WK, NST) \
     return launch_ring<BM, BN, WK, NST>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw)
     if (wk == 4) {
-        if (b64 > 128) NG_RING(64, 64, 4, 3);
-        NG_RING(64, 32, 4, 4);
+        if (b32 * rows32 <= 256) NG_RING(32, 32, 4, 3);
+        if (longest <= 4 && b32 <= 256 && M <= 64) NG_RING(64, 32, 4, 4);
+        if (count > 1 && most >= 4 && b32 * rows32 <= 512) NG_RING(32, 32, 4, 3);
+        if (7 * rounds(b64 * rows32) < 10 * rounds(b64 * ((M + 63) / 64))) NG_RING(32, 64, 4, 4);
+        if (serial) {
+            for (int i = 0; i < count; ++i) pl.S[i] = 1;
+            return launch_ring<64, 64, 4, 3, true>(count, c, ap, b, scales, n, M, K, pl, scratch, scratch_bytes, ep, sw);
+        }
+        NG_RING(64, 64, 4, 3);
     }
     if (M <= 64) {
-        if (b128 >= 128) NG_RING(64, 128, 2, 4);
-        NG_RING(64, 64, 2, 6);
+        if (!sw && b64 <= 256 && M <= 48 && K > 2048) NG_RING(64, 64, 2, 6);
+        if (!sw && (b64 <= 256 || (b64 <= 512 && (b64 > 448 ? K <= 4096 : count == 1 && K <= 1024)))) NG_RING(64, 64, 2, 3);
+        NG_RING(64, 128, 2, 4);
     }
-    if (b64 <= 64) NG_RING(32, 64, 2, 8);
+    if (b64 * rows32 <= (most >= 4 ? 512 : 256)) NG_RING(32, 64, 2, 4);
     if (b64 <= 128) NG_RING(64, 64, 2, 6);
     if (b128 >= 160) {
         if (M <= 96) NG_RING(96, 128, 2, 3);

@@ -451,9 +451,12 @@ def test_capture_of_a_set_after_a_call(lib, cold_stream, M, K, ns):
 
 # A set at 33 - 128 rows whose products were called one by one before: the
 # buffer holds the partial sums of the largest, not of all, and the set is
-# captured as the separate launches.
-@pytest.mark.parametrize("M,K,ns,kernels", [(64, 4096, [4096, 1024, 1024], 6), (128, 4096, [2048, 1024], 4)])
-def test_capture_of_a_set_after_its_products(lib, cold_stream, M, K, ns, kernels):
+# captured as the separate launches; a set whose blocks take both K slices of
+# their tile needs no buffer at all.
+@pytest.mark.parametrize("M,K,ns,warm,kernels", [(64, 4096, [4096, 1024, 1024], True, 6),
+                                                 (128, 4096, [2048, 1024], True, 4),
+                                                 (40, 4096, [4096, 4096, 4096], False, 1)])
+def test_capture_of_a_set_after_its_products(lib, cold_stream, M, K, ns, warm, kernels):
     hip, stream = cold_stream
     banner(f"graph capture of a set after its products M={M} K={K} n={ns}")
     rng = np.random.Generator(np.random.PCG64(8))
@@ -477,7 +480,8 @@ def test_capture_of_a_set_after_its_products(lib, cold_stream, M, K, ns, kernels
         return [get(c, np.uint16, (M, n)) for c, n in zip(outs, ns)]
 
     try:
-        separate()
+        if warm:
+            separate()
         graph, ex = hip.capture(stream, lambda: ok(shared(), "set under capture"))
         try:
             assert hip.kernel_nodes(graph) == kernels

@@ -486,6 +486,8 @@ TILE_EDGES = [(33, 64, 1), (33, 128, 127), (64, 192, 129), (65, 320, 130), (96, 
               (128, 4160, 1000), (127, 64, 10240), (64, 8256, 257), (100, 11008, 132), (128, 14336, 4099),
               (64, 4160, 9000), (50, 2112, 10300), (34, 192, 20500), (70, 4160, 5000), (66, 4288, 9000),
               (90, 192, 20500), (128, 192, 20500), (110, 4160, 9000),
+              (50, 4160, 4999), (40, 2112, 10300), (100, 4160, 6001), (64, 2112, 16400), (97, 192, 1000),
+              (33, 16448, 8200), (66, 4160, 500), (40, 4160, 1000), (64, 960, 5000), (90, 1088, 3000),
               (129, 16, 1), (129, 64, 127), (191, 80, 129), (192, 128, 128), (193, 192, 255), (255, 208, 257),
               (257, 256, 300), (384, 320, 4097), (385, 336, 4100), (511, 1024, 14344), (1025, 2048, 8200),
               (130, 14336, 512), (333, 11008, 1000), (200, 8208, 66), (255, 528, 8200), (257, 528, 14340),
@@ -507,7 +509,9 @@ def test_int8_prefill_tile_edges(lib, M, K, N):
 
 @pytest.mark.parametrize("M,K,N,off", [(333, 1024, 4096, 0), (1000, 4096, 14336, 0), (200, 1040, 1002, 0),
                                        (257, 128, 257, 2), (40, 4096, 14336, 0), (100, 192, 10250, 0),
-                                       (128, 4096, 1000, 0), (64, 1024, 10241, 2)])
+                                       (128, 4096, 1000, 0), (64, 1024, 10241, 2),
+                                       (127, 1088, 500, 0), (50, 1088, 2808, 0), (127, 1088, 4000, 0),
+                                       (65, 320, 2100, 0)])
 def test_int8_prefill_epilogues(lib, M, K, N, off):
     """SwiGLU and the residual add in the epilogue (one K slice) or the reduction
     of the kernels above 32 rows give the bits of the calls they replace, also with

@@ -148,6 +148,26 @@ def test_shared_a_prefill_slices_bit_for_bit(lib, M, K, ns):
         assert_bits_equal(g, w)
 
 
+# The kernel of 33 to 128 rows: sets whose blocks take both K slices of their
+# tile (with products of one slice between, with N and K off the tiles), and
+# short products on each small tile; alone each product has tiles and slices of
+# its own.
+@pytest.mark.parametrize("M,K,ns", [(40, 4096, [4096, 4096, 4096]), (64, 4160, [4096, 4100, 4090]),
+                                    (33, 4160, [4096, 4099, 9000]), (48, 8256, [8192, 8190]),
+                                    (128, 1088, [2048, 2048, 2048]), (100, 2048, [2048, 256, 250]),
+                                    (66, 1088, [1000, 77, 130]), (64, 4096, [2048, 512, 500]),
+                                    (64, 4096, [1024, 1000])])
+def test_shared_a_33_to_128_rows_bit_for_bit(lib, M, K, ns):
+    banner(f"gemm_int8_shared_a 33 - 128 rows M={M} K={K} n={ns}")
+    a, qs, scales = problem(M, K, ns, exact=False)
+    for g, w in zip(shared(lib, a, qs, scales, M, K), separate(lib, a, qs, scales, M, K)):
+        assert_bits_equal(g, w)
+    a, qs, scales = problem(M, K, ns, exact=True)
+    for g, q, s in zip(shared(lib, a, qs, scales, M, K), qs, scales):
+        want = ((f16val(a) @ q.astype(np.float64).T).astype(np.float32) * s[None, :]).astype(np.float16)
+        assert_bits_equal(g, want.view(np.uint16))
+
+
 @pytest.mark.parametrize("M,K,ns", SETS)
 def test_shared_a_is_cuda_gemm_int8_bit_for_bit(lib, M, K, ns):
     banner(f"gemm_int8_shared_a random M={M} K={K} n={ns}")
