@@ -146,11 +146,14 @@ extern "C" int cuda_softmax(void* output, const void* input, int num_rows, int r
     const auto* x = static_cast<const uint16_t*>(input);
     const dim3 grid(num_rows);
     if (row_size % 8 == 0 && aligned16(output) && aligned16(input)) {
-        // One wave for rows of up to 512 elements, four up to 2048, sixteen
-        // above: few long rows need every wave a block can have.
+        // One wave for rows of up to 512 elements, four up to 8192, sixteen
+        // above: a block of 16 waves pays for its barriers and for threads with
+        // no vector (4096 rows of 2056: 11.2 us with 4 waves, 29.2 with 16; of
+        // 8192: 22.3 and 36.4; 64 rows of 4096: 3.5 and 4.1).
         if (row_size <= 512) softmax_vec_kernel<1, 64><<<grid, dim3(64), 0, stream()>>>(y, x, row_size);
         else if (row_size <= 2048) softmax_vec_kernel<1, 256><<<grid, dim3(256), 0, stream()>>>(y, x, row_size);
-        else if (row_size <= 8192) softmax_vec_kernel<1, 1024><<<grid, dim3(1024), 0, stream()>>>(y, x, row_size);
+        else if (row_size <= 4096) softmax_vec_kernel<2, 256><<<grid, dim3(256), 0, stream()>>>(y, x, row_size);
+        else if (row_size <= 8192) softmax_vec_kernel<4, 256><<<grid, dim3(256), 0, stream()>>>(y, x, row_size);
         else if (row_size <= 16384) softmax_vec_kernel<2, 1024><<<grid, dim3(1024), 0, stream()>>>(y, x, row_size);
         else if (row_size <= 32768) softmax_vec_kernel<4, 1024><<<grid, dim3(1024), 0, stream()>>>(y, x, row_size);
         else if (row_size <= 65536) softmax_vec_kernel<8, 1024><<<grid, dim3(1024), 0, stream()>>>(y, x, row_size);

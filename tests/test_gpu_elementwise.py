@@ -150,7 +150,7 @@ def test_softmax_close(lib, ora):
 # rounding to fp16 (half an ulp, 2^-25 below 2^-14) and 2^-16 of the value: the
 # exponential's and the quotient's last bits and a sum of at most cols / 1024 + 20
 # rounded additions a thread (2^-24 each).
-@pytest.mark.parametrize("rows,cols,off", [(3, 8, 0), (2, 512, 0), (2, 520, 0), (5, 2048, 0), (3, 2056, 0), (2, 8192, 0),
+@pytest.mark.parametrize("rows,cols,off", [(3, 8, 0), (2, 512, 0), (2, 520, 0), (5, 2048, 0), (3, 2056, 0), (2, 4096, 0), (2, 4104, 0), (2, 8192, 0),
                                            (2, 8200, 0), (2, 16392, 0), (64, 32000, 0), (2, 65536, 0), (2, 65544, 0),
                                            (1, 131080, 0), (2, 1001, 0), (3, 4096, 1)])
 def test_softmax_rows(lib, rows, cols, off):
