@@ -145,7 +145,9 @@ extern "C" int cuda_softmax(void* output, const void* input, int num_rows, int r
     auto* y = static_cast<uint16_t*>(output);
     const auto* x = static_cast<const uint16_t*>(input);
     const dim3 grid(num_rows);
-    if (row_size % 8 == 0 && aligned16(output) && aligned16(input)) {
+    // A launch takes fewer than 2^32 threads: from 2^22 rows on no 1024 to a row.
+    const bool wide = num_rows < (1 << 22);
+    if (row_size % 8 == 0 && aligned16(output) && aligned16(input) && (row_size <= 8192 || wide)) {
         // One wave for rows of up to 512 elements, four up to 8192, sixteen
         // above: a block of 16 waves pays for its barriers and for threads with
         // no vector (4096 rows of 2056: 11.2 us with 4 waves, 29.2 with 16; of

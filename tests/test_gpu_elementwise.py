@@ -178,3 +178,28 @@ def test_softmax_nonfinite_rows(lib, cols):
     ok(lib.cuda_softmax(ob.vp, xb.vp, 4, cols))
     got = get(ob, np.uint16, x.shape).view(np.float16)
     assert np.isnan(got[:3]).all() and np.isfinite(got[3]).all()
+
+
+# As many rows as a launch of 256 threads a row takes but one of 1024 does not,
+# at a row size of each: accepted, first and last row right (in place).
+@pytest.mark.parametrize("cols", [2056, 8200])
+def test_softmax_many_rows(lib, cols):
+    rows = 1 << 22
+    banner(f"softmax {rows}x{cols}")
+    x = bits(RNG.standard_normal((2, cols)) * 4, "f16")
+    buf = empty(2 * rows * cols)
+    try:
+        ends = (buf.ptr, buf.ptr + 2 * (rows - 1) * cols)
+        for p, row in zip(ends, x):
+            ok(lib.cuda_copy_int8_to_device(C.c_void_p(p), row.ctypes.data_as(C.c_void_p), 2 * cols), "upload")
+        ok(lib.cuda_softmax(buf.vp, buf.vp, rows, cols), "softmax")
+        got = np.empty_like(x)
+        for p, row in zip(ends, got):
+            ok(lib.cuda_copy_int8_to_host(row.ctypes.data_as(C.c_void_p), C.c_void_p(p), 2 * cols), "download")
+    finally:
+        buf.free()
+    v = x.view(np.float16).astype(np.float64)
+    e = np.exp(v - v.max(1, keepdims=True))
+    want = e / e.sum(1, keepdims=True)
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(want, 2.0 ** -14))) - 10)
+    assert (np.abs(got.view(np.float16).astype(np.float64) - want) <= 0.5 * ulp + want * 2.0 ** -16).all()
