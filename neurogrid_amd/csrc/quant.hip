@@ -115,14 +115,15 @@ __global__ void tensor_scale_finalize_kernel(float* scale) {
 }
 
 // ---- per column of [K, N] ------------------------------------------------------
-// Vector form (N % 8 == 0, aligned pointers, K >= kColMinRows): three launches.
+// Vector form (N % 8 == 0, aligned pointers, K >= 2): three launches.
 //   1. The matrix is cut into chunks of `rows` rows x 512 columns, a block each:
 //      lane l of a wave owns 8 neighbouring columns (16-byte loads, 1 KiB per
 //      instruction), the 4 waves take every fourth row, kColLoads rows requested
 //      before any is folded. The maxima are taken on packed magnitude patterns
 //      and stored, 16 bits per column and chunk, in the output buffer: chunks N
-//      2 <= K N bytes, as a chunk holds 16 rows or more. No atomics and nothing
-//      to clear first.
+//      2 <= K N bytes, as a chunk holds 16 rows or more or, where K has fewer, is
+//      the only one (15 x 2^22 then takes 80 us, 210 element by element). No
+//      atomics and nothing to clear first.
 //   2. One thread group per 8 columns folds the chunks and writes the scales.
 //   3. The same chunks are quantised (the codes overwrite the partial maxima),
 //      the 8 scales and reciprocals of a thread computed once per chunk.
@@ -135,7 +136,7 @@ __global__ void tensor_scale_finalize_kernel(float* scale) {
 // dequantisation that follows 38.6 instead of 25.3.
 constexpr int kColCols = 8 * kWave;   // columns of a chunk
 constexpr int kColLoads = 4;          // rows in flight per wave
-constexpr int kColMinRows = 16;       // rows of a chunk, at least
+constexpr int kColMinRows = 16;       // rows of a chunk, at least (all K of them if fewer)
 
 // Largest magnitude pattern per half; patterns above inf's are NaNs.
 __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
@@ -470,7 +471,7 @@ extern "C" int cuda_quantize_weights(void* output, void* scales, const void* inp
     NG_REQUIRE(K > 0 && N > 0, "cuda_quantize_weights: K=%d N=%d must be > 0", K, N);
     const uint16_t* x = static_cast<const uint16_t*>(input);
     int8_t* q = static_cast<int8_t*>(output);
-    if (N % 8 == 0 && K >= kColMinRows && aligned16(input) && aligned8(output)) {
+    if (N % 8 == 0 && K >= 2 && aligned16(input) && aligned8(output)) {
         // Rows per chunk: 64, or fewer down to 16 while that leaves under
         // 1024 chunks (four blocks per CU).
         const unsigned gx = static_cast<unsigned>((N + kColCols - 1) / kColCols);

@@ -209,9 +209,10 @@ def test_per_tensor_quant_with_nan_and_inf(lib, ora, n):
 
 
 # The vector form: fewest rows, chunks and columns of a chunk that end early,
-# more chunks than threads that fold them, and back to the element-wise form.
+# more chunks than threads that fold them, and back to the element-wise form
+# (a single row, N % 8 != 0).
 @pytest.mark.parametrize("K,N", [(16, 8), (17, 520), (63, 512), (65, 1032), (129, 4104), (4099, 1016), (15, 64),
-                                 (200, 36)])
+                                 (2, 8), (3, 1032), (15, 4104), (1, 520), (200, 36)])
 def test_per_column_quant_chunks(lib, ora, K, N):
     banner(f"per-column quant chunks {K}x{N}")
     x = f16(RNG.standard_normal((K, N)) * RNG.uniform(0.01, 10, (1, N)))
