@@ -1350,14 +1350,25 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // 16 bytes per lane from (voff + soff) of a buffer to LDS at lds + 16 lane.
 // Written out because the compiler waits for all outstanding loads (vmcnt(0))
 // before any LDS read that follows its builtin; the kernel waits by count. The
-// load has no register result. m0 is no allocatable register: the compiler sets
-// it before each use of its own and keeps nothing in it. s_nop: the wait state
-// between a write of m0 and a load that reads it.
+// load has no register result. s_nop: the wait state between a write of m0 and a
+// load that reads it. m0 is declared as written, so that the compiler sets it
+// again for uses of its own; it warns that it keeps nothing in a reserved register
+// across the statement, which is what is meant.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
                  "s"(r), "s"(soff)
-                 : "memory");
+                 : "memory", "m0");
 }
+
+// Likewise, non-temporal.
+__device__ __forceinline__ void load_lds16_nt(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff),
+                 "s"(r), "s"(soff)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
 
 // At most N of this wave's vector memory operations still outstanding.
 template <int N>
@@ -1789,12 +1800,6 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_swiglu_kerne
 // Bound at 64 rows: gate/up move 117 MB of weights in 32 us (3.7 TB/s) and A 224
 // times from L2 (as much again); 8 or 16 us calls are launch, first loads and the
 // reduction.
-__device__ __forceinline__ void load_lds16_nt(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff),
-                 "s"(r), "s"(soff)
-                 : "memory");
-}
-
 // SERIAL: a block takes both K slices of its tile (S = 1; cps: the first one's
 // steps), one after the other, and adds the second sum to the first as the
 // reduction does: the bits of a launch with a block per slice, without its partial sums.
