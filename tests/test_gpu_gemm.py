@@ -507,11 +507,18 @@ def test_int8_prefill_tile_edges(lib, M, K, N):
     assert_bits_equal(get(cb, np.uint16, (M * N + 1,))[1:].reshape(M, N), want.view(np.uint16), "C off 16 bytes")
 
 
+# SwiGLU with one K slice on every tile shape of both kernels, M and N off the
+# tiles: 64, 128, 192 and 256 x 128, 128, 192 and 256 x 256 of the prefill kernel;
+# 32 x 32, 64 x 32, 32 x 64 and 64 x 64 with four groups, 32 x 64, 64 x 64, 64, 96 and
+# 128 x 128 and 96 and 128 x 64 with two.
 @pytest.mark.parametrize("M,K,N,off", [(333, 1024, 4096, 0), (1000, 4096, 14336, 0), (200, 1040, 1002, 0),
                                        (257, 128, 257, 2), (40, 4096, 14336, 0), (100, 192, 10250, 0),
                                        (128, 4096, 1000, 0), (64, 1024, 10241, 2),
-                                       (127, 1088, 500, 0), (50, 1088, 2808, 0), (127, 1088, 4000, 0),
-                                       (65, 320, 2100, 0)])
+                                       (129, 1040, 14340, 0), (255, 1040, 10248, 0), (900, 1040, 4098, 0),
+                                       (899, 1040, 4104, 0), (1025, 1040, 3004, 0),
+                                       (127, 1088, 500, 0), (64, 960, 2500, 2), (50, 1088, 2808, 0), (63, 320, 5630, 0),
+                                       (127, 1088, 4000, 0), (65, 320, 2100, 0), (127, 320, 4000, 2),
+                                       (95, 192, 10250, 0), (95, 320, 5632, 0), (127, 320, 5630, 0)])
 def test_int8_prefill_epilogues(lib, M, K, N, off):
     """SwiGLU and the residual add in the epilogue (one K slice) or the reduction
     of the kernels above 32 rows give the bits of the calls they replace, also with
