@@ -2588,19 +2588,23 @@ constexpr TileShape kTileShapes[] = {
     {64, 128, 4.4, 0.324, 0.398, 0.58, 0.349}};
 constexpr int kTileShapeCount = 7, kTileSerialFirst = 2;
 
-// Time of a launch of `blocks` blocks whose steps add up to `steps`.
-double tile_time(const TileShape& ts, long long blocks, long long steps) {
-    const long long full = blocks / 256;
-    const double rest = static_cast<double>(blocks % 256) / 256.0;
+// CUs of the device that the times were fitted on. Not the present device's: slices,
+// and with them the bits, would then depend on how it is partitioned.
+constexpr int kTileCus = 256;
+
+// Time of a launch of `blocks` blocks of `steps` steps each on average.
+double tile_time(const TileShape& ts, long long blocks, double steps) {
+    const long long full = blocks / kTileCus;
+    const double rest = static_cast<double>(blocks % kTileCus) / kTileCus;
     double step;
     if (full == 0) step = ts.lo + (rest > ts.knee ? (ts.hi - ts.lo) * (rest - ts.knee) / (1.0 - ts.knee) : 0.0);
     else if (rest == 0.0) step = full == 1 ? ts.hi : ts.more * full;
     else step = ts.more * full + ts.lo + (ts.more - ts.lo) * rest;
-    return ts.fixed + step * (static_cast<double>(steps) / blocks);
+    return ts.fixed + step * steps;
 }
 
-long long tile_blocks(const TileShape& ts, int M, int N, int S) {
-    return ((static_cast<long long>(M) + ts.BM - 1) / ts.BM) * ((static_cast<long long>(N) + ts.BN - 1) / ts.BN) * S;
+long long tile_blocks(const TileShape& ts, int M, int N) {
+    return ((static_cast<long long>(M) + ts.BM - 1) / ts.BM) * ((static_cast<long long>(N) + ts.BN - 1) / ts.BN);
 }
 
 // K slices of a product on the prefill kernel: a function of M, N and K alone,
@@ -2615,14 +2619,16 @@ void prefill_slices(int M, int N, int K, int& S, int& cps) {
     double one = 0.0, best = 0.0;
     S = 1;
     cps = nk;
+    long long tiles[kTileShapeCount];
+    for (int k = 0; k < kTileShapeCount; ++k) tiles[k] = tile_blocks(kTileShapes[k], M, N);
     for (int s = 1; s <= 8; ++s) {
         const int per = (nk + s - 1) / s, ss = (nk + per - 1) / per;
         const double bytes = static_cast<double>(ss) * M * N * sizeof(float);
         if (s > 1 && (per < 8 || ss < s || bytes > static_cast<double>(kNoAllocScratchBytes))) continue;
+        const double steps = static_cast<double>(nk) / ss;
         double t = 0.0;
-        for (const TileShape& ts : kTileShapes) {
-            const long long blocks = tile_blocks(ts, M, N, ss);
-            const double v = tile_time(ts, blocks, blocks / ss * nk);
+        for (int k = 0; k < kTileShapeCount; ++k) {
+            const double v = tile_time(kTileShapes[k], tiles[k] * ss, steps);
             if (t == 0.0 || v < t) t = v;
         }
         if (ss > 1) t += 3.0 + 0.3e-6 * bytes;
@@ -2694,11 +2700,11 @@ int gemm_tiles(int count, void* const* c, const void* a, const void* const* b, c
         for (int k = first; k < kTileShapeCount; ++k) {
             long long blocks = 0, steps = 0;
             for (int i = 0; i < count; ++i) {
-                const long long bl = tile_blocks(kTileShapes[k], M, n[i], serial ? 1 : pl.S[i]);
-                blocks += bl;
-                steps += serial ? bl * nk : bl / pl.S[i] * nk;
+                const long long tiles = tile_blocks(kTileShapes[k], M, n[i]);
+                blocks += serial ? tiles : tiles * pl.S[i];
+                steps += tiles * nk;
             }
-            double t = tile_time(kTileShapes[k], blocks, steps);
+            double t = tile_time(kTileShapes[k], blocks, static_cast<double>(steps) / blocks);
             if (!serial) t = reduce + std::max(t, kTileShapes[k].fixed + kTileShapes[k].lo * longest);
             if (k == first || t < least) {
                 least = t;
