@@ -23,12 +23,14 @@ into a HIP graph and replayed: the GPU then never waits for the host.
 
 Printed JSON line: value = layer algorithmic bytes / step time (GB/s);
 us_per_layer = sum of the six kernels' average durations; per-kernel GB/s
-and fraction of 8 TB/s; extra layer configurations (decode T=64, Llama-2-13B,
-Mistral-Nemo bf16) and kernels (gather per forward, fused RMSNorm+int8, int8
-dequant, QK LayerNorm + RoPE, cuda_gemm_int8 at Mistral-7B's INT8 projections);
-the layer with this library's fused entry points; the roofline of the dominant
-kernel (SwiGLU); and the CPU oracle timed on the host cores on a bounded token
-sample of the same layer.
+and fraction of 8 TB/s; the layer with this library's fused entry points; the
+roofline of the dominant kernel (SwiGLU); and the CPU oracle timed on the host
+cores on a bounded token sample of the same layer. The line is kept short (5
+digits a number, under 8 KB): some readers of a program's output take no longer
+ones. A line "[bench-extra] {...}" on stderr holds the further measurements:
+extra layer configurations (decode T=64, Llama-2-13B, Mistral-Nemo bf16) and
+kernels (gather per forward, fused RMSNorm+int8, int8 dequant, QK LayerNorm +
+RoPE, cuda_gemm_int8 at Mistral-7B's INT8 projections).
 
 Usage: python bench.py [--gpus 1] [--steps 50] [--warmup 5] [--no-cpu] [--no-extra]
        python bench.py --profile-pass  (eager launches of every kernel for rocprofv3: the kernel trace and
@@ -148,6 +150,17 @@ class Graph:
 
 def log(msg):
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+def rounded(v):
+    """v with every float in it to 5 significant digits."""
+    if isinstance(v, float):
+        return float(f"{v:.5g}")
+    if isinstance(v, dict):
+        return {k: rounded(x) for k, x in v.items()}
+    if isinstance(v, (list, tuple)):
+        return [rounded(x) for x in v]
+    return v
 
 
 # ----------------------------------------------------------------------------- layer kernel set
@@ -1938,11 +1951,12 @@ def main():
         "per_kernel": kernels,
         "copy_note": "copy_us: a plain device-to-device hipMemcpyAsync moving the kernel's algorithmic bytes "
                      "(half read, half written), timed the same way; vs_copy = copy_us / us",
-        "extra": extra,
         "roofline": roof,
         "cpu_baseline": cpu,
     }
-    print(json.dumps(line), flush=True)
+    if extra:
+        print(f"[bench-extra] {json.dumps(rounded(extra))}", file=sys.stderr, flush=True)
+    print(json.dumps(rounded(line)), flush=True)
 
 
 if __name__ == "__main__":

@@ -90,3 +90,13 @@ def test_floor_kernels_compile_for_gfx950():
     rtc.hiprtcGetCodeSize(prog, C.byref(n))
     rtc.hiprtcDestroyProgram(C.byref(prog))
     assert rc == 0 and n.value > 0
+
+
+def test_bench_rounds_its_numbers():
+    """Five significant digits of every float, counts and texts as they are."""
+    sys.path.insert(0, str(ROOT))
+    import bench
+
+    v = {"us": 119.34567891, "bytes": 738197504, "list": [0.000123456789, 2], "note": "x", "none": None, "yes": True}
+    assert bench.rounded(v) == {"us": 119.35, "bytes": 738197504, "list": [0.00012346, 2], "note": "x", "none": None,
+                                "yes": True}
