@@ -318,17 +318,17 @@ def test_concurrent_calls(gpu):
 
 def test_concurrent_gemm_int8(gpu):
     """Several host threads call cuda_gemm_int8 on the one launch stream at
-    once, through the split-K path (M = 40, two kernels per call sharing the
-    stream's partial-sum buffer) and the library path (M = 200, the stream's
-    fp16 weight copy); every result is exact."""
+    once, through the kernels with K slices (24, 40 and 200 rows, two launches
+    per call that share the stream's partial-sum buffer) and the library path
+    (K = 520, the stream's fp16 weight copy); every result is exact."""
     banner("bindings concurrent GEMMINT8")
-    K, N = 512, 256
+    N = 256
     errors = []
 
     def worker(seed):
         try:
             rng = np.random.Generator(np.random.PCG64(100 + seed))
-            for M in (40, 200, 40, 200):
+            for M, K in ((40, 4096), (200, 520), (24, 512), (200, 4096), (40, 4096), (200, 520)):
                 data_a = (rng.integers(-64, 65, (M, K)) / 64.0).astype(np.float32)
                 codes = rng.integers(-128, 128, (N, K)).astype(np.int8)
                 scale = np.full(N, 2.0 ** -7, np.float32)

@@ -13,9 +13,11 @@ of this library, within the fp16 bar (|d| <= 1e-2 or 2 ulp) for the calls that
 go through hipBLASLt. Inputs are never written, so a replay recomputes the
 same values. No entry point may record a memset node (a kernel fills instead).
 
-A last test captures a split-K GEMM, then makes an eager call whose partial
-sums need a larger buffer, and replays the graph: the buffer the graph holds
-must still be valid.
+Where a case is there for its K slices, the launches of the graph are counted:
+the product's and its reduction's. One test captures a product with K slices,
+then makes eager calls whose partial sums need larger buffers, and replays the
+graph: the buffer the graph holds must still be valid. The last ones capture on
+streams for which the library holds no buffer, or one that is too small.
 """
 from __future__ import annotations
 
@@ -29,6 +31,7 @@ pytestmark = pytest.mark.gpu
 T, H, I, NQ, NKV, D, V = 24, 512, 1024, 4, 2, 128, 100
 GK, GN = 512, 256
 GNW = 12288  # wide N for the GEMM
+GKD = 4096  # deep K for the GEMM: K slices at 33 rows and more
 EPS, THETA = C.c_float(1e-5), C.c_float(1e6)
 
 
@@ -71,6 +74,9 @@ def inp():
     a["wsc"] = rng.uniform(1e-3, 1e-2, GN).astype(np.float32)
     a["wq_wide"] = rng.integers(-127, 128, (GNW, GK)).astype(np.int8)
     a["wsc_wide"] = rng.uniform(1e-3, 1e-2, GNW).astype(np.float32)
+    a["wq_deep"] = rng.integers(-127, 128, (GN, GKD)).astype(np.int8)
+    for m in (40, 100, 200):
+        a[f"d{m}"] = f16_bits(n(m, GKD))
     a["tsc"] = np.array([0.0125], np.float32)
     a["wh"] = f16_bits(n(GK, GN, s=0.05))
     for m in (1, 3, 16, 24, 40, 64, 100, 200, 4096):
@@ -159,29 +165,44 @@ def _ops():
         lambda L, i, o: L.cuda_dequantize_weights(o["y"].vp, i["wq"].vp, i["wsc"].vp, GN, GK, 1))
     add("cuda_dequantize_weights_col", {"y": (E2, (GK, GN))},
         lambda L, i, o: L.cuda_dequantize_weights(o["y"].vp, i["wq_kn"].vp, i["wsc"].vp, GK, GN, 0))
-    # GEMMs: GEMV (M <= 4), small-M MFMA, split-K at three tile heights, the
-    # prefill kernel with two K slices (M > 128), the library path
-    # (transpose_b false), and the fp16 GEMM.
+    # GEMMs: GEMV (M <= 4), small-M MFMA, the ring kernel (33 to 128 rows) and
+    # the tile kernel (M > 128) in one K slice each and, at K = 4096, with K
+    # slices and the reduction, the library path (transpose_b false), and the
+    # fp16 GEMM.
     for m in (1, 3, 16, 40, 64, 100):
         add(f"cuda_gemm_int8_M{m}", {"y": (E2, (m, GN))},
             lambda L, i, o, m=m: L.cuda_gemm_int8(o["y"].vp, i[f"a{m}"].vp, i["wq"].vp, i["wsc"].vp, m, GK, GN, True))
-    # N >= 12288: one slice of K, two wave groups per block
+    for m in (40, 100, 200):
+        add(f"cuda_gemm_int8_M{m}_sliced", {"y": (E2, (m, GN))},
+            lambda L, i, o, m=m: L.cuda_gemm_int8(o["y"].vp, i[f"d{m}"].vp, i["wq_deep"].vp, i["wsc"].vp, m, GKD, GN,
+                                                  True))
+    # N >= 12288: tiles of 64 rows
     add("cuda_gemm_int8_M40_wide", {"y": (E2, (40, GNW))},
         lambda L, i, o: L.cuda_gemm_int8(o["y"].vp, i["a40"].vp, i["wq_wide"].vp, i["wsc_wide"].vp, 40, GK, GNW, True))
     add("cuda_gemm_int8_M200_prefill", {"y": (E2, (200, GN))},
         lambda L, i, o: L.cuda_gemm_int8(o["y"].vp, i["a200"].vp, i["wq"].vp, i["wsc"].vp, 200, GK, GN, True))
-    # the allocation-free entry point: split-K weight streaming (M = 64: two
-    # slices of K) and the prefill kernel with K slices (M = 200), partial sums
-    # in the library's fixed device array
+    # the allocation-free entry point: the ring kernel (M = 64) and the tile
+    # kernel (M = 200) in one K slice, and with K slices, their partial sums in
+    # the library's fixed device array
     add("ng_gemm_int8_noalloc_M64", {"y": (E2, (64, GN))},
         lambda L, i, o: L.ng_gemm_int8_noalloc(o["y"].vp, i["a64"].vp, i["wq"].vp, i["wsc"].vp, 64, GK, GN, True))
     add("ng_gemm_int8_noalloc_M200_prefill", {"y": (E2, (200, GN))},
         lambda L, i, o: L.ng_gemm_int8_noalloc(o["y"].vp, i["a200"].vp, i["wq"].vp, i["wsc"].vp, 200, GK, GN, True))
-    # products that share A in one launch: the prefill kernel with two K slices (M = 200)
+    for m in (100, 200):
+        add(f"ng_gemm_int8_noalloc_M{m}_sliced", {"y": (E2, (m, GN))},
+            lambda L, i, o, m=m: L.ng_gemm_int8_noalloc(o["y"].vp, i[f"d{m}"].vp, i["wq_deep"].vp, i["wsc"].vp, m, GKD,
+                                                        GN, True))
+    # products that share A in one launch: the tile kernel in one K slice and
+    # with K slices and the shared reduction (M = 200)
     add("ng_gemm_int8_shared_a_M200_prefill", {"y": (E2, (200, GN)), "y2": (E2, (200, GN))},
         lambda L, i, o: L.ng_gemm_int8_shared_a(
             2, (C.c_void_p * 2)(o["y"].ptr, o["y2"].ptr), i["a200"].vp, (C.c_void_p * 2)(i["wq"].ptr, i["wq"].ptr),
             (C.c_void_p * 2)(i["wsc"].ptr, i["wsc"].ptr), (C.c_int * 2)(GN, GN), 200, GK))
+    add("ng_gemm_int8_shared_a_M200_sliced", {"y": (E2, (200, GN)), "y2": (E2, (200, GN))},
+        lambda L, i, o: L.ng_gemm_int8_shared_a(
+            2, (C.c_void_p * 2)(o["y"].ptr, o["y2"].ptr), i["d200"].vp,
+            (C.c_void_p * 2)(i["wq_deep"].ptr, i["wq_deep"].ptr), (C.c_void_p * 2)(i["wsc"].ptr, i["wsc"].ptr),
+            (C.c_int * 2)(GN, GN), 200, GKD))
     # the split kernel with two K slices and the shared reduction (M = 24)
     add("ng_gemm_int8_shared_a_M24_split", {"y": (E2, (24, GN)), "y2": (E2, (24, GN))},
         lambda L, i, o: L.ng_gemm_int8_shared_a(
@@ -253,6 +274,9 @@ def _ops():
 
 OPS = _ops()
 
+# Launches of the cases with K slices: the product (or the set) and its reduction.
+KERNELS = {n: 2 for n in OPS if n.endswith("_sliced")} | {"ng_gemm_int8_shared_a_M24_split": 2}
+
 
 @pytest.fixture()
 def capture_stream(lib):
@@ -266,7 +290,20 @@ def capture_stream(lib):
         hip.h.hipStreamDestroy(stream)
 
 
-def replay_and_check(lib, hip, stream, outs, call, exact, label, between=None):
+@pytest.fixture()
+def cold_stream(lib):
+    """A stream for which the library holds no buffer yet."""
+    hip = HipRuntime()
+    stream = hip.unused_stream()
+    lib.ng_set_stream(stream)
+    try:
+        yield hip, stream
+    finally:
+        lib.ng_set_stream(None)
+        hip.h.hipStreamDestroy(stream)
+
+
+def replay_and_check(lib, hip, stream, outs, call, exact, label, between=None, kernels=None):
     def snapshot():
         return {n: get(b, outs[n][0], outs[n][1]) for n, b in bufs.items()}
 
@@ -280,6 +317,7 @@ def replay_and_check(lib, hip, stream, outs, call, exact, label, between=None):
         eager = snapshot()
         graph, ex = hip.capture(stream, lambda: ok(call(bufs), f"{label} under capture"))
         try:
+            assert kernels in (None, hip.kernel_nodes(graph)), label
             for rep in range(3):
                 for n, (dt, shape) in outs.items():
                     bufs[n].upload(np.zeros(shape, dt))
@@ -308,24 +346,26 @@ def test_capture_replay(lib, inp, capture_stream, name):
     hip, stream = capture_stream
     outs, fn, exact = OPS[name]
     banner(f"graph capture: {name}")
-    eager = replay_and_check(lib, hip, stream, outs, lambda o: fn(lib, inp, o), exact, name)
+    eager = replay_and_check(lib, hip, stream, outs, lambda o: fn(lib, inp, o), exact, name,
+                             kernels=KERNELS.get(name))
     if name == "ng_gather_embeddings_checked":
         assert int(eager["n"][0]) == 2
 
 
-def test_capture_survives_buffer_growth(lib, inp, capture_stream):
-    """A graph holding a split-K GEMM keeps replaying correctly after an eager
+def test_capture_survives_buffer_growth(lib, inp, cold_stream):
+    """A graph holding a product with K slices keeps replaying correctly after an eager
     call on the same stream has replaced the partial-sum buffer by a larger one."""
-    hip, stream = capture_stream
-    banner("graph capture: split-K GEMM, then buffer growth, then replay")
+    hip, stream = cold_stream
+    banner("graph capture: K slices, then buffer growth, then replay")
     K, N = 4096, 4096
     rng = np.random.Generator(np.random.PCG64(3))
     a = dev(f16_bits(rng.standard_normal((128, K)).astype(np.float32)))
     w = dev(rng.integers(-127, 128, (N, K)).astype(np.int8))
     sc = dev(rng.uniform(1e-3, 1e-2, N).astype(np.float32))
     big = empty(128 * N * 2)
-    # (M, N) of the eager calls: their split-K partial sums take 2, 4 and 8 MB
-    # (8, 4 and 4 slices of M x N floats), each more than the buffer holds.
+    # (M, N) of the eager calls: their partial sums take 1, 2 and 4 MiB (4, 2
+    # and 2 slices of M x N floats), each more than the buffer holds; the
+    # captured product's 4 slices take 160 KiB.
     shapes = [(64, 1024), (64, 4096), (128, 4096)]
 
     def grow_partials(rep):
@@ -333,27 +373,14 @@ def test_capture_survives_buffer_growth(lib, inp, capture_stream):
         ok(lib.cuda_gemm_int8(big.vp, a.vp, w.vp, sc.vp, m, K, n, True), "eager larger GEMM")
 
     try:
-        outs = {"y": (E2, (64, GN))}
+        outs = {"y": (E2, (40, GN))}
         replay_and_check(
             lib, hip, stream, outs,
-            lambda o: lib.cuda_gemm_int8(o["y"].vp, inp["a64"].vp, inp["wq"].vp, inp["wsc"].vp, 64, GK, GN, True),
-            True, "split-K GEMM across buffer growth", between=grow_partials)
+            lambda o: lib.cuda_gemm_int8(o["y"].vp, inp["d40"].vp, inp["wq_deep"].vp, inp["wsc"].vp, 40, GKD, GN, True),
+            True, "K slices across buffer growth", between=grow_partials, kernels=2)
     finally:
         for b in (a, w, sc, big):
             b.free()
-
-
-@pytest.fixture()
-def cold_stream(lib):
-    """A stream for which the library holds no buffer yet."""
-    hip = HipRuntime()
-    stream = hip.unused_stream()
-    lib.ng_set_stream(stream)
-    try:
-        yield hip, stream
-    finally:
-        lib.ng_set_stream(None)
-        hip.h.hipStreamDestroy(stream)
 
 
 def kernels_captured(hip, stream, call, label):

@@ -124,10 +124,10 @@ def assert_fused_tight(got_bits, a, q, scale, what: str) -> None:
 
 # M, K, N: the weight-streaming path takes transpose_b, M <= 128 and K % 64 == 0
 # (K % 16 == 0 for M <= 4). M <= 4 runs the GEMV kernel (K in 1024-code
-# segments, the last one possibly partial); M > 16, and 4 < M <= 16 with K or
-# N >= 8192, the split-K kernel with 1 to 8 slices of K (4 waves per block, 8
-# for K >= 8192 and M > 16); 4 < M <= 16 otherwise the MFMA kernel that reads
-# A from L2.
+# segments, the last one possibly partial); 16 < M <= 32, and M <= 16 with K or
+# N >= 8192, the split kernel with 1 to 8 slices of K (4 waves per block, 8 for
+# K >= 8192 and M > 16); 4 < M <= 16 otherwise the MFMA kernel that reads A from
+# L2; M > 32 the ring kernel with 1 to 8 slices of K.
 FUSED = [
     (1, 4096, 4096), (3, 4096, 1024), (16, 4096, 4096), (17, 4096, 1000), (32, 1024, 512), (33, 4096, 4096),
     (64, 4096, 4096), (64, 4096, 1024), (8, 14336, 4096), (64, 14336, 4096), (5, 64, 16), (2, 128, 7),
@@ -135,14 +135,15 @@ FUSED = [
     (2, 256, 9000), (48, 4096, 1024), (65, 4096, 1024), (96, 4096, 4096), (128, 14336, 4096), (100, 1024, 300),
     (7, 8192, 64), (128, 64, 64), (4, 4096, 4096), (1, 1040, 100), (4, 2064, 33), (2, 14352, 64),
     (3, 16, 5), (12, 1024, 4096),
-    # K >= 8192 with M > 16: eight waves per block in the split kernel (one case with K % 128 == 64)
+    # K >= 8192 with M > 16: eight waves per block in the split kernel, the ring kernel from 33 rows on (one
+    # case with K % 128 == 64)
     (24, 8192, 1000), (100, 8256, 384), (48, 9216, 2048),
     # M = 3, 4 with K or N >= 8192: the split kernel (two wave groups per block for N >= 12288 at K < 8192)
     (4, 4096, 14336), (3, 4096, 12300), (3, 14336, 4096), (4, 14336, 100), (4, 8256, 200),
-    # N >= 12288 at K < 8192: two wave groups per block at every tile height, odd batch counts, a half batch
+    # N >= 12288 at K < 8192: one slice at every tile height, odd batch counts, a half batch
     (128, 4096, 14336), (80, 4160, 12288), (20, 1088, 13000), (33, 2048, 12290), (9, 192, 12288),
     (3, 64, 12288), (4, 128, 12300), (70, 64, 12288),
-    # N <= 2048 at K < 8192 with M > 32: token tiles of 32 rows of A as separate blocks
+    # N <= 2048 with M > 32: the ring kernel's smallest tiles
     (96, 4096, 1000), (128, 4096, 2048), (33, 1024, 64), (127, 4160, 1030),
 ]
 
@@ -203,8 +204,8 @@ def test_int8_weight_streaming_inf_activations(lib, M, K, N):
 
 # The prefill kernel (transpose_b, M > 128, K % 16 == 0): ragged M and N,
 # K with a partial last step of 128 (K % 128 = 64, 16), full model shapes.
-# 256 x 256 tiles from 192 of them on: 1000 x 14336, 777 x 16000 (ragged in M
-# and N), 3072 x 4096, 1000 x 4112 x 12300 (K % 64 = 16).
+# Large tiles at 1000 x 14336, 777 x 16000 (ragged in M and N), 3072 x 4096,
+# 1000 x 4112 x 12300 (K % 64 = 16).
 PREFILL = [(129, 4096, 1024), (256, 4096, 4096), (4096, 4096, 1024), (200, 4160, 1000), (300, 1040, 384),
            (4100, 1024, 300), (130, 14336, 256), (1000, 4096, 14336), (2049, 2048, 2056), (640, 16, 64),
            (777, 1024, 16000), (3072, 4096, 4096), (1000, 4112, 12300)]
@@ -386,8 +387,8 @@ def test_int8_across_shutdown_and_init():
         rng = np.random.Generator(np.random.PCG64(3))
         for rnd in range(2):
             assert L.cuda_init(0) == 0
-            # streaming (tb, small M), split-K (M = 40) and dequant + hipBLASLt (M = 200)
-            for M, K, N, tb in [(1, 256, 64, True), (40, 512, 128, True), (200, 128, 64, False)]:
+            # streaming (tb, small M), K slices (M = 40, K = 4096) and dequant + hipBLASLt (M = 200)
+            for M, K, N, tb in [(1, 256, 64, True), (40, 4096, 128, True), (200, 128, 64, False)]:
                 a = (rng.integers(-64, 65, (M, K)) / 64.0).astype(np.float16)
                 q = rng.integers(-128, 128, (N, K) if tb else (K, N)).astype(np.int8)
                 s = np.full(N, 2.0 ** -7, np.float32)
@@ -474,8 +475,8 @@ def test_reference_kat_gemm_transpose(lib):
     assert np.abs(got - _cpu_matmul(A.T, B)).max() < 0.1
 
 
-# The prefill kernel at the edges of its tiles (64, 128 and 256 rows of A, 128
-# and 256 of B), of its stages (fewer steps of 64 k than stages, a partial last
+# The prefill kernel at the edges of its tiles (64, 128, 192 and 256 rows of A,
+# 128 and 256 of B), of its stages (fewer steps of 64 k than stages, a partial last
 # step after none, one or more whole ones), with K slices, with N that no 16-byte
 # store divides and with C off 16 bytes. Inputs whose sums are exact in fp32, so
 # every tile shape and slice count has to give the same bits.

@@ -3,11 +3,11 @@
 Bar: c and out are bit-identical to the calls they replace,
 cuda_gemm_int8(c, a, b, scale, M, K, N, true) and then cuda_add(out, c,
 residual, M N), on the same inputs: in the fused GEMV launch (M <= 4 on the
-GEMV kernel's shapes), in the split-K reduction's epilogue (up to 128 rows on
-the split kernel with several K slices, with 4-wide and scalar reductions, and
-on the prefill kernel's 128 x 128 tiles with K slices), after a launch of one K
-slice or the small-M MFMA kernel (the add as its own launch), and as the two
-calls (K not a multiple of 16, 4096 rows and more), with
+GEMV kernel's shapes), in the reduction of the K slices (the split kernel up to
+32 rows, the ring kernel up to 128, the tile kernel above, with 4-wide and
+scalar reductions), after a launch of one K slice or the small-M MFMA kernel
+(the add as its own launch), and as the two calls (K not a multiple of 16, 4096
+rows and more), with
 out apart from c and the residual or in place on either (the engine writes
 the layer output apart, layer.cu:593-598).
 """
@@ -24,16 +24,15 @@ RNG = np.random.Generator(np.random.PCG64(73))
 
 # (M, K, N): Mistral-7B's down projection at 1-2 tokens, Llama-2-7B's, M = 3-4
 # below 8192, ragged N and K, tiny shapes (the fused GEMV launch); down at
-# 4, 8, 20 and 64 tokens and token tiles at 40 (the split reduction with the
-# add), N not a multiple of 4 (its scalar form), gate's shape at 8 tokens
-# (one K slice) and the small-M MFMA kernel; then the two calls.
+# 4, 8, 20 and 64 tokens (the reduction with the add), N not a multiple of 4
+# (its scalar form), the ring kernel in one K slice (40 tokens), gate's shape
+# at 8 tokens (one K slice) and the small-M MFMA kernel; then the two calls.
 FUSED = [(1, 14336, 4096), (2, 14336, 4096), (1, 11008, 4096), (2, 13824, 5120), (3, 4096, 4096), (4, 2048, 5000),
          (1, 4112, 1000), (3, 2064, 17), (1, 16, 5)]
 SPLIT = [(4, 14336, 4096), (8, 14336, 4096), (20, 4096, 4096), (64, 14336, 4096), (40, 1024, 2048),
          (24, 4096, 1002), (8, 4096, 14336), (8, 4096, 4096)]
-# the prefill kernel: 128 x 128 tiles with K slices (512, 1000 and 2048 rows,
-# the add in the reduction), 256 x 256 tiles in one slice (3072 rows: the add
-# after it)
+# the tile kernel: K slices (512, 1000 and 2048 rows: the add in the
+# reduction) and one slice (3072 rows: the add after it)
 PREFILL = [(512, 14336, 4096), (1000, 4096, 1000), (2048, 14336, 4096), (3072, 4096, 4096)]
 TWO_CALLS = [(1, 4104, 64), (4096, 1024, 512)]
 

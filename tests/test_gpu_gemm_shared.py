@@ -4,8 +4,9 @@ Bars:
   * every C_i is bit-identical to its own cuda_gemm_int8(c_i, a, b_i, scale_i,
     M, K, n_i, true) on the same inputs (random activations, random codes and
     scales), whether a product ran in a shared launch (with the products of
-    the same launch shape: the GEMV kernel, the small-M MFMA kernel, or the
-    split kernel and its reduction) or as its own call;
+    the same launch shape: the GEMV kernel, the small-M MFMA kernel, the split
+    kernel, the ring kernel or the tile kernel, and their reduction) or as its
+    own call;
   * exact inputs (activations on a grid 2^-e, so that every partial sum of
     A @ q is exact in fp32) give fp16(fp32(sum_k a_k q_k) * scale[n]) bit for
     bit, the weight-streaming paths' formula, checked against numpy;
@@ -45,7 +46,7 @@ SETS = [
     (5, 4160, [1000, 77, 2048]),
     # one split-kernel launch (and one reduction): q/k/v at 17-32 tokens, with
     # a half last batch of K (K % 128 == 64), and with reductions of two forms;
-    # gate/up from 3 to 128 tokens (one slice of K, two wave groups per block)
+    # gate/up in one K slice from 3 to 128 tokens (from 33 on the ring kernel)
     (17, 4096, [4096, 1024, 1024]),
     (32, 4096, [4096, 1024, 1024]),
     (24, 4160, [1000, 77, 2048]),
@@ -56,17 +57,16 @@ SETS = [
     (20, 4096, [14336, 14336]),
     (64, 4096, [14336, 14336]),
     (100, 4096, [14336, 14336]),
-    # the one-group split shapes with several K slices (Llama-2-7B's gate/up at
-    # 3-16, 17-32, 33-64 and 65-128 tokens, q/k/v of TinyLlama's width at 24)
+    # Llama-2-7B's gate/up at 3-16 and 17-32 tokens (K slices) and on the ring
+    # kernel, q/k/v of TinyLlama's width at 24
     (8, 4096, [11008, 11008]),
     (24, 4096, [11008, 11008]),
     (40, 4096, [11008, 11008]),
     (100, 4096, [11008, 11008]),
     (24, 2048, [5632, 5634]),
-    # the fused prefill kernel (129-4095 tokens): q/k/v on 128 x 128 tiles with
-    # K slices of several counts, ragged shapes, gate/up on 256 x 256 tiles,
-    # and q on 256 x 256 tiles beside k/v on 128 x 128 (two launches); from
-    # 4096 tokens on hipBLASLt, one call each
+    # the tile kernel (129-4095 tokens): q/k/v with K slices of several counts,
+    # ragged shapes, gate/up, tiles that cross no product's edge; from 4096
+    # tokens on hipBLASLt, one call each
     (512, 4096, [4096, 1024, 1024]),
     (300, 1040, [4100, 1000, 77]),
     (200, 4096, [14336, 4096]),
@@ -74,8 +74,8 @@ SETS = [
     (2048, 4096, [4096, 1024, 1024]),
     (3000, 4096, [4096, 1024, 1024]),
     (4096, 4096, [4096, 1024]),
-    # products of different shapes, grouped: k and v with token tiles in one
-    # launch beside q alone (M = 33-128), two GEMV products and two split ones
+    # products of different shapes: q/k/v on the ring kernel (M = 33-128, the
+    # narrow products with more K slices), two GEMV products and two split ones
     # in two launches, a small-M MFMA product with a split one, a GEMV product
     # with a split one; and down's deep shape, which has no shared form
     (64, 4096, [4096, 1024, 1024]),

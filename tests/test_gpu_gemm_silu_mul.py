@@ -3,15 +3,14 @@
 Bar: out, gate and up are bit-identical to the calls they replace,
 ng_gemm_int8_shared_a (gate and up on one A, each bit for bit its own
 cuda_gemm_int8) and then cuda_silu_mul(out, gate, up), on the same inputs:
-in the fused GEMV launch (M <= 4 on the GEMV kernel's shapes), in the split
-kernel's SwiGLU form (3 to 128 rows where gate/up takes the two-group split
-kernel with one K slice: every one of its four shapes, ragged N), in the
-split-K reduction's SwiGLU form (the one-group split shapes with several K
-slices: Llama-2-7B and TinyLlama widths, each of the four shapes, N not a
-multiple of 4), and where the call is the two calls (the small-M MFMA kernel,
-token tiles, K not a multiple of 16, M > 128), with out apart from
-gate and up or in place on either, as the engine runs SwiGLU in place on gate
-(layer.cu:585-588).
+in the fused GEMV launch (M <= 4 on the GEMV kernel's shapes), in the SwiGLU
+forms of the split kernel (3 to 32 rows) and of the ring kernel (33 to 128)
+where gate/up takes one K slice (ragged N), in the SwiGLU form of the reduction
+where it takes several (Llama-2-7B and TinyLlama widths, N not a multiple of
+4), in the SwiGLU form of the tile kernel (from 129 rows on), and where the
+call is the two calls (the small-M MFMA kernel, K not a multiple of 16), with
+out apart from gate and up or in place on either, as the engine runs SwiGLU in
+place on gate (layer.cu:585-588).
 """
 from __future__ import annotations
 
@@ -29,19 +28,21 @@ RNG = np.random.Generator(np.random.PCG64(71))
 # the two calls.
 FUSED = [(1, 4096, 14336), (2, 4096, 14336), (1, 4096, 11008), (2, 5120, 13824), (3, 4096, 4096), (4, 2048, 5000),
          (1, 4112, 1000), (3, 2064, 17), (1, 16, 5)]
-# the split kernel's SwiGLU form: <1,4,2> at 3-16 rows, <2,4,2> at 17-32,
-# <4,4,2> at 33-64, <8,4,2> at 65-128 (Mistral-7B), N not a multiple of 32
+# one K slice: the split kernel's <1,4,2> at 3-16 rows and <2,4,2> at 17-32, the
+# ring kernel's tiles of 64 and 128 rows (Mistral-7B), N not a multiple of 32
 # (12300), Llama-2-13B's width, K with a half last batch (4160)
 SPLIT = [(3, 4096, 14336), (4, 4096, 14336), (8, 4096, 14336), (16, 4096, 14336), (17, 4096, 14336),
          (32, 4096, 14336), (40, 4096, 14336), (64, 4096, 14336), (65, 4096, 14336), (128, 4096, 14336),
          (8, 4096, 12300), (20, 5120, 13824), (12, 4160, 12400)]
-# the reduction's SwiGLU form: <1,4,1> at 3-16 rows, <2,4,1> at 17-32,
-# <4,4,1> at 33-64, <8,4,1> at 65-128 (Llama-2-7B: 2 K slices), TinyLlama's
-# width (3 slices), N % 4 != 0 (one output per thread), K with a half last
-# batch
+# several K slices: the split kernel's <1,4,1> at 3-16 rows and <2,4,1> at
+# 17-32 (Llama-2-7B: 2 slices), TinyLlama's width (3 slices), N % 4 != 0 (one
+# output per thread), K with a half last batch; at 40 and 100 rows one slice on
+# the ring kernel
 SLICED = [(3, 4096, 11008), (8, 4096, 11008), (16, 4096, 11008), (17, 4096, 11008), (40, 4096, 11008),
           (100, 4096, 11008), (24, 2048, 5632), (24, 2048, 5634), (8, 4160, 11000)]
-TWO_CALLS = [(8, 4096, 4096), (1, 4104, 64), (40, 1024, 2048), (200, 1024, 2048)]
+# the ring kernel's and the tile kernel's smallest tiles in one K slice
+SMALL_TILES = [(40, 1024, 2048), (200, 1024, 2048)]
+TWO_CALLS = [(8, 4096, 4096), (1, 4104, 64)]
 
 
 def f16bits(x) -> np.ndarray:
@@ -86,7 +87,7 @@ def check(got, want):
         assert_bits_equal(got[k], want[k], k)
 
 
-@pytest.mark.parametrize("M,K,N", FUSED + SPLIT + SLICED + TWO_CALLS)
+@pytest.mark.parametrize("M,K,N", FUSED + SPLIT + SLICED + SMALL_TILES + TWO_CALLS)
 def test_silu_mul_is_the_two_calls(lib, M, K, N):
     banner(f"gemm_int8_silu_mul M={M} K={K} N={N}")
     p = problem(M, K, N)

@@ -51,8 +51,8 @@ def both(lib, M, K, N):
 
 
 def test_noalloc_two_calls_second_smaller(lib):
-    # 1st: down_proj at M = 64 (8 slices of K: 8 MiB of partial sums);
-    # 2nd: smaller, also split (q_proj-like at M = 20, fewer outputs and slices).
+    # 1st: down_proj at M = 64 (4 slices of K: 4 MiB of partial sums);
+    # 2nd: smaller, also with K slices (q_proj-like at M = 20, fewer outputs).
     first, second = (64, 14336, 4096), (20, 4096, 1000)
     banner(f"ng_gemm_int8_noalloc two calls: {first} then {second}")
     data = [inputs(*sh) for sh in (first, second)]
@@ -67,9 +67,10 @@ def test_noalloc_two_calls_second_smaller(lib):
         assert_bits_equal(get(c, np.uint16, (M, N)), ref, f"noalloc {M}x{K}x{N}")
 
 
-# GEMV (M <= 4), the small-M MFMA kernel, the split kernel with 1 to 8 slices
-# (4 and 8 waves), and two wave groups per block (N >= 12288 at K < 8192).
-# The prefill kernel with 1 to 8 slices of K, both tile shapes, ragged M and N.
+# GEMV (M <= 4), the small-M MFMA kernel, the split kernel with one K slice and
+# two wave groups per block (M = 3, N >= 12288 at K < 8192), the ring kernel
+# (33 to 128 rows) with 1 to 8 K slices and two and four wave groups; the tile
+# kernel with 1 to 8 K slices, several tile shapes, ragged M and N.
 SHAPES = [(1, 4096, 4096), (4, 2064, 33), (8, 4096, 4096), (12, 1088, 4096), (33, 4096, 1024),
           (64, 4096, 14336), (128, 14336, 4096), (100, 8256, 384), (128, 4096, 1024), (3, 4096, 12300),
           (129, 256, 64), (200, 4096, 1000), (512, 4096, 4096), (300, 14336, 4096), (1024, 4096, 14336),
