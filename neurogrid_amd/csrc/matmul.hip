@@ -29,9 +29,10 @@
 // Above 128 rows of A (prefill) the product is bound by the matrix cores:
 // gemm_i8w_tile_kernel, a tiled GEMM that loads A and the codes of B straight
 // into LDS and converts the codes on their way to the matrix cores (see the
-// prefill section), with the residual add or SwiGLU in its epilogue; from 4096 rows on (kLtMinM) the
-// reference's composition through hipBLASLt, which is faster there. B stored
-// [K, N] always goes through the composition (dequantize, then hipBLASLt).
+// prefill section), with the residual add or SwiGLU in its epilogue; from 4096
+// rows on (kLtMinM) the reference's composition through hipBLASLt, which is
+// faster there. B stored [K, N] always goes through the composition (dequantize,
+// then hipBLASLt).
 // Each fused kernel also has a shared form (ng_gemm_int8_shared_a) that runs
 // several products with the same A and the same launch shape in one launch,
 // each product's blocks as in its own launch; the GEMV kernel's shared form
@@ -938,8 +939,8 @@ __device__ __forceinline__ void gemm_i8w_split_block(
 
     // A and B are read with buffer loads: B from this wave's first row (rows
     // past N clamp to the last one), A from its start, so that per-load
-    // offsets are 32-bit instead of 64-bit addresses (2-6% faster at
-    // M = 64-128). Offsets are below 16 K bytes for B and 2 M K bytes for A.
+    // offsets are 32-bit instead of 64-bit addresses. Offsets are below 16 K
+    // bytes for B and 2 M K bytes for A.
     const int nbase = min(nw, N - 1);
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(b + static_cast<size_t>(nbase) * K), 0, 0x7fffffff, 0x00020000);
@@ -1025,7 +1026,7 @@ __device__ __forceinline__ void gemm_i8w_split_block(
             f16x8 b0, b1;
             codes16_to_operands(v, b0, b1);
             // All tiles' first halves, then their second halves: consecutive
-            // MFMAs update different accumulators (2-4% faster at M = 64-128).
+            // MFMAs update different accumulators.
             u32x4 a0[MT], a1[MT];
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
@@ -1332,12 +1333,12 @@ __global__ __launch_bounds__(256) void split_reduce_shared_kernel(SharedSet s, S
 //     tiles); each block stores its fp32 sums in `part` [S][M][N] and the
 //     reduction adds the slices in slice order.
 // Every output is the sum over k in one order whatever the tile shape, so only
-// S (a function of M, N and K alone) shows in the bits. Measured on MI355X, back
-// to back, against the kernel this replaces (A and B through registers, B stored
-// to LDS as fp16, two LDS buffers): o at 1024 tokens of Mistral-7B 46.8 against
-// 55.3 us, gate/up with SwiGLU 224.8 against 244.2, down 138.2 against 148.1; o
-// at 333 tokens 28.0 against 37.0; a whole layer at 333 tokens of Llama-2-7B 261
-// against 350 us, at 1024 tokens of Mistral-7B 526 against 598. What bounds it on
+// S (a function of M, N and K alone) shows in the bits. Measured on MI355X, in
+// turn with the kernel this replaces (A and B through registers, B stored to LDS
+// as fp16, two LDS buffers): a whole layer at 333 tokens of Llama-2-7B 220
+// against 344 us, at 1024 tokens of Mistral-7B 468 against 574. In that last
+// layer's kernel trace (weights cold): q/k/v 59 us, o 43, gate/up with SwiGLU 213
+// (1.13 PFLOP/s), down 110 and 18 for its reduction. What bounds it on
 // 256 x 256 tiles (1024 x 28672, K = 4096: 206 us, 1.17 PFLOP/s): the power limit
 // with the matrix cores 64% busy (1.75 GHz). The MFMAs alone (no loads, no LDS
 // reads) took 130 us, without the LDS reads 164, without the loads into LDS 182,
@@ -3079,9 +3080,12 @@ int shared_group(int path, int count, void* const* c, const void* a, const void*
 // Products that share A (the engine's q/k/v and gate/up projections): they
 // are grouped by the launch shape gemm_i8w would take for each, and each group
 // runs in one launch of that kernel's shared form (plus one launch of the
-// split kernel's reduction), each product's blocks exactly as its own launch
-// would. Products outside the weight-streaming path are one cuda_gemm_int8
-// call each. Either way the results are cuda_gemm_int8's, bit for bit.
+// reduction where K slices have blocks of their own). Up to 32 rows each
+// product's blocks are exactly its own launch's; above, the tile may be another
+// (no bit depends on it). Products that take no kernel of the library's are one
+// cuda_gemm_int8 call each, and so are those of a set whose partial sums have no
+// room while a graph is captured. Either way the results are cuda_gemm_int8's,
+// bit for bit.
 extern "C" int ng_gemm_int8_shared_a(int count, void* const* c, const void* a, const void* const* b,
                                      const void* const* scales, const int* n, int M, int K) {
     NG_REQUIRE(c && a && b && scales && n, "ng_gemm_int8_shared_a: null pointer");
@@ -3304,10 +3308,11 @@ static int swiglu_split(const SwigluArgs& sa, const uint16_t* a, int M, int K, i
 // gate/up (cuda_gemm_int8 on one A, as ng_gemm_int8_shared_a) and SwiGLU
 // (cuda_silu_mul), when no output overlaps an input or another output (out
 // may be gate or up exactly): one launch of gemv_i8w_swiglu_kernel when both
-// products take the GEMV kernel, one of gemm_i8w_split_swiglu_kernel (33 to 128
-// rows: _ring_, above and below kLtMinM: _tile_) when they take that kernel with
-// one K slice, its shared launch and split_reduce_swiglu_kernel when they have
-// several; otherwise the two calls. The same bits either way.
+// products take the GEMV kernel; one of the SwiGLU form of the split kernel (up
+// to 32 rows), the ring kernel (33 to 128) or the tile kernel (below kLtMinM) when
+// they take that kernel with one K slice; the kernel's shared launch and
+// split_reduce_swiglu_kernel when they have several; otherwise the two calls.
+// The same bits either way.
 extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void* a, const void* b_gate,
                                      const void* scale_gate, const void* b_up, const void* scale_up, int M, int K,
                                      int N) {
@@ -3373,9 +3378,9 @@ extern "C" int ng_gemm_int8_silu_mul(void* out, void* gate, void* up, const void
 // output (out may be c or the residual exactly), one launch of
 // gemv_i8w_add_kernel on the GEMV kernel's shapes, and on cuda_gemm_int8's
 // other fused paths (the weight-streaming kernels up to 128 rows, the prefill
-// kernel below kLtMinM) the add in the split-K reduction, or with one K slice in
-// the epilogue of the 33 - 128 row and the prefill kernel (up to 32 rows after
-// the product as cuda_add); otherwise the two calls. The same bits either way.
+// kernel below kLtMinM) the add in the reduction of the K slices, or with one K
+// slice in the epilogue of the ring and the tile kernel (up to 32 rows after the
+// product as cuda_add); otherwise the two calls. The same bits either way.
 extern "C" int ng_gemm_int8_add(void* out, void* c, const void* a, const void* b, const void* scale,
                                 const void* residual, int M, int K, int N) {
     NG_REQUIRE(out && c && a && b && scale && residual, "ng_gemm_int8_add: null pointer");
