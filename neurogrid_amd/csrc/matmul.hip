@@ -1337,8 +1337,8 @@ __global__ __launch_bounds__(256) void split_reduce_shared_kernel(SharedSet s, S
 // turn with the kernel this replaces (A and B through registers, B stored to LDS
 // as fp16, two LDS buffers): a whole layer at 333 tokens of Llama-2-7B 220
 // against 344 us, at 1024 tokens of Mistral-7B 468 against 574. In that last
-// layer's kernel trace (weights cold): q/k/v 59 us, o 43, gate/up with SwiGLU 213
-// (1.13 PFLOP/s), down 110 and 18 for its reduction. What bounds it on
+// layer's kernel trace (weights cold): q/k/v 62 us, o 44, gate/up with SwiGLU 222
+// (1.08 PFLOP/s), down 113 and 18 for its reduction. What bounds it on
 // 256 x 256 tiles (1024 x 28672, K = 4096: 206 us, 1.17 PFLOP/s): the power limit
 // with the matrix cores 64% busy (1.75 GHz). The MFMAs alone (no loads, no LDS
 // reads) took 130 us, without the LDS reads 164, without the loads into LDS 182,
@@ -1785,7 +1785,7 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_i8w_tile_swiglu_kerne
 //   * B is loaded, and lies in LDS, in 128-byte pieces of rows (128 k, two
 //     groups): whole lines; 16-byte piece q of row r at q xor ((r / 2) mod 8), as
 //     for A;
-//   * S slices of K (a function of N and K) where one slice leaves most CUs
+//   * S slices of K (a function of M, N and K) where one slice leaves most CUs
 //     idle, added in slice order by the reduction; with one slice the epilogues
 //     of the prefill kernel. Gate and up with SwiGLU load B non-temporally (at 64
 //     rows 29.2 against 31.2 us); with K slices that was 2-8% slower.
